@@ -109,9 +109,9 @@ int cth_ctx_create(int device, cth_ctx** out) {
     c->device = device;
     c->num_cus = prop.multiProcessorCount;
     int rc = check_hip(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
-    if (rc == CTH_OK) rc = check_hip(hipMalloc((void**)&c->counters, 2 * COUNTER_RING * sizeof(uint32_t)), "hipMalloc");
+    if (rc == CTH_OK) rc = check_hip(hipMalloc((void**)&c->counters, counter_words(COUNTER_RING) * sizeof(uint32_t)), "hipMalloc");
     if (rc == CTH_OK)
-        rc = check_hip(hipMemset(c->counters, 0, 2 * COUNTER_RING * sizeof(uint32_t)), "hipMemset counters");
+        rc = check_hip(hipMemset(c->counters, 0, counter_words(COUNTER_RING) * sizeof(uint32_t)), "hipMemset counters");
     if (rc == CTH_OK) rc = check_hip(hipHostMalloc((void**)&c->pinned, 8 * sizeof(uint64_t)), "hipHostMalloc");
     if (rc == CTH_OK) rc = vjp_scratch_init(device);
     if (rc == CTH_OK) rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
@@ -523,27 +523,27 @@ int cth_wall_clock_khz(const cth_ctx* c) {
 struct cth_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    uint32_t* pairs = nullptr;  // the graph's own work-counter pairs
+    uint32_t* counters = nullptr;  // the graph's own work-counter entries
 };
 
-// The graph's counter pairs are allocated and zeroed before the capture
+// The graph's counter entries are allocated and zeroed before the capture
 // starts (no allocation may happen inside it) and kept until the graph is
-// destroyed, so its replays never share a pair with other launches.
+// destroyed, so its replays never share an entry with other launches.
 int cth_graph_begin(void* stream) {
     if (!stream) return fail(CTH_E_INVALID, "graph capture needs a non-null stream");
-    if (g_capture.pairs) return fail(CTH_E_INVALID, "a capture is already in progress on this thread");
-    uint32_t* pairs = nullptr;
-    const size_t bytes = 2 * GRAPH_PAIRS * sizeof(uint32_t);
-    int rc = check_hip(hipMalloc((void**)&pairs, bytes), "hipMalloc graph counters");
-    if (!rc) rc = check_hip(hipMemsetAsync(pairs, 0, bytes, (hipStream_t)stream), "zero graph counters");
+    if (g_capture.counters) return fail(CTH_E_INVALID, "a capture is already in progress on this thread");
+    uint32_t* counters = nullptr;
+    const size_t bytes = counter_words(GRAPH_ENTRIES) * sizeof(uint32_t);
+    int rc = check_hip(hipMalloc((void**)&counters, bytes), "hipMalloc graph counters");
+    if (!rc) rc = check_hip(hipMemsetAsync(counters, 0, bytes, (hipStream_t)stream), "zero graph counters");
     if (!rc) rc = check_hip(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
     if (!rc) rc = check_hip(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal), "begin capture");
     if (rc) {
-        if (pairs) (void)hipFree(pairs);
+        if (counters) (void)hipFree(counters);
         return rc;
     }
     g_capture.stream = (hipStream_t)stream;
-    g_capture.pairs = pairs;
+    g_capture.counters = counters;
     g_capture.pos = 0;
     return CTH_OK;
 }
@@ -552,8 +552,8 @@ int cth_graph_end(void* stream, cth_graph** out) {
     if (!stream || !out) return fail(CTH_E_INVALID, "null argument");
     *out = nullptr;
     cth_graph* g = new cth_graph();
-    if (g_capture.pairs && g_capture.stream == (hipStream_t)stream) {
-        g->pairs = g_capture.pairs;
+    if (g_capture.counters && g_capture.stream == (hipStream_t)stream) {
+        g->counters = g_capture.counters;
         g_capture = CapturePool{};
     }
     int rc = check_hip(hipStreamEndCapture((hipStream_t)stream, &g->graph), "end capture");
@@ -575,7 +575,7 @@ void cth_graph_destroy(cth_graph* g) {
     if (!g) return;
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
-    if (g->pairs) (void)hipFree(g->pairs);
+    if (g->counters) (void)hipFree(g->counters);
     delete g;
 }
 

@@ -11,24 +11,38 @@
 
 namespace cth {
 
-// Work counters: a ring of {next, done} pairs, zeroed at context creation.
-// Each launch takes the next pair, and the launch's last wave zeroes it again
-// (work_loop.h), so launches on different streams never share a pair unless
-// more than COUNTER_RING launches are in flight at once.  Launches recorded
-// into a graph through cth_graph_begin take their pairs from the graph's own
-// pool instead (CapturePool), since a graph replays with the pairs it was
-// captured with for as long as it lives.
+// Work counters of the dynamic launches: a ring of entries, zeroed at context
+// creation.  Each launch takes the next entry, and the last waves of its
+// shards zero it again (work_loop.h), so launches on different streams never
+// share an entry unless more than COUNTER_RING launches are in flight at once.
+// Launches recorded into a graph through cth_graph_begin take their entries
+// from the graph's own pool instead (CapturePool), since a graph replays with
+// the entries it was captured with for as long as it lives.
+//
+// An entry is one {claimed, left} pair in each of kMaxShards 128-byte lines;
+// the 16 pairs of a line belong to 16 successive entries, so a launch's shards
+// never share a line and the ring stays at 1 MiB.
 constexpr uint32_t COUNTER_RING = 4096;
+constexpr uint32_t kMaxShards = 32;
+constexpr uint32_t kShardStride = 32;  // words between an entry's shards
+constexpr uint32_t kLineEntries = kShardStride / 2;
+constexpr size_t counter_words(uint32_t entries) {
+    return (size_t)(entries / kLineEntries) * kMaxShards * kShardStride;
+}
+inline uint32_t* counter_entry(uint32_t* base, uint32_t i) {
+    return base + (size_t)(i / kLineEntries) * kMaxShards * kShardStride + 2 * (i % kLineEntries);
+}
 
-// Counter pairs owned by the graph being captured on this thread: launches
-// recorded on `stream` take pairs from `pairs` (zeroed before the capture
+// Counter entries owned by the graph being captured on this thread: launches
+// recorded on `stream` take entries from `counters` (zeroed before the capture
 // began), cycling through them.  Launches of one graph on its one stream run
-// one after another, and each leaves its pair at zero, so a pair can serve
+// one after another, and each leaves its entry at zero, so an entry can serve
 // several of them.
-constexpr uint32_t GRAPH_PAIRS = 64;
+constexpr uint32_t GRAPH_ENTRIES = 64;
+static_assert(COUNTER_RING % kLineEntries == 0 && GRAPH_ENTRIES % kLineEntries == 0, "whole lines");
 struct CapturePool {
     hipStream_t stream = nullptr;
-    uint32_t* pairs = nullptr;  // 2 * GRAPH_PAIRS, device
+    uint32_t* counters = nullptr;  // GRAPH_ENTRIES entries, device
     uint32_t pos = 0;
 };
 CapturePool& capture_pool();  // this thread's (capi.hip)
@@ -62,7 +76,7 @@ struct Ctx {
     int num_cus = 0;
     int mode = CTH_MODE_PARITY;
     hipStream_t stream = nullptr;
-    uint32_t* counters = nullptr;  // 2 * COUNTER_RING
+    uint32_t* counters = nullptr;  // COUNTER_RING entries
     uint32_t ring_pos = 0;
     void* ws[WS_SLOTS] = {};
     size_t ws_bytes[WS_SLOTS] = {};
@@ -90,14 +104,14 @@ struct Ctx {
     }
     LaunchShape shape_de;
     LaunchShape shape_spans{256, 8, 1024, 32, 1};
-    // The counter pair of a launch on stream `st`: the capturing graph's own
-    // pairs while cth_graph_begin captures `st` on this thread, else the next
-    // pair of the ring.
+    // The counter entry of a launch on stream `st`: from the capturing graph's
+    // own while cth_graph_begin captures `st` on this thread, else the next of
+    // the ring.
     uint32_t* take_counters(hipStream_t st) {
         CapturePool& cp = capture_pool();
-        if (cp.pairs && cp.stream == st) return cp.pairs + 2 * (cp.pos++ % GRAPH_PAIRS);
+        if (cp.counters && cp.stream == st) return counter_entry(cp.counters, cp.pos++ % GRAPH_ENTRIES);
         uint32_t i = __atomic_fetch_add(&ring_pos, 1u, __ATOMIC_RELAXED) % COUNTER_RING;
-        return counters + 2 * i;
+        return counter_entry(counters, i);
     }
     LaunchShape shape_trace{256, 16, 256, 32, 0};
     LaunchShape shape_adj{256, 16, 256, 32, 0};

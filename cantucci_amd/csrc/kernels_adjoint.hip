@@ -47,11 +47,12 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
     bool live = false, hold = false;
     uint32_t idx = 0, k = 0;
     float r = 0.0f;
-    uint32_t c_next = 0, c_end = 0, round = 0;
+    Window win;
     bool exhausted = false;
+    uint32_t refill_at = q.refill_min;
     const size_t stride = (size_t)u.max_iters + 1;
     for (;;) {
-        if ((uint32_t)__popcll(wave_mask(!live)) >= q.refill_min) {
+        if ((uint32_t)__popcll(wave_mask(!live)) >= refill_at) {
             if (hold) {
                 float d = ev.finish(r);
                 if (dout) dout[idx] = d;
@@ -63,21 +64,16 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
             while (!exhausted) {
                 uint64_t need = wave_mask(!live);
                 if (need == 0) break;
-                if (c_next >= c_end) {
-                    uint32_t b = next_chunk(q, round);
-                    if (b >= q.total) {
-                        exhausted = true;
-                        break;
-                    }
-                    c_next = b;
-                    c_end = (q.total - b < q.chunk) ? q.total : b + q.chunk;
+                if (win.next >= win.end && !next_chunk(q, win)) {
+                    exhausted = true;
+                    break;
                 }
-                uint32_t avail = c_end - c_next;
+                uint32_t avail = win.end - win.next;
                 uint32_t nneed = (uint32_t)__popcll(need);
                 if (!live) {
                     uint32_t rank = lane_rank(need);
                     if (rank < avail) {
-                        idx = c_next + rank;
+                        idx = win.next + rank;
                         float px, py, pz, pw;
                         src.get(idx, px, py, pz, pw);
                         ev.start(px, py, pz, pw, u);
@@ -92,9 +88,10 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
                         }
                     }
                 }
-                c_next += (nneed < avail) ? nneed : avail;
+                win.next += (nneed < avail) ? nneed : avail;
             }
             if (wave_mask(live) == 0) break;
+            if (exhausted || win.drained()) refill_at = 64u;
         }
         if (live) orbit[(size_t)idx * stride + k] = make_float4(ev.x, ev.y, ev.z, ev.dr);
         ev.body(r, u, live);
@@ -290,29 +287,25 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
     float P = 0.0f, px = 0.0f, py = 0.0f, pz = 0.0f;
     float zbx = 0.0f, zby = 0.0f, zbz = 0.0f, drb = 0.0f, cbx = 0.0f, cby = 0.0f, cbz = 0.0f, Pb = 0.0f;
     float rb_extra = 0.0f;
-    uint32_t c_next = 0, c_end = 0, round = 0;
+    Window win;
     bool exhausted = false;
+    uint32_t refill_at = q.refill_min;
     const size_t stride = (size_t)u.max_iters + 1;
     for (;;) {
-        if ((uint32_t)__popcll(wave_mask(!live)) >= q.refill_min) {
+        if ((uint32_t)__popcll(wave_mask(!live)) >= refill_at) {
             while (!exhausted) {
                 uint64_t need = wave_mask(!live);
                 if (need == 0) break;
-                if (c_next >= c_end) {
-                    uint32_t b = next_chunk(q, round);
-                    if (b >= q.total) {
-                        exhausted = true;
-                        break;
-                    }
-                    c_next = b;
-                    c_end = (q.total - b < q.chunk) ? q.total : b + q.chunk;
+                if (win.next >= win.end && !next_chunk(q, win)) {
+                    exhausted = true;
+                    break;
                 }
-                uint32_t avail = c_end - c_next;
+                uint32_t avail = win.end - win.next;
                 uint32_t nneed = (uint32_t)__popcll(need);
                 if (!live) {
                     uint32_t rank = lane_rank(need);
                     if (rank < avail) {
-                        idx = c_next + rank;
+                        idx = win.next + rank;
                         src.get(idx, px, py, pz, P);
                         AdjRecord rc = rec[idx];
                         float g = out.grad_d ? out.grad_d[idx] : 1.0f;
@@ -346,9 +339,10 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
                         }
                     }
                 }
-                c_next += (nneed < avail) ? nneed : avail;
+                win.next += (nneed < avail) ? nneed : avail;
             }
             if (wave_mask(live) == 0) break;
+            if (exhausted || win.drained()) refill_at = 64u;
         }
         if (live) {
             float4 s = orbit[(size_t)idx * stride + j];

@@ -61,12 +61,13 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
     // (the job's cap counted from the tick at which the lane took the point).
     uint32_t tick = 0, tcap = 0;
     float r = 0.0f;
-    uint32_t c_next = 0, c_end = 0, round = 0;
+    Window win;
     bool exhausted = false;
+    uint32_t refill_at = q.refill_min;
     SinkGrad sink{dists, normals, nullptr, nullptr, nullptr, 0u};
 
     for (;;) {
-        if ((uint32_t)__popcll(wave & ~live_m) >= q.refill_min) {
+        if ((uint32_t)__popcll(wave & ~live_m) >= refill_at) {
             // write back held points, then stamp their jobs (one atomic per job per wave)
             // SinkGrad reads k only as k == max_iters (the point stopped at the cap).
             if (__builtin_amdgcn_inverse_ballot_w64(hold_m)) {
@@ -89,22 +90,17 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
             while (!exhausted) {
                 const uint64_t need = wave & ~live_m;
                 if (need == 0) break;
-                if (c_next >= c_end) {
-                    uint32_t b = next_chunk(q, round);
-                    if (b >= q.total) {
-                        exhausted = true;
-                        break;
-                    }
-                    c_next = b;
-                    c_end = (q.total - b < q.chunk) ? q.total : b + q.chunk;
+                if (win.next >= win.end && !next_chunk(q, win)) {
+                    exhausted = true;
+                    break;
                 }
-                uint32_t avail = c_end - c_next;
+                uint32_t avail = win.end - win.next;
                 uint32_t nneed = (uint32_t)__popcll(need);
                 const uint32_t rank = lane_rank(need);
                 const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
                 {
                     if (take) {
-                        idx = c_next + rank;
+                        idx = win.next + rank;
                         // job of idx: the last offset <= idx
                         uint32_t lo = 0, hi = njobs;
                         while (hi - lo > 1) {
@@ -136,9 +132,10 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
                     }
                 }
                 live_m |= wave_mask(take) & ~wave_mask(r > u.bailout);
-                c_next += (nneed < avail) ? nneed : avail;
+                win.next += (nneed < avail) ? nneed : avail;
             }
             if (live_m == 0) break;
+            if (exhausted || win.drained()) refill_at = (uint32_t)__popcll(wave);
         }
         const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
         const uint64_t cap_m = wave_mask(tcap == tick) & live_m;

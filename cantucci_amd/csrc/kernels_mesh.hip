@@ -798,7 +798,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
     uint32_t vid = 0, t = 0;
     uint32_t tick = 0, t0 = 0;  // wave's body count; tick at which the lane's tap started
     float r = 0.0f;
-    uint32_t c_next = 0, c_end = 0, round = 0;
+    Window win;
     bool exhausted = false;
     WorkTally<kCount> tally;
 
@@ -833,28 +833,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
                 }
                 const uint64_t need = wave_mask(!has_v) & ~live_m;
                 if (need != 0 && !exhausted) {
-                    if (c_next >= c_end) {
-                        const uint32_t b = next_chunk(q, round);
-                        if (b >= q.total) {
-                            exhausted = true;
-                        } else {
-                            c_next = b;
-                            c_end = (q.total - b < q.chunk) ? q.total : b + q.chunk;
-                        }
-                    }
+                    if (win.next >= win.end && !next_chunk(q, win)) exhausted = true;
                     if (!exhausted) {
-                        const uint32_t avail = c_end - c_next;
+                        const uint32_t avail = win.end - win.next;
                         const uint32_t nneed = (uint32_t)__popcll(need);
                         const uint32_t rank = lane_rank(need);
                         if (__builtin_amdgcn_inverse_ballot_w64(need) && rank < avail) {
-                            vid = c_next + rank;
+                            vid = win.next + rank;
                             const float* rec = verts + 7 * (size_t)vid;
 #pragma unroll
                             for (int j = 0; j < 6; ++j) slot[256 * j] = rec[j];
                             t = 0;
                             has_v = true;
                         }
-                        c_next += (nneed < avail) ? nneed : avail;
+                        win.next += (nneed < avail) ? nneed : avail;
                     }
                 }
                 const uint64_t start_m = wave_mask(has_v) & ~live_m;

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void k_trace(
     uint32_t tick = 0, t0 = 0;  // wave's body count; tick at which the lane's evaluation started
     float r = 0.0f, t = 0.0f;
     float pos[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f};
-    uint32_t c_next = 0, c_end = 0, round = 0;
+    Window win;
     bool exhausted = false;
     WorkTally<kCount> tally;
 
@@ -221,21 +221,16 @@ __global__ __launch_bounds__(256) void k_trace(
         uint64_t need = wave & ~ray_m;
         if (!exhausted && (uint32_t)__popcll(need) >= q.refill_min) {
             while (need != 0) {
-                if (c_next >= c_end) {
-                    const uint32_t b = next_chunk(q, round);
-                    if (b >= q.total) {
-                        exhausted = true;
-                        break;
-                    }
-                    c_next = b;
-                    c_end = (q.total - b < q.chunk) ? q.total : b + q.chunk;
+                if (win.next >= win.end && !next_chunk(q, win)) {
+                    exhausted = true;
+                    break;
                 }
-                const uint32_t avail = c_end - c_next;
+                const uint32_t avail = win.end - win.next;
                 const uint32_t nneed = (uint32_t)__popcll(need);
                 const uint32_t rank = lane_rank(need);
                 const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
                 if (take) {
-                    idx = c_next + rank;
+                    idx = win.next + rank;
                     rays.get(idx, pos, dir);
                     t = 0.0f;
                     nsteps = 0;
@@ -250,7 +245,7 @@ __global__ __launch_bounds__(256) void k_trace(
                 step_m |= zero;
                 ray_m |= took;
                 need &= ~took;
-                c_next += (nneed < avail) ? nneed : avail;
+                win.next += (nneed < avail) ? nneed : avail;
             }
         }
         // Every lane with a ray is live or has a step due; none left means

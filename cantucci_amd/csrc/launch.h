@@ -33,24 +33,37 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
     if (iters) iters[i] = 0;
 }
 
+// Waves per CU that a small launch is spread over (8 per SIMD, what the P8
+// kernels can hold).  At the configured chunk alone a 64^3 grid was 256
+// workgroups, one wave per SIMD, and took 25 us; filled, 10 us.  One leaf's
+// 65^3 corners: 60 -> 11 us; its 9,868 vertices' taps: 249 -> 26 us.
+constexpr uint64_t kFillWaves = 32;
+
 inline WorkQueue make_queue(Ctx& c, uint32_t total, const LaunchShape& ls, uint32_t& blocks, hipStream_t st) {
-    uint32_t waves_per_block = (uint32_t)ls.block / 64u;
-    uint64_t want = (uint64_t)c.num_cus * (uint64_t)ls.blocks_per_cu;
-    uint64_t need = ((uint64_t)total + (uint64_t)ls.chunk * waves_per_block - 1) / ((uint64_t)ls.chunk * waves_per_block);
-    blocks = (uint32_t)std::max<uint64_t>(1, std::min(want, need));
+    // Workgroups: enough for the configured chunks, and for a small launch
+    // enough that its 64-index chunks fill kFillWaves waves per CU.
+    const uint64_t waves_per_block = (uint64_t)ls.block / 64u;
+    const uint64_t per_block = 64u * waves_per_block;
+    const uint64_t want = (uint64_t)c.num_cus * (uint64_t)ls.blocks_per_cu;
+    const uint64_t full = ((uint64_t)total + ls.chunk * waves_per_block - 1) / (ls.chunk * waves_per_block);
+    const uint64_t fill = std::min(((uint64_t)total + per_block - 1) / per_block,
+                                   (uint64_t)c.num_cus * kFillWaves / waves_per_block);
+    blocks = (uint32_t)std::max<uint64_t>(1, std::min(want, std::max(full, fill)));
     WorkQueue q;
-    uint32_t* pair = c.take_counters(st);
-    q.next = pair;
-    q.done = pair + 1;
-    q.waves = blocks * waves_per_block;
+    q.waves = blocks * (uint32_t)waves_per_block;
     q.total = total;
     // At least ~8 chunks per wave, so that small launches still balance:
     // chunk = clamp(total / (8 waves), 64, configured), a multiple of 64.
     uint64_t fair = (uint64_t)total / ((uint64_t)q.waves * 8u);
     uint64_t ch = std::min<uint64_t>(ls.chunk, std::max<uint64_t>(64, fair));
     q.chunk = (uint32_t)(ch & ~63ull);
+    q.chunks = (uint32_t)(((uint64_t)total + q.chunk - 1) / q.chunk);
     q.refill_min = ls.refill_min < 1 ? 1 : (ls.refill_min > 64 ? 64 : ls.refill_min);
-    q.dynamic = ls.dynamic ? 1u : 0u;
+    // Only chunks beyond every wave's first are claimed.
+    q.dynamic = ls.dynamic && q.chunks > q.waves ? 1u : 0u;
+    q.shards = 1;
+    while (q.shards < kMaxShards && 2 * q.shards <= blocks) q.shards *= 2;
+    q.ctr = q.dynamic ? c.take_counters(st) : nullptr;
     q.stats = c.stats;
     return q;
 }
