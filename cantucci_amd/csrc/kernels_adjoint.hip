@@ -89,6 +89,7 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
                     }
                 }
                 win.next += (nneed < avail) ? nneed : avail;
+                if (!refill_again(nneed, avail, wave_mask(live), ~0ull, q)) break;
             }
             if (wave_mask(live) == 0) break;
             if (exhausted || win.drained()) refill_at = 64u;
@@ -340,6 +341,7 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
                     }
                 }
                 win.next += (nneed < avail) ? nneed : avail;
+                if (!refill_again(nneed, avail, wave_mask(live), ~0ull, q)) break;
             }
             if (wave_mask(live) == 0) break;
             if (exhausted || win.drained()) refill_at = 64u;

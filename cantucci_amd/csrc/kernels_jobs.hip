@@ -133,6 +133,7 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
                 }
                 live_m |= wave_mask(take) & ~wave_mask(r > u.bailout);
                 win.next += (nneed < avail) ? nneed : avail;
+                if (!refill_again(nneed, avail, live_m, wave, q)) break;
             }
             if (live_m == 0) break;
             if (exhausted || win.drained()) refill_at = (uint32_t)__popcll(wave);
