@@ -46,7 +46,7 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
     Ev ev;
     bool live = false, hold = false;
     uint32_t idx = 0, k = 0;
-    float r = 0.0f;
+    float r = idle_start(ev, u);
     Window win;
     bool exhausted = false;
     uint32_t refill_at = q.refill_min;

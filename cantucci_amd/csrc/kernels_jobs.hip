@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
     // The wave's body count, and per lane the tick of its point's last body
     // (the job's cap counted from the tick at which the lane took the point).
     uint32_t tick = 0, tcap = 0;
-    float r = 0.0f;
+    float r = idle_start(ev, u);
     Window win;
     bool exhausted = false;
     uint32_t refill_at = q.refill_min;

@@ -797,7 +797,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
     bool has_v = false;
     uint32_t vid = 0, t = 0;
     uint32_t tick = 0, t0 = 0;  // wave's body count; tick at which the lane's tap started
-    float r = 0.0f;
+    float r = idle_start(ev, u);
     Window win;
     bool exhausted = false;
     WorkTally<kCount> tally;

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_trace(
     bool has_ray = false;
     uint32_t idx = 0, nsteps = 0;
     uint32_t tick = 0, t0 = 0;  // wave's body count; tick at which the lane's evaluation started
-    float r = 0.0f, t = 0.0f;
+    float r = idle_start(ev, u), t = 0.0f;
     float pos[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f};
     Window win;
     bool exhausted = false;

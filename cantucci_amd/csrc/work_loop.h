@@ -185,7 +185,7 @@ __device__ __forceinline__ void refill_loop(const Src& src, const MandelUniform&
     uint32_t idx = 0;
     uint32_t t0 = 0;      // tick at which the lane took its point
     uint32_t kh = 0;      // body count of a held point (kept if the sink reads it)
-    float r = 0.0f;
+    float r = idle_start(ev, u);
     Window win;
     bool exhausted = false;
     uint32_t refill_at = q.refill_min;  // idle lanes that trigger the next refill
