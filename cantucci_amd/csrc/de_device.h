@@ -198,11 +198,19 @@ struct MandelUniform {
     float radius;
 };
 
+// How an evaluator's launches spread over the chip, in waves per CU
+// (make_queue): a small launch to `fill` waves, no launch beyond `most` (as
+// many as are resident, where later workgroups measured slower).
+struct WaveSpread {
+    uint32_t fill, most;
+};
+
 // ---------------------------------------------------------------------------
 // Exact P8 polynomial evaluator (reference `Mandelbulb<8>`)
 // ---------------------------------------------------------------------------
 struct P8Exact {
     static constexpr int kWavesPerSimd = 8;  // fits 64 VGPRs in the refill kernel
+    static constexpr WaveSpread kSpread{32, ~0u};
     // The evaluator has last_dr(): the work loops end a point that reaches
     // the iteration cap after max_iters - 1 bodies and apply the last body's
     // dr update alone (see last_dr).
@@ -429,6 +437,7 @@ struct P8Contract : P8Exact {
 // ---------------------------------------------------------------------------
 struct TrigExact {
     static constexpr int kWavesPerSimd = 1;  // no constraint (64 VGPRs would spill)
+    static constexpr WaveSpread kSpread{16, ~0u};
     static constexpr bool kLastDr = true;
     float px, py, pz, x, y, z, dr, P;
     int Pi;       // integer power of the powi ladder (when `ladder`)

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
                 if (!refill_again(nneed, avail, wave_mask(live), ~0ull, q)) break;
             }
             if (wave_mask(live) == 0) break;
-            if (exhausted || win.drained()) refill_at = 64u;
+            refill_at = win.refill_at(q, exhausted);
         }
         if (live) orbit[(size_t)idx * stride + k] = make_float4(ev.x, ev.y, ev.z, ev.dr);
         ev.body(r, u, live);
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
                 if (!refill_again(nneed, avail, wave_mask(live), ~0ull, q)) break;
             }
             if (wave_mask(live) == 0) break;
-            if (exhausted || win.drained()) refill_at = 64u;
+            refill_at = win.refill_at(q, exhausted);
         }
         if (live) {
             float4 s = orbit[(size_t)idx * stride + j];
@@ -482,7 +482,8 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
         SrcPoints src{pts + 3 * off, powers ? powers + off : nullptr, s.power};
         // kernel 1: parity forward with orbit recording
         uint32_t blocks = 0;
-        WorkQueue q = make_queue(c, m, c.shape_adj, blocks, st);
+        const WaveSpread spread = family == FAM_P8 ? P8Exact::kSpread : TrigExact::kSpread;
+        WorkQueue q = make_queue(c, m, c.shape_adj, spread, blocks, st);
         if (family == FAM_P8)
             hipLaunchKernelGGL((k_adj_forward<P8Exact>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src, u, orbit, rec,
                                d ? d + off : nullptr, q);
@@ -495,7 +496,7 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
         AdjOut out{grad_d ? grad_d + off : nullptr,         grad_p ? grad_p + 3 * off : nullptr,
                    grad_power ? grad_power + off : nullptr, normals ? normals + 3 * off : nullptr,
                    grad_z0 ? grad_z0 + 3 * off : nullptr,   grad_c ? grad_c + 3 * off : nullptr};
-        WorkQueue q2 = make_queue(c, m, c.shape_adj, blocks, st);
+        WorkQueue q2 = make_queue(c, m, c.shape_adj, spread, blocks, st);
         if (family == FAM_P8)
             hipLaunchKernelGGL((k_adj_reverse<false>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src, u, orbit, rec,
                                out, q2);
@@ -522,7 +523,8 @@ int launch_tangent(Ctx& c, const cth_shape& s, const float* pts, const float* po
     SrcPoints src{pts, powers, s.power};
     SinkGrad sink{d, normals, grad_p, grad_power, grad_d, u.max_iters};
     uint32_t blocks = 0;
-    WorkQueue q = make_queue(c, n, c.shape_adj, blocks, st);
+    WorkQueue q = make_queue(c, n, c.shape_adj, family == FAM_P8 ? P8Tangent::kSpread : TrigNormal::kSpread,
+                             blocks, st);
     if (family == FAM_P8)
         hipLaunchKernelGGL((k_refill<P8Tangent, SrcPoints, SinkGrad>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src,
                            u, sink, q);

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
                 if (!refill_again(nneed, avail, live_m, wave, q)) break;
             }
             if (live_m == 0) break;
-            if (exhausted || win.drained()) refill_at = (uint32_t)__popcll(wave);
+            refill_at = win.refill_at(q, exhausted);
         }
         const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
         const uint64_t cap_m = wave_mask(tcap == tick) & live_m;
@@ -240,7 +240,8 @@ int jobs_run(Ctx& c, const JobSet& js, float* dists, float* normals, unsigned lo
     int rc = check_hip(hipGetLastError(), "jobs reset launch");
     if (rc) return rc;
     uint32_t blocks = 0;
-    WorkQueue q = make_queue(c, js.total, c.shape_jobs, blocks, st);
+    WorkQueue q = make_queue(c, js.total, c.shape_jobs,
+                             js.kind == CTH_SHAPE_MANDELBULB ? P8Tangent::kSpread : TrigNormal::kSpread, blocks, st);
     if (js.kind == CTH_SHAPE_MANDELBULB)
         hipLaunchKernelGGL((k_jobs<P8Tangent>), dim3(blocks), dim3(c.shape_jobs.block), 0, st, js.dev, js.njobs, u,
                            dists, normals, done, start, q);

@@ -1098,7 +1098,8 @@ int mesh_vertices(Ctx& c, const cth_shape& s, int normals, uint64_t nverts, floa
     if (normals == CTH_NORMALS_TANGENT) {
         if (nverts >= (1ull << 31)) return fail(CTH_E_INVALID, "more than 2^31 vertices");
         uint32_t blocks = 0;
-        WorkQueue q = make_queue(c, (uint32_t)nverts, c.shape_mesh, blocks, st);
+        WorkQueue q = make_queue(c, (uint32_t)nverts, c.shape_mesh,
+                                 family == FAM_P8 ? P8Tangent::kSpread : TrigNormal::kSpread, blocks, st);
         SrcMeshVerts src{verts, s.power};
         SinkMeshVerts sink{verts, u.max_iters};
         if (family == FAM_P8)
@@ -1115,7 +1116,8 @@ int mesh_vertices(Ctx& c, const cth_shape& s, int normals, uint64_t nverts, floa
     if (family != FAM_SPHERE) {
         if (nverts >= (1ull << 31)) return fail(CTH_E_INVALID, "more than 2^31 vertices");
         uint32_t blocks = 0;
-        WorkQueue q = make_queue(c, (uint32_t)nverts, c.shape_mesh, blocks, st);
+        WorkQueue q = make_queue(c, (uint32_t)nverts, c.shape_mesh,
+                                 family == FAM_P8 ? P8Exact::kSpread : TrigExact::kSpread, blocks, st);
         dim3 grid(blocks), block(c.shape_mesh.block);
         if (family == FAM_P8) {
             with_p8(c.mode, [&](auto ev) {

@@ -308,7 +308,8 @@ static int run_trace(Ctx& c, const cth_shape& s, const Rays& rays, uint32_t tota
         if (rc) return rc;
     }
     uint32_t blocks = 0;
-    WorkQueue q = make_queue(c, total, c.shape_trace, blocks, st);
+    WorkQueue q = make_queue(c, total, c.shape_trace, family == FAM_P8 ? P8Exact::kSpread : TrigExact::kSpread,
+                             blocks, st);
     dim3 grid(blocks), block(c.shape_trace.block);
     if (family == FAM_SPHERE) {
         hipLaunchKernelGGL((k_trace<SphereEv, Rays>), grid, block, 0, st, rays, u, tp, out, q);

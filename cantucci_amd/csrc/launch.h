@@ -33,26 +33,29 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
     if (iters) iters[i] = 0;
 }
 
-// Waves per CU that a small launch is spread over (8 per SIMD, what the P8
-// kernels can hold).  At the configured chunk alone a 64^3 grid was 256
-// workgroups, one wave per SIMD, and took 25 us; filled, 10 us.  One leaf's
-// 65^3 corners: 60 -> 11 us; its 9,868 vertices' taps: 249 -> 26 us.
-constexpr uint64_t kFillWaves = 32;
-
-inline WorkQueue make_queue(Ctx& c, uint32_t total, const LaunchShape& ls, uint32_t& blocks, hipStream_t st) {
-    // Workgroups: enough for the configured chunks, and for a small launch
-    // enough that its 64-index chunks fill kFillWaves waves per CU.
-    const uint64_t waves_per_block = (uint64_t)ls.block / 64u;
-    const uint64_t per_block = 64u * waves_per_block;
-    const uint64_t want = (uint64_t)c.num_cus * (uint64_t)ls.blocks_per_cu;
-    const uint64_t full = ((uint64_t)total + ls.chunk * waves_per_block - 1) / (ls.chunk * waves_per_block);
-    const uint64_t fill = std::min(((uint64_t)total + per_block - 1) / per_block,
-                                   (uint64_t)c.num_cus * kFillWaves / waves_per_block);
-    blocks = (uint32_t)std::max<uint64_t>(1, std::min(want, std::max(full, fill)));
+// A launch's workgroups and chunks.  Up to a chunk of 64 indices for each of
+// spread.fill waves per CU a launch is spread as thinly as possible; from four
+// chunks per wave on it grows to the launch shape's (and spread.most) waves.
+// In between it stays at `fill`: a lane that takes a second point while its
+// wave's slowest is still iterating costs little, more waves on a SIMD cost
+// their share of its issue slots.
+//
+// Measured on the default shapes, us per launch (in parentheses with the
+// workgroup count taken from the configured 256-index chunk): 64^3 grid 10.5
+// (24.6), 2 M points at power 8 34.5 (47), 700,000 at power 5 33 (49; 47 at
+// fill 32), tangent normals of 300,000 points with powers 48 (68; 69 at fill
+// 16), of 2 M points 153 (195; 175 without `most`).
+inline WorkQueue make_queue(Ctx& c, uint32_t total, const LaunchShape& ls, WaveSpread spread, uint32_t& blocks,
+                            hipStream_t st) {
+    const uint64_t cus = (uint64_t)c.num_cus, waves_per_block = (uint64_t)ls.block / 64u;
+    const uint64_t chunks64 = ((uint64_t)total + 63u) / 64u;
+    uint64_t waves = std::max(std::min(chunks64, cus * spread.fill), std::min(chunks64 / 4u, cus * spread.most));
+    blocks = (uint32_t)std::max<uint64_t>(
+        1, std::min(cus * (uint64_t)ls.blocks_per_cu, (waves + waves_per_block - 1) / waves_per_block));
     WorkQueue q;
     q.waves = blocks * (uint32_t)waves_per_block;
     q.total = total;
-    // At least ~8 chunks per wave, so that small launches still balance:
+    // At least ~8 chunks per wave, so that launches still balance:
     // chunk = clamp(total / (8 waves), 64, configured), a multiple of 64.
     uint64_t fair = (uint64_t)total / ((uint64_t)q.waves * 8u);
     uint64_t ch = std::min<uint64_t>(ls.chunk, std::max<uint64_t>(64, fair));
@@ -72,7 +75,7 @@ template <class Src, class Sink>
 inline int run_refill(Ctx& c, int family, const MandelUniform& u, const Src& src, const Sink& sink,
                       uint32_t total, hipStream_t st, const LaunchShape& ls) {
     uint32_t blocks = 0;
-    WorkQueue q = make_queue(c, total, ls, blocks, st);
+    WorkQueue q = make_queue(c, total, ls, family == FAM_P8 ? P8Exact::kSpread : TrigExact::kSpread, blocks, st);
     dim3 grid(blocks), block(ls.block);
     if (family == FAM_P8) {
         with_p8(c.mode, [&](auto ev) {

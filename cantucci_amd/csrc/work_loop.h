@@ -90,9 +90,13 @@ struct Window {
     uint32_t next = 0, end = 0;  // indices not handed out yet
     uint32_t round = 0;          // chunks taken
     bool last = false;           // no chunk follows the current one
-    // Known to hold no index any more: a wave then writes its held points once
-    // all its lanes are idle (a batch that could not take new points anyway).
-    __device__ __forceinline__ bool drained() const { return last && next >= end; }
+    // Idle lanes that trigger the wave's next refill: refill_min, or as few as
+    // take the whole rest of the wave's last chunk, or, with no index left, the
+    // whole wave (a batch that could not take new points is only written).
+    __device__ __forceinline__ uint32_t refill_at(const WorkQueue& q, bool exhausted) const {
+        if (exhausted || (last && next >= end)) return 64u;
+        return last && end - next < q.refill_min ? end - next : q.refill_min;
+    }
 };
 
 // The next chunk of the wave; false when the index space is exhausted.
@@ -245,7 +249,7 @@ __device__ __forceinline__ void refill_loop(const Src& src, const MandelUniform&
                 if (!refill_again(nneed, avail, live_m, wave, q)) break;
             }
             if (live_m == 0) break;
-            if (exhausted || win.drained()) refill_at = (uint32_t)__popcll(wave);
+            refill_at = win.refill_at(q, exhausted);
             tick_guard(ev, u);  // the started points' squares
         }
         const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
