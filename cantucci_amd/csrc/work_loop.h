@@ -27,6 +27,7 @@ struct WorkQueue {
     uint32_t total;    // indices in [0, total)
     uint32_t chunk;    // indices per chunk
     uint32_t chunks;   // ceil(total / chunk)
+    uint32_t rotate;   // a wave's step from row to row of `waves` chunks (static), below `waves`
     uint32_t refill_min;  // idle lanes that trigger a write-back + refill (1..64)
     uint32_t dynamic;     // 1: claim chunks after the first with an atomic; 0: static interleave
     // Work counters (nullable): the launch adds its loop bodies, its
@@ -85,10 +86,13 @@ __device__ __forceinline__ uint32_t wave_id() {
     return blockIdx.x * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
+constexpr uint32_t kNoChunk = ~0u;
+
 // The wave's window of claimed indices (wave-uniform, scalar registers).
 struct Window {
     uint32_t next = 0, end = 0;  // indices not handed out yet
-    uint32_t round = 0;          // chunks taken
+    uint32_t row = 0;            // first chunk of the row of `waves` chunks it takes one of (static)
+    uint32_t pos = kNoChunk;     // its place in that row; kNoChunk before the first chunk
     bool last = false;           // no chunk follows the current one
     // Idle lanes that trigger the wave's next refill: refill_min, or as few as
     // take the whole rest of the wave's last chunk, or, with no index left, the
@@ -102,9 +106,11 @@ struct Window {
 // The next chunk of the wave; false when the index space is exhausted.
 // Chunk w goes to wave w first, so that a launch starts without claims and one
 // that has no more chunks than waves makes none.  Further chunks are, static,
-// w + W, w + 2W, ... (W waves: every wave is spread over the whole domain, so
-// that slow and fast regions average out); dynamic, the next unclaimed chunk
-// of the workgroup's shard.  Claims on one counter serialise at about 14 ns
+// one of each further row of W chunks (W waves: every wave is spread over the
+// whole domain, so that slow and fast regions average out; its place moves by
+// `rotate` from row to row, so that a row length that fits the domain, 4096
+// waves of 256 indices in 128^3 grids, does not give a wave the same region
+// every time); dynamic, the next unclaimed chunk of the workgroup's shard.  Claims on one counter serialise at about 14 ns
 // each, whatever the number of waves (17.6 M corners in 68,600 chunks of 256
 // took 971 us, and 137 us with 32 shards), hence the shards: row j of the
 // remaining chunks holds one for each shard, rotated from row to row so that
@@ -112,19 +118,27 @@ struct Window {
 __device__ __forceinline__ bool next_chunk(const WorkQueue& q, Window& w) {
     if (w.last) return false;
     uint32_t c;
-    if (!q.dynamic || w.round == 0) {
-        c = w.round * q.waves + wave_id();
+    if (w.pos == kNoChunk) {
+        w.pos = c = wave_id();
+    } else if (!q.dynamic) {
+        w.row += q.waves;
+        w.pos += q.rotate;
+        if (w.pos >= q.waves) w.pos -= q.waves;
+        c = w.row + w.pos;
     } else {
         const uint32_t s = blockIdx.x & (q.shards - 1u);
         const uint32_t j = wave_claim(q.ctr + s * kShardStride, 1u);
         c = q.waves + j * q.shards + ((s + 11u * j) & (q.shards - 1u));
     }
-    ++w.round;
     w.last = c >= q.chunks;
     if (w.last) return false;
     w.next = c * q.chunk;
     w.end = (q.total - w.next < q.chunk) ? q.total : w.next + q.chunk;
-    if (!q.dynamic) w.last = q.chunks - c <= q.waves;
+    if (!q.dynamic) {
+        uint32_t p = w.pos + q.rotate;
+        if (p >= q.waves) p -= q.waves;
+        w.last = w.row + q.waves + p >= q.chunks;
+    }
     return true;
 }
 
