@@ -15,6 +15,8 @@
 // one), a ray escapes when t > t_max (+inf: never, like the reference).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "internal.h"
 #include "launch.h"
 #include "point_sources.h"
@@ -307,9 +309,17 @@ static int run_trace(Ctx& c, const cth_shape& s, const Rays& rays, uint32_t tota
         int rc = resolve_mandel(s, u, family);
         if (rc) return rc;
     }
+    // Few rays go a few to a wave (at most kSmallWaves waves per CU): a ray is a
+    // chain of up to max_steps evaluations, and rays that share a wave wait for
+    // each other's slowest.  25 focus rays, all in one wave before: 207 -> 163 us
+    // (6 iterations), 298 -> 183 us (15); 64 x 25: 768 -> 284 us; 16 waves per CU
+    // were slower from 256 x 25 rays on.
+    constexpr uint64_t kSmallWaves = 8;
+    const uint64_t small = (uint64_t)c.num_cus * kSmallWaves;
+    const uint32_t least = (uint32_t)std::min<uint64_t>(64, (total + small - 1) / small);
     uint32_t blocks = 0;
     WorkQueue q = make_queue(c, total, c.shape_trace, family == FAM_P8 ? P8Exact::kSpread : TrigExact::kSpread,
-                             blocks, st);
+                             blocks, st, least);
     dim3 grid(blocks), block(c.shape_trace.block);
     if (family == FAM_SPHERE) {
         hipLaunchKernelGGL((k_trace<SphereEv, Rays>), grid, block, 0, st, rays, u, tp, out, q);

@@ -33,8 +33,8 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
     if (iters) iters[i] = 0;
 }
 
-// A launch's workgroups and chunks.  Up to a chunk of 64 indices for each of
-// spread.fill waves per CU a launch is spread as thinly as possible; from four
+// A launch's workgroups and chunks.  Up to a chunk of `least` indices (64 or
+// fewer) for each of spread.fill waves per CU a launch is spread as thinly as possible; from four
 // chunks per wave on it grows to the launch shape's (and spread.most) waves.
 // In between it stays at `fill`: a lane that takes a second point while its
 // wave's slowest is still iterating costs little, more waves on a SIMD cost
@@ -46,10 +46,10 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
 // fill 32), tangent normals of 300,000 points with powers 48 (68; 69 at fill
 // 16), of 2 M points 153 (195; 175 without `most`).
 inline WorkQueue make_queue(Ctx& c, uint32_t total, const LaunchShape& ls, WaveSpread spread, uint32_t& blocks,
-                            hipStream_t st) {
+                            hipStream_t st, uint32_t least = 64) {
     const uint64_t cus = (uint64_t)c.num_cus, waves_per_block = (uint64_t)ls.block / 64u;
-    const uint64_t chunks64 = ((uint64_t)total + 63u) / 64u;
-    uint64_t waves = std::max(std::min(chunks64, cus * spread.fill), std::min(chunks64 / 4u, cus * spread.most));
+    const uint64_t small = ((uint64_t)total + least - 1) / least;
+    uint64_t waves = std::max(std::min(small, cus * spread.fill), std::min(small / 4u, cus * spread.most));
     blocks = (uint32_t)std::max<uint64_t>(
         1, std::min(cus * (uint64_t)ls.blocks_per_cu, (waves + waves_per_block - 1) / waves_per_block));
     WorkQueue q;
@@ -59,7 +59,7 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, const LaunchShape& ls, WaveS
     // chunk = clamp(total / (8 waves), 64, configured), a multiple of 64.
     uint64_t fair = (uint64_t)total / ((uint64_t)q.waves * 8u);
     uint64_t ch = std::min<uint64_t>(ls.chunk, std::max<uint64_t>(64, fair));
-    q.chunk = (uint32_t)(ch & ~63ull);
+    q.chunk = least < 64 ? least : (uint32_t)(ch & ~63ull);
     q.chunks = (uint32_t)(((uint64_t)total + q.chunk - 1) / q.chunk);
     q.refill_min = ls.refill_min < 1 ? 1 : (ls.refill_min > 64 ? 64 : ls.refill_min);
     // Only chunks beyond every wave's first are claimed.
