@@ -44,67 +44,57 @@ __global__ __launch_bounds__(256) void k_adj_forward(SrcPoints src, MandelUnifor
                                                      AdjRecord* __restrict__ rec, float* __restrict__ dout,
                                                      WorkQueue q) {
     Ev ev;
-    bool live = false, hold = false;
+    uint64_t live_m = 0, hold_m = 0;  // as in refill_loop
     uint32_t idx = 0, k = 0;
     float r = idle_start(ev, u);
     Window win;
-    bool exhausted = false;
-    uint32_t refill_at = q.refill_min;
     const size_t stride = (size_t)u.max_iters + 1;
     for (;;) {
-        if ((uint32_t)__popcll(wave_mask(!live)) >= refill_at) {
-            if (hold) {
+        do {
+            if (__builtin_amdgcn_inverse_ballot_w64(hold_m)) {
                 float d = ev.finish(r);
                 if (dout) dout[idx] = d;
                 rec[idx] = AdjRecord{k, r, ev.dr, 0.0f};
                 // z_K (the state the bailout magnitude was taken of)
-                orbit[(size_t)idx * stride + k] = make_float4(ev.x, ev.y, ev.z, ev.dr);
-                hold = false;
+                if (k != 0) orbit[(size_t)idx * stride + k] = make_float4(ev.x, ev.y, ev.z, ev.dr);
             }
-            while (!exhausted) {
-                uint64_t need = wave_mask(!live);
-                if (need == 0) break;
-                if (win.next >= win.end && !next_chunk(q, win)) {
-                    exhausted = true;
-                    break;
+            hold_m = 0;
+            uint64_t need = ~live_m;
+            while (need != 0) {
+                if (win.next >= win.end && !next_chunk(q, win)) break;
+                const uint32_t avail = win.end - win.next;
+                const uint32_t nneed = (uint32_t)__popcll(need);
+                const uint32_t rank = lane_rank(need);
+                const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
+                if (take) {
+                    idx = win.next + rank;
+                    float px, py, pz, pw;
+                    src.get(idx, px, py, pz, pw);
+                    ev.start(px, py, pz, pw, u);
+                    k = 0;
+                    r = ev.mag();
                 }
-                uint32_t avail = win.end - win.next;
-                uint32_t nneed = (uint32_t)__popcll(need);
-                if (!live) {
-                    uint32_t rank = lane_rank(need);
-                    if (rank < avail) {
-                        idx = win.next + rank;
-                        float px, py, pz, pw;
-                        src.get(idx, px, py, pz, pw);
-                        ev.start(px, py, pz, pw, u);
-                        k = 0;
-                        r = ev.mag();
-                        if (r > u.bailout) {
-                            float d = ev.finish(r);
-                            if (dout) dout[idx] = d;
-                            rec[idx] = AdjRecord{0u, r, ev.dr, 0.0f};
-                        } else {
-                            live = true;
-                        }
-                    }
-                }
+                const uint64_t took = wave_mask(take);
+                const uint64_t bailed = wave_mask(r > u.bailout) & took;
+                hold_m |= bailed;
+                live_m |= took & ~bailed;
+                need &= ~took;
                 win.next += (nneed < avail) ? nneed : avail;
-                if (!refill_again(nneed, avail, wave_mask(live), ~0ull, q)) break;
             }
-            if (wave_mask(live) == 0) break;
-            refill_at = win.refill_at(q, exhausted);
-        }
-        if (live) orbit[(size_t)idx * stride + k] = make_float4(ev.x, ev.y, ev.z, ev.dr);
-        ev.body(r, u, live);
-        k += live ? 1u : 0u;
-        bool cap = live && (k == u.max_iters);
-        float rn = ev.mag();
-        bool bail = live && !cap && (rn > u.bailout);
-        if (live && !cap) r = rn;
-        if (cap || bail) {
-            live = false;
-            hold = true;
-        }
+        } while (live_m == 0 && hold_m != 0);
+        if (live_m == 0) break;
+        const uint32_t limit = 64u - win.refill_at(q);
+        do {
+            if (__builtin_amdgcn_inverse_ballot_w64(live_m)) {
+                orbit[(size_t)idx * stride + k] = make_float4(ev.x, ev.y, ev.z, ev.dr);
+                ++k;
+            }
+            const uint64_t cap_m = wave_mask(k == u.max_iters) & live_m;
+            const float rn = tick_full(ev, r, u, live_m, cap_m);
+            const uint64_t done_m = cap_m | (wave_mask(rn > u.bailout) & live_m);
+            live_m &= ~done_m;
+            hold_m |= done_m;
+        } while ((uint32_t)__popcll(live_m) > limit);
     }
     if (q.dynamic) wave_retire(q);
 }
@@ -289,22 +279,18 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
     float zbx = 0.0f, zby = 0.0f, zbz = 0.0f, drb = 0.0f, cbx = 0.0f, cby = 0.0f, cbz = 0.0f, Pb = 0.0f;
     float rb_extra = 0.0f;
     Window win;
-    bool exhausted = false;
     uint32_t refill_at = q.refill_min;
     const size_t stride = (size_t)u.max_iters + 1;
     for (;;) {
         if ((uint32_t)__popcll(wave_mask(!live)) >= refill_at) {
-            while (!exhausted) {
-                uint64_t need = wave_mask(!live);
-                if (need == 0) break;
-                if (win.next >= win.end && !next_chunk(q, win)) {
-                    exhausted = true;
-                    break;
-                }
+            uint64_t need = wave_mask(!live);
+            bool any = false;
+            while (need != 0) {
+                if (win.next >= win.end && !next_chunk(q, win)) break;
                 uint32_t avail = win.end - win.next;
                 uint32_t nneed = (uint32_t)__popcll(need);
-                if (!live) {
-                    uint32_t rank = lane_rank(need);
+                const uint32_t rank = lane_rank(need);
+                if (__builtin_amdgcn_inverse_ballot_w64(need)) {
                     if (rank < avail) {
                         idx = win.next + rank;
                         src.get(idx, px, py, pz, P);
@@ -340,11 +326,15 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
                         }
                     }
                 }
+                need &= ~(wave_mask(rank < avail) & need);
+                any = true;
                 win.next += (nneed < avail) ? nneed : avail;
-                if (!refill_again(nneed, avail, wave_mask(live), ~0ull, q)) break;
             }
-            if (wave_mask(live) == 0) break;
-            refill_at = win.refill_at(q, exhausted);
+            if (wave_mask(live) == 0) {
+                if (!any) break;
+                continue;
+            }
+            refill_at = win.refill_at(q);
         }
         if (live) {
             float4 s = orbit[(size_t)idx * stride + j];
@@ -553,7 +543,7 @@ int launch_fd_normals(Ctx& c, const cth_shape& s, const float* pts, const float*
         MandelUniform u;
         int family = 0;
         rc = resolve_mandel(s, u, family);
-        if (!rc) rc = run_refill(c, family, u, src, SinkDist{taps, nullptr}, n * 7, st, c.shape_de);
+        if (!rc) rc = run_refill(c, family, u, src, SinkDist{taps}, n * 7, st, c.shape_de);
     }
     if (!rc) {
         hipLaunchKernelGGL(k_fd_combine, dim3(cdiv_adj(n, 256)), dim3(256), 0, st, taps, n, normals, grad_p, d,

@@ -92,8 +92,7 @@ int launch_de_points(Ctx& c, const cth_shape& s, const float* pts, const float* 
         SinkState sink{r_out, dr_out, iters};
         return run_refill(c, family, u, src, sink, n, st, c.shape_de);
     }
-    SinkDist sink{out, iters};
-    return run_refill(c, family, u, src, sink, n, st, c.shape_de);
+    return run_dist(c, family, u, src, out, iters, n, st, c.shape_de);
 }
 
 static bool is_pow2_float(float v, float& inv) {
@@ -131,8 +130,7 @@ int launch_de_grid(Ctx& c, const cth_shape& s, const float* start, const float* 
     int family = 0;
     int rc = resolve_mandel(s, u, family);
     if (rc != CTH_OK) return rc;
-    SinkDist sink{out, iters};
-    return run_refill(c, family, u, src, sink, (uint32_t)total, st, c.shape_de);
+    return run_dist(c, family, u, src, out, iters, (uint32_t)total, st, c.shape_de);
 }
 
 int launch_sample_spans(Ctx& c, const cth_shape& s, const float* spans, uint32_t nspans, uint32_t res, float* dists,
@@ -161,8 +159,7 @@ int launch_sample_spans(Ctx& c, const cth_shape& s, const float* spans, uint32_t
         int family = 0;
         rc = resolve_mandel(s, u, family);
         if (rc != CTH_OK) return rc;
-        SinkDist sink{dists, iters};
-        rc = run_refill(c, family, u, src, sink, (uint32_t)total, st, c.shape_spans);
+        rc = run_dist(c, family, u, src, dists, iters, (uint32_t)total, st, c.shape_spans);
     }
     if (rc != CTH_OK || cross == nullptr) return rc;
     uint32_t res_log2 = 0;

@@ -76,12 +76,10 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
     unsigned long long stamp = 0;
     float r = idle_start(ev, u);
     Window win;
-    bool exhausted = false;
-    uint32_t refill_at = q.refill_min;
     SinkGrad sink{dists, normals, nullptr, nullptr, nullptr, 0u};
 
     for (;;) {
-        if ((uint32_t)__popcll(wave & ~live_m) >= refill_at) {
+        do {
             // write back held points and note the time for their jobs
             // SinkGrad reads k only as k == max_iters (the point stopped at the cap).
             if (__builtin_amdgcn_inverse_ballot_w64(hold_m)) {
@@ -104,67 +102,60 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
             }
             hold_m = 0;
             capd_m = 0;
-            while (!exhausted) {
-                const uint64_t need = wave & ~live_m;
-                if (need == 0) break;
-                if (win.next >= win.end && !next_chunk(q, win)) {
-                    exhausted = true;
-                    break;
-                }
-                uint32_t avail = win.end - win.next;
-                uint32_t nneed = (uint32_t)__popcll(need);
+            // a point that bails before its first body is held (see refill_loop)
+            uint64_t need = wave & ~live_m;
+            while (need != 0) {
+                if (win.next >= win.end && !next_chunk(q, win)) break;
+                const uint32_t avail = win.end - win.next;
+                const uint32_t nneed = (uint32_t)__popcll(need);
                 const uint32_t rank = lane_rank(need);
                 const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
-                {
-                    if (take) {
-                        idx = win.next + rank;
-                        // job of idx: the last offset <= idx
-                        uint32_t lo = 0, hi = njobs;
-                        while (hi - lo > 1) {
-                            uint32_t mid = (lo + hi) >> 1;
-                            if (offs[mid] <= idx) lo = mid; else hi = mid;
-                        }
-                        job = lo;
-                        const JobDev& J = jobs[job];
-                        uint32_t local = idx - J.offset;
-                        uint32_t i = fdiv(local, J.n2);
-                        uint32_t rem = local - i * J.n2.d;
-                        uint32_t j = fdiv(rem, J.n);
-                        uint32_t kk = rem - j * J.n.d;
-                        uint32_t ijk[3] = {i, j, kk};
-                        float c[3];
-#pragma unroll
-                        for (int a = 0; a < 3; ++a) {
-                            float v = (J.inv != 0.0f) ? (float)ijk[a] * J.inv : div_rn((float)ijk[a], J.divisor);
-                            c[a] = J.start[a] + J.across[a] * v;
-                        }
-                        kcap = J.max_iters;
-                        tcap = tick + kcap - 1u;
-                        ev.start(c[0], c[1], c[2], J.power, u);
-                        r = ev.mag();
-                        if (r > u.bailout) {
-                            sink.max_iters = kcap;
-                            sink.put(idx, ev.finish(r), 0u, r, ev.dr, ev);
-                        }
+                if (take) {
+                    idx = win.next + rank;
+                    // job of idx: the last offset <= idx
+                    uint32_t lo = 0, hi = njobs;
+                    while (hi - lo > 1) {
+                        uint32_t mid = (lo + hi) >> 1;
+                        if (offs[mid] <= idx) lo = mid; else hi = mid;
                     }
+                    job = lo;
+                    const JobDev& J = jobs[job];
+                    uint32_t local = idx - J.offset;
+                    uint32_t i = fdiv(local, J.n2);
+                    uint32_t rem = local - i * J.n2.d;
+                    uint32_t j = fdiv(rem, J.n);
+                    uint32_t kk = rem - j * J.n.d;
+                    uint32_t ijk[3] = {i, j, kk};
+                    float c[3];
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) {
+                        float v = (J.inv != 0.0f) ? (float)ijk[a] * J.inv : div_rn((float)ijk[a], J.divisor);
+                        c[a] = J.start[a] + J.across[a] * v;
+                    }
+                    kcap = J.max_iters;
+                    tcap = tick + kcap - 1u;
+                    ev.start(c[0], c[1], c[2], J.power, u);
+                    r = ev.mag();
                 }
-                live_m |= wave_mask(take) & ~wave_mask(r > u.bailout);
+                const uint64_t took = wave_mask(take);
+                const uint64_t bailed = wave_mask(r > u.bailout) & took;
+                hold_m |= bailed;
+                live_m |= took & ~bailed;
+                need &= ~took;
                 win.next += (nneed < avail) ? nneed : avail;
-                if (!refill_again(nneed, avail, live_m, wave, q)) break;
             }
-            if (live_m == 0) break;
-            refill_at = win.refill_at(q, exhausted);
-        }
-        const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
-        const uint64_t cap_m = wave_mask(tcap == tick) & live_m;
-        ev.body(r, u, live);
-        ++tick;
-        const float rn = ev.mag();
-        const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
-        if (__builtin_amdgcn_inverse_ballot_w64(live_m & ~cap_m)) r = rn;
-        live_m &= ~(cap_m | bail_m);
-        hold_m |= cap_m | bail_m;
-        capd_m |= cap_m;
+        } while (live_m == 0 && hold_m != 0);
+        if (live_m == 0) break;
+        const uint32_t limit = 64u - win.refill_at(q);
+        do {
+            const uint64_t cap_m = wave_mask(tcap == tick) & live_m;
+            const float rn = tick_full(ev, r, u, live_m, cap_m);
+            ++tick;
+            const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
+            live_m &= ~(cap_m | bail_m);
+            hold_m |= cap_m | bail_m;
+            capd_m |= cap_m;
+        } while ((uint32_t)__popcll(live_m) > limit);
     }
     stamp_job(done, sjob, stamp);
     if (q.dynamic) wave_retire(q);

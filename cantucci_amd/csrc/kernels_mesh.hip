@@ -781,7 +781,7 @@ __device__ __forceinline__ void put_fd_normal(float* v, const float t[7]) {
 // VGPRs without spilling, and 7 waves share each SIMD (5 with the record in
 // registers); asking for 8 forces spills and is slower.
 template <class Ev, bool kCount = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_mesh_taps(float* __restrict__ verts,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_mesh_taps(float* __restrict__ verts,
                                                                                           MandelUniform u, WorkQueue q) {
     // slots 0..2: vertex position, 3..5: half-steps, 6 + t: distance of tap t
     __shared__ float lane_slots[13][256];
@@ -799,11 +799,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
     uint32_t tick = 0, t0 = 0;  // wave's body count; tick at which the lane's tap started
     float r = idle_start(ev, u);
     Window win;
-    bool exhausted = false;
     WorkTally<kCount> tally;
 
+    const uint32_t limit = 64u - q.refill_min;
     for (;;) {
-        if ((uint32_t)__popcll(wave & ~live_m) >= q.refill_min) {
+        do {
             if (__builtin_amdgcn_inverse_ballot_w64(hold_m)) {
                 if constexpr (Ev::kLastDr) {
                     if (__builtin_amdgcn_inverse_ballot_w64(last_m)) ev.last_dr(r);
@@ -813,111 +813,92 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
             }
             hold_m = 0;
             last_m = 0;
-            for (;;) {
-                // every lane here is idle; a lane with all 7 taps writes its
-                // vertex: the whole 28-byte record, position unchanged.  A
-                // 16-byte write of normal and distance alone dirties every
-                // 32-byte sector the record touches anyway (measured: 28 B
-                // per vertex written back either way), so the record is
-                // written whole and in one place.
-                if (has_v && t == 7u && !__builtin_amdgcn_inverse_ballot_w64(live_m)) {
-                    float tv[7];
+            // every idle lane's tap is stored; a lane with all 7 taps writes its
+            // vertex: the whole 28-byte record, position unchanged.  A 16-byte
+            // write of normal and distance alone dirties every 32-byte sector
+            // the record touches anyway (measured: 28 B per vertex written back
+            // either way), so the record is written whole and in one place.
+            if (has_v && t == 7u && !__builtin_amdgcn_inverse_ballot_w64(live_m)) {
+                float tv[7];
 #pragma unroll
-                    for (int j = 0; j < 7; ++j) tv[j] = slot[256 * (6 + j)];
-                    float* rec = verts + 7 * (size_t)vid;
-                    rec[0] = slot[0];
-                    rec[1] = slot[256];
-                    rec[2] = slot[512];
-                    put_fd_normal(rec, tv);
-                    has_v = false;
-                }
-                const uint64_t need = wave_mask(!has_v) & ~live_m;
-                if (need != 0 && !exhausted) {
-                    if (win.next >= win.end && !next_chunk(q, win)) exhausted = true;
-                    if (!exhausted) {
-                        const uint32_t avail = win.end - win.next;
-                        const uint32_t nneed = (uint32_t)__popcll(need);
-                        const uint32_t rank = lane_rank(need);
-                        if (__builtin_amdgcn_inverse_ballot_w64(need) && rank < avail) {
-                            vid = win.next + rank;
-                            const float* rec = verts + 7 * (size_t)vid;
-#pragma unroll
-                            for (int j = 0; j < 6; ++j) slot[256 * j] = rec[j];
-                            t = 0;
-                            has_v = true;
-                        }
-                        win.next += (nneed < avail) ? nneed : avail;
-                    }
-                }
-                const uint64_t start_m = wave_mask(has_v) & ~live_m;
-                if (start_m == 0) {
-                    if (exhausted || (wave_mask(!has_v) & ~live_m) == 0) break;
-                    continue;
-                }
-                bool now = false;  // the tap needs no full body
-                if (__builtin_amdgcn_inverse_ballot_w64(start_m)) {
-                    // tap t: p, or p + unit_a * (+-delta_a) (src/mesh/buffer.rs:259-264)
-                    float c[3] = {slot[0], slot[256], slot[512]};
-                    if (t > 0) {
-                        const int a = (int)(t - 1) >> 1;
-                        const float da = slot[256 * (3 + a)];
-                        const float h = (t & 1u) ? da : -da;
-#pragma unroll
-                        for (int b = 0; b < 3; ++b) c[b] = c[b] + ((a == b) ? 1.0f : 0.0f) * h;
-                    }
-                    ev.start(c[0], c[1], c[2], 0.0f, u);
-                    t0 = tick;
-                    r = ev.mag();
-                    now = r > u.bailout || cap0;
-                    if (now) {
-                        if constexpr (Ev::kLastDr) {
-                            if (!(r > u.bailout)) ev.last_dr(r);
-                        }
-                        slot[256 * (6 + t)] = ev.finish(r);
-                        ++t;
-                    }
-                }
-                const uint64_t zero_m = wave_mask(r > u.bailout) & start_m;
-                const uint64_t now_m = wave_mask(now) & start_m;
-                live_m |= start_m & ~now_m;
-                tally.eval(start_m);
-                tally.bail(zero_m);
-                tally.body(now_m & ~zero_m);
+                for (int j = 0; j < 7; ++j) tv[j] = slot[256 * (6 + j)];
+                float* rec = verts + 7 * (size_t)vid;
+                rec[0] = slot[0];
+                rec[1] = slot[256];
+                rec[2] = slot[512];
+                put_fd_normal(rec, tv);
+                has_v = false;
             }
-            if (live_m == 0) break;
-            tick_guard(ev, u);  // the started taps' squares
-        }
-        const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
+            uint64_t need = wave_mask(!has_v) & ~live_m;
+            while (need != 0) {
+                if (win.next >= win.end && !next_chunk(q, win)) break;
+                const uint32_t avail = win.end - win.next;
+                const uint32_t nneed = (uint32_t)__popcll(need);
+                const uint32_t rank = lane_rank(need);
+                const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
+                if (take) {
+                    vid = win.next + rank;
+                    const float* rec = verts + 7 * (size_t)vid;
+#pragma unroll
+                    for (int j = 0; j < 6; ++j) slot[256 * j] = rec[j];
+                    t = 0;
+                    has_v = true;
+                }
+                need &= ~wave_mask(take);
+                win.next += (nneed < avail) ? nneed : avail;
+            }
+            // The idle lanes that own a vertex start their next tap.  A tap that
+            // needs no full body is held until the next refill.
+            const uint64_t start_m = wave_mask(has_v) & ~live_m;
+            if (__builtin_amdgcn_inverse_ballot_w64(start_m)) {
+                // tap t: p, or p + unit_a * (+-delta_a) (src/mesh/buffer.rs:259-264)
+                float c[3] = {slot[0], slot[256], slot[512]};
+                if (t > 0) {
+                    const int a = (int)(t - 1) >> 1;
+                    const float da = slot[256 * (3 + a)];
+                    const float h = (t & 1u) ? da : -da;
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) c[b] = c[b] + ((a == b) ? 1.0f : 0.0f) * h;
+                }
+                ev.start(c[0], c[1], c[2], 0.0f, u);
+                t0 = tick;
+                r = ev.mag();
+            }
+            const uint64_t zero_m = wave_mask(r > u.bailout) & start_m;
+            last_m = cap0 ? start_m & ~zero_m : 0;
+            hold_m = zero_m | last_m;
+            live_m |= start_m & ~hold_m;
+            tally.eval(start_m);
+            tally.bail(zero_m);
+            tally.body(last_m);
+        } while (live_m == 0 && hold_m != 0);
+        if (live_m == 0) break;
+        tick_guard(ev, u);  // the started taps' squares
         if constexpr (Ev::kLastDr) {
             // as in refill_loop: a tap at the cap leaves after max_iters - 1
             // bodies and its last body's dr update is applied when it is held
-            tick_body(ev, r, u, live);
-            ++tick;
-            tally.body(live_m);
-            const float rn = tick_mag(ev, u);
-            const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m;
-            tally.bail(bail_m);
-            // Every lane takes rn: a lane without a live point ran the body
-            // without committing it, so rn is its last magnitude again, bit
-            // for bit (a held point's r, the one its finish needs).
-            r = rn;
-            const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m & ~bail_m;
-            tally.body(cap_m);
-            last_m |= cap_m;
-            live_m &= ~(cap_m | bail_m);
-            hold_m |= cap_m | bail_m;
+            run_ticks(ev, r, u, live_m, limit, [&]() {
+                ++tick;
+                tally.body(live_m);
+                const uint64_t bail_m = wave_mask(r > u.bailout) & live_m;
+                tally.bail(bail_m);
+                const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m & ~bail_m;
+                tally.body(cap_m);
+                last_m |= cap_m;
+                live_m &= ~(cap_m | bail_m);
+                hold_m |= cap_m | bail_m;
+            });
         } else {
-            const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;  // the max_iters-th body
-            tick_body(ev, r, u, live);
-            ++tick;
-            tally.body(live_m);
-            const float rn = tick_mag(ev, u);
-            const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
-            tally.bail(bail_m);
-            // at the cap r stays the magnitude before the last body (src/shape/mandelbulb.rs:65-78)
-            if (__builtin_amdgcn_inverse_ballot_w64(live_m & ~cap_m)) r = rn;
-            live_m &= ~(cap_m | bail_m);
-            hold_m |= cap_m | bail_m;
+            do {
+                const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;  // the max_iters-th body
+                const float rn = tick_full(ev, r, u, live_m, cap_m);
+                ++tick;
+                tally.body(live_m);
+                const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
+                tally.bail(bail_m);
+                live_m &= ~(cap_m | bail_m);
+                hold_m |= cap_m | bail_m;
+            } while ((uint32_t)__popcll(live_m) > limit);
         }
     }
     tally.flush(q.stats);

@@ -255,17 +255,12 @@ __global__ __launch_bounds__(256) void k_trace(
         if (ray_m == 0) break;
         uint64_t done_m = 0;
         if (live_m != 0) {
-            const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
             const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;  // the max_iters-th body
-            ev.body(r, u, live);
+            const float rn = tick_full(ev, r, u, live_m, cap_m);
             ++tick;
             tally.body(live_m);
-            const float rn = ev.mag();
             const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
             tally.bail(bail_m);
-            // at the cap r stays the magnitude before the last body
-            // (src/shape/mandelbulb.rs:65-78)
-            if (__builtin_amdgcn_inverse_ballot_w64(live_m & ~cap_m)) r = rn;
             done_m = cap_m | bail_m;
             live_m &= ~done_m;
         }

@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "internal.h"
+#include "point_sources.h"
 #include "work_loop.h"
 
 namespace cth {
@@ -96,6 +97,14 @@ inline int run_refill(Ctx& c, int family, const MandelUniform& u, const Src& src
         hipLaunchKernelGGL((k_refill<TrigExact, Src, Sink>), grid, block, 0, st, src, u, sink, q);
     }
     return check_hip(hipGetLastError(), "refill kernel launch");
+}
+
+// Distances, with the loop-body counts where they are asked for.
+template <class Src>
+inline int run_dist(Ctx& c, int family, const MandelUniform& u, const Src& src, float* out, uint32_t* iters,
+                    uint32_t total, hipStream_t st, const LaunchShape& ls) {
+    return iters ? run_refill(c, family, u, src, SinkDistIters{out, iters}, total, st, ls)
+                 : run_refill(c, family, u, src, SinkDist{out}, total, st, ls);
 }
 
 }  // namespace cth

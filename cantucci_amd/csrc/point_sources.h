@@ -118,12 +118,21 @@ struct SrcSpans {
 // ---------------------------------------------------------------------------
 struct SinkDist {
     float* out;
+    __device__ __forceinline__ static constexpr bool wants_k() { return false; }
+    template <class E>
+    __device__ __forceinline__ void put(uint32_t i, float d, uint32_t, float, float, const E&) const {
+        out[i] = d;
+    }
+};
+
+struct SinkDistIters {
+    float* out;
     uint32_t* iters;
-    __device__ __forceinline__ bool wants_k() const { return iters != nullptr; }
+    __device__ __forceinline__ static constexpr bool wants_k() { return true; }
     template <class E>
     __device__ __forceinline__ void put(uint32_t i, float d, uint32_t k, float, float, const E&) const {
         out[i] = d;
-        if (iters) iters[i] = k;
+        iters[i] = k;
     }
 };
 
@@ -131,7 +140,7 @@ struct SinkState {
     float* r;
     float* dr;
     uint32_t* iters;
-    __device__ __forceinline__ bool wants_k() const { return true; }
+    __device__ __forceinline__ static constexpr bool wants_k() { return true; }
     template <class E>
     __device__ __forceinline__ void put(uint32_t i, float, uint32_t k, float rr, float drr, const E&) const {
         r[i] = rr;
@@ -149,7 +158,7 @@ struct SinkGrad {
     float* grad_power;
     const float* grad_d;
     uint32_t max_iters;
-    __device__ __forceinline__ bool wants_k() const { return true; }
+    __device__ __forceinline__ static constexpr bool wants_k() { return true; }
     template <class E>
     __device__ __forceinline__ void put(uint32_t i, float dv, uint32_t k, float r, float, const E& ev) const {
         float g[4];

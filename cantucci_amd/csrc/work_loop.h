@@ -97,9 +97,9 @@ struct Window {
     // Idle lanes that trigger the wave's next refill: refill_min, or as few as
     // take the whole rest of the wave's last chunk, or, with no index left, the
     // whole wave (a batch that could not take new points is only written).
-    __device__ __forceinline__ uint32_t refill_at(const WorkQueue& q, bool exhausted) const {
-        if (exhausted || (last && next >= end)) return 64u;
-        return last && end - next < q.refill_min ? end - next : q.refill_min;
+    __device__ __forceinline__ uint32_t refill_at(const WorkQueue& q) const {
+        if (!last) return q.refill_min;
+        return next >= end ? 64u : (end - next < q.refill_min ? end - next : q.refill_min);
     }
 };
 
@@ -159,15 +159,6 @@ __device__ __forceinline__ void wave_retire(const WorkQueue& q) {
     }
 }
 
-// Whether a refill goes on after offering `avail` indices to `need` idle lanes:
-// lanes that were offered none take from the next chunk; lanes that are idle
-// again (their point needed no loop body) only in batches of refill_min, or
-// when no lane is live.
-__device__ __forceinline__ bool refill_again(uint32_t need, uint32_t avail, uint64_t live, uint64_t wave,
-                                             const WorkQueue& q) {
-    return need > avail || live == 0 || (uint32_t)__popcll(wave & ~live) >= q.refill_min;
-}
-
 // Drive evaluator `Ev` over the indices of `q`, reading points from `src`
 // and writing results through `sink`.
 //   src.get(i, x, y, z, power)
@@ -205,12 +196,11 @@ __device__ __forceinline__ void refill_loop(const Src& src, const MandelUniform&
     uint32_t kh = 0;      // body count of a held point (kept if the sink reads it)
     float r = idle_start(ev, u);
     Window win;
-    bool exhausted = false;
-    uint32_t refill_at = q.refill_min;  // idle lanes that trigger the next refill
     WorkTally<kCount> tally;
 
     for (;;) {
-        if ((uint32_t)__popcll(wave & ~live_m) >= refill_at) {
+        // Refill; again at once if every point taken bailed before its first body.
+        do {
             if (__builtin_amdgcn_inverse_ballot_w64(hold_m)) {
                 if constexpr (Ev::kLastDr) {
                     if (__builtin_amdgcn_inverse_ballot_w64(last_m)) ev.last_dr(r);
@@ -220,17 +210,13 @@ __device__ __forceinline__ void refill_loop(const Src& src, const MandelUniform&
             hold_m = 0;
             last_m = 0;
             // Hand new points to idle lanes.  A point that bails before its
-            // first body (|p| > bailout) is written on the spot.  Its lane is
-            // refilled again only in a batch (refill_again): a few idle lanes
-            // that took a run of such points in turn would hold up the wave
-            // (one lane, 64 points: 50 us of a 96^3 grid's 66).
-            while (!exhausted) {
-                const uint64_t need = wave & ~live_m;
-                if (need == 0) break;
-                if (win.next >= win.end && !next_chunk(q, win)) {
-                    exhausted = true;
-                    break;
-                }
+            // first body (|p| > bailout) is held like any finished one, until
+            // the next refill; a few idle lanes that took a run of such points
+            // in turn would hold up the wave (one lane, 64 points: 50 us of a
+            // 96^3 grid's 66).
+            uint64_t need = wave & ~live_m;
+            while (need != 0) {
+                if (win.next >= win.end && !next_chunk(q, win)) break;
                 const uint32_t avail = win.end - win.next;
                 const uint32_t nneed = (uint32_t)__popcll(need);
                 const uint32_t rank = lane_rank(need);
@@ -251,64 +237,58 @@ __device__ __forceinline__ void refill_loop(const Src& src, const MandelUniform&
                 // at once is at its cap before any full body.
                 const uint64_t capped = (Ev::kLastDr && u.max_iters == 1u) ? took & ~bailed : 0;
                 tally.body(capped);
-                if (__builtin_amdgcn_inverse_ballot_w64(bailed | capped)) {
-                    const bool c = __builtin_amdgcn_inverse_ballot_w64(capped);
-                    if constexpr (Ev::kLastDr) {
-                        if (c) ev.last_dr(r);
-                    }
-                    sink.put(idx, ev.finish(r), c ? 1u : 0u, r, ev.dr, ev);
+                last_m |= capped;
+                hold_m |= bailed | capped;
+                if (sink.wants_k() && (bailed | capped) != 0) {
+                    if (__builtin_amdgcn_inverse_ballot_w64(bailed | capped))
+                        kh = __builtin_amdgcn_inverse_ballot_w64(capped) ? 1u : 0u;
                 }
                 live_m |= took & ~(bailed | capped);
+                need &= ~took;
                 win.next += (nneed < avail) ? nneed : avail;
-                if (!refill_again(nneed, avail, live_m, wave, q)) break;
             }
-            if (live_m == 0) break;
-            refill_at = win.refill_at(q, exhausted);
-            tick_guard(ev, u);  // the started points' squares
-        }
-        const bool live = __builtin_amdgcn_inverse_ballot_w64(live_m);
-        uint64_t done_m;
+        } while (live_m == 0 && hold_m != 0);
+        if (live_m == 0) break;
+        tick_guard(ev, u);  // the started points' squares
+        // Idle lanes, win.refill_at() of them, trigger the next refill.
+        const uint32_t limit = 64u - win.refill_at(q);
         if constexpr (Ev::kLastDr) {
-            tick_body(ev, r, u, live);
-            ++tick;
-            tally.body(live_m);
-            const float rn = tick_mag(ev, u);
-            const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m;
-            tally.bail(bail_m);
-            // Every lane takes rn: a lane without a live point ran the body
-            // without committing it, so rn is its last magnitude again, bit
-            // for bit (a held point's r, the one its finish needs).
-            r = rn;
-            // Lanes that have now run max_iters - 1 bodies without bailing:
-            // their max_iters-th body is the dr update alone (max_iters >= 2
-            // here; max_iters == 1 ends at the start).
-            const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m & ~bail_m;
-            tally.body(cap_m);
-            done_m = cap_m | bail_m;
-            last_m |= cap_m;
-            if (done_m != 0 && sink.wants_k()) {
-                if (__builtin_amdgcn_inverse_ballot_w64(done_m))
-                    kh = tick - t0 + (__builtin_amdgcn_inverse_ballot_w64(cap_m) ? 1u : 0u);
-            }
+            run_ticks(ev, r, u, live_m, limit, [&]() {
+                ++tick;
+                tally.body(live_m);
+                const uint64_t bail_m = wave_mask(r > u.bailout) & live_m;
+                tally.bail(bail_m);
+                // Lanes that have now run max_iters - 1 bodies without bailing:
+                // their max_iters-th body is the dr update alone (max_iters >= 2
+                // here; max_iters == 1 ends at the start).
+                const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m & ~bail_m;
+                tally.body(cap_m);
+                const uint64_t done_m = cap_m | bail_m;
+                last_m |= cap_m;
+                if (sink.wants_k() && done_m != 0) {
+                    if (__builtin_amdgcn_inverse_ballot_w64(done_m))
+                        kh = tick - t0 + (__builtin_amdgcn_inverse_ballot_w64(cap_m) ? 1u : 0u);
+                }
+                live_m &= ~done_m;
+                hold_m |= done_m;
+            });
         } else {
-            // Lanes making their max_iters-th body in this tick (max_iters >= 1).
-            const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;
-            tick_body(ev, r, u, live);
-            ++tick;
-            tally.body(live_m);
-            const float rn = tick_mag(ev, u);
-            const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
-            tally.bail(bail_m);
-            // At the iteration cap, r stays the magnitude computed before the
-            // last body (the reference's off-by-one, src/shape/mandelbulb.rs:65-78).
-            if (__builtin_amdgcn_inverse_ballot_w64(live_m & ~cap_m)) r = rn;
-            done_m = cap_m | bail_m;
-            if (done_m != 0 && sink.wants_k()) {
-                if (__builtin_amdgcn_inverse_ballot_w64(done_m)) kh = tick - t0;
-            }
+            do {
+                // Lanes making their max_iters-th body in this tick (max_iters >= 1).
+                const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;
+                const float rn = tick_full(ev, r, u, live_m, cap_m);
+                ++tick;
+                tally.body(live_m);
+                const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
+                tally.bail(bail_m);
+                const uint64_t done_m = cap_m | bail_m;
+                if (sink.wants_k() && done_m != 0) {
+                    if (__builtin_amdgcn_inverse_ballot_w64(done_m)) kh = tick - t0;
+                }
+                live_m &= ~done_m;
+                hold_m |= done_m;
+            } while ((uint32_t)__popcll(live_m) > limit);
         }
-        live_m &= ~done_m;
-        hold_m |= done_m;
     }
     tally.flush(q.stats);
     if (q.dynamic) wave_retire(q);
