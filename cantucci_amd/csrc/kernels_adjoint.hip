@@ -7,6 +7,9 @@
 //   z_{k+1} = F(z_k; P) + c,      z_0 = c = p
 // with respect to p (and the power P) comes from one reverse sweep:
 //
+// in one kernel with the orbit in LDS (k_adjoint), or, for large iteration
+// caps, in two:
+//
 //   kernel 1 (k_adj_forward): the forward iteration, recomputed per lane in
 //     parity arithmetic, records each point's orbit (z_k, dr_k) in a
 //     workspace (point-major, so a lane's own records are contiguous) plus the
@@ -15,7 +18,7 @@
 //     reverse sweep k = K-1 .. 0 through the spherical power map (trig family)
 //     or the closed-form P8 polynomial, accumulating c_bar and P_bar.
 //
-// Both kernels use the lane-refill schedule of work_loop.h: one forward body
+// They use the lane-refill schedule of work_loop.h: one forward body
 // or one reverse step per lane per tick, finished lanes take new points, so
 // neither phase pays for the spread of iteration counts.
 #include <hip/hip_runtime.h>
@@ -353,6 +356,134 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
 }
 
 // ---------------------------------------------------------------------------
+// Both sweeps in one kernel, the orbit in LDS: no workspace, one launch, and no
+// orbit traffic (300,000 points at 15 iterations wrote and read 77 MB).
+//
+// A lane's point goes through the forward bodies, waits (hold_m) for the seeds
+// of its reverse sweep, goes back through the reverse steps and waits (out_m)
+// to be written.  Bodies and reverse steps are different instruction streams,
+// so each tick runs the one that more lanes are due; writing, seeding and
+// taking new points wait for refill_min lanes.
+//
+// Workgroups are single waves: a wave needs (max_iters - 1) KiB of LDS, which
+// bounds the waves per CU (10 at 15 iterations, 5 at 30), and a SIMD needs
+// about three waves to issue at full rate.  So large caps stay with the two
+// kernels above: us for power 8 and for per-point powers, two kernels -> one,
+//   15 iterations: 300,000 points 62 -> 38, 94 -> 65; 1 M 135 -> 96, 158 -> 167;
+//                  4 M 545 -> 272, 615 -> 469;
+//   30 iterations: 300,000 points 107 -> 73, 162 -> 137; 1 M 196 -> 170,
+//                  232 -> 314; 4 M 674 -> 500, 883 -> 962.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kFusedIters = 32;            // any point count at power 8
+constexpr uint32_t kFusedTrigIters = 20;        // trig map, any point count
+constexpr uint32_t kFusedTrigPoints = 1u << 18;  // trig map, up to kFusedIters
+
+template <class Ev, bool TRIG>
+__global__ __launch_bounds__(64) void k_adjoint(SrcPoints src, MandelUniform u, float* __restrict__ dout, AdjOut out,
+                                                WorkQueue q) {
+    extern __shared__ float4 orbit_lds[];
+    float4* const orbit = orbit_lds + threadIdx.x;  // (z_k, dr_k), k >= 1, at orbit[64 (k - 1)]
+    Ev ev;
+    uint64_t fwd_m = 0, hold_m = 0, rev_m = 0, out_m = 0;
+    uint32_t idx = 0, k = 0;  // k: bodies run; in the reverse sweep, steps left
+    float P = 0.0f;
+    float zbx = 0.0f, zby = 0.0f, zbz = 0.0f, drb = 0.0f, cbx = 0.0f, cby = 0.0f, cbz = 0.0f, Pb = 0.0f;
+    float rb_extra = 0.0f;
+    float r = idle_start(ev, u);
+    Window win;
+    for (;;) {
+        do {
+            if (__builtin_amdgcn_inverse_ballot_w64(out_m))
+                adj_write(out, idx, cbx + zbx, cby + zby, cbz + zbz, zbx, zby, zbz, cbx, cby, cbz, Pb);
+            out_m = 0;
+            bool zero = false;  // no loop body: nothing to sweep back through
+            if (__builtin_amdgcn_inverse_ballot_w64(hold_m)) {
+                const float d = ev.finish(r);
+                if (dout) dout[idx] = d;
+                const float g = out.grad_d ? out.grad_d[idx] : 1.0f;
+                // seeds of d = 0.5 ln(r_f) r_f / dr_f
+                const float rf = r, drf = ev.dr;
+                const float lnr = __logf(rf);
+                const float rbar = g * 0.5f * (lnr + 1.0f) / drf;
+                drb = -g * (0.5f * lnr * rf / drf) / drf;
+                cbx = cby = cbz = Pb = 0.0f;
+                rb_extra = 0.0f;
+                const float ir = 1.0f / rf;
+                if (k == 0) {
+                    // r_f = |z_0|: no loop body, so c does not reach d
+                    const float gx = rbar * ev.px * ir, gy = rbar * ev.py * ir, gz = rbar * ev.pz * ir;
+                    adj_write(out, idx, gx, gy, gz, gx, gy, gz, 0.0f, 0.0f, 0.0f, 0.0f);
+                    zero = true;
+                } else if (k == u.max_iters) {
+                    // iteration cap: r_f = |z_{K-1}|, z_K unused
+                    zbx = zby = zbz = 0.0f;
+                    rb_extra = rbar;
+                } else {
+                    // bailout: r_f = |z_K|
+                    zbx = rbar * ev.x * ir;
+                    zby = rbar * ev.y * ir;
+                    zbz = rbar * ev.z * ir;
+                }
+            }
+            rev_m |= hold_m & ~wave_mask(zero);
+            hold_m = 0;
+            uint64_t need = ~(fwd_m | rev_m);
+            while (need != 0) {
+                if (win.next >= win.end && !next_chunk(q, win)) break;
+                const uint32_t avail = win.end - win.next;
+                const uint32_t nneed = (uint32_t)__popcll(need);
+                const uint32_t rank = lane_rank(need);
+                const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
+                if (take) {
+                    idx = win.next + rank;
+                    float px, py, pz;
+                    src.get(idx, px, py, pz, P);
+                    ev.start(px, py, pz, P, u);
+                    k = 0;
+                    r = ev.mag();
+                }
+                const uint64_t took = wave_mask(take);
+                const uint64_t bailed = wave_mask(r > u.bailout) & took;
+                hold_m |= bailed;
+                fwd_m |= took & ~bailed;
+                need &= ~took;
+                win.next += (nneed < avail) ? nneed : avail;
+            }
+        } while ((fwd_m | rev_m) == 0 && hold_m != 0);
+        if ((fwd_m | rev_m) == 0) break;
+        const uint32_t limit = 64u - win.refill_at(q);
+        do {
+            if (__popcll(fwd_m) >= __popcll(rev_m)) {
+                if (__builtin_amdgcn_inverse_ballot_w64(fwd_m)) {
+                    if (k != 0) orbit[64 * (k - 1)] = make_float4(ev.x, ev.y, ev.z, ev.dr);
+                    ++k;
+                }
+                const uint64_t cap_m = wave_mask(k == u.max_iters) & fwd_m;
+                const float rn = tick_full(ev, r, u, fwd_m, cap_m);
+                const uint64_t done_m = cap_m | (wave_mask(rn > u.bailout) & fwd_m);
+                fwd_m &= ~done_m;
+                hold_m |= done_m;
+            } else {
+                if (__builtin_amdgcn_inverse_ballot_w64(rev_m)) {
+                    --k;
+                    // z_0 = p, dr_0 = 1
+                    const float4 s = k != 0 ? orbit[64 * (k - 1)] : make_float4(ev.px, ev.py, ev.pz, 1.0f);
+                    if (TRIG)
+                        rev_step_trig(s.x, s.y, s.z, s.w, P, rb_extra, zbx, zby, zbz, drb, cbx, cby, cbz, Pb);
+                    else
+                        rev_step_p8(s.x, s.y, s.z, s.w, rb_extra, zbx, zby, zbz, drb, cbx, cby, cbz);
+                    rb_extra = 0.0f;
+                }
+                const uint64_t done_m = wave_mask(k == 0) & rev_m;
+                rev_m &= ~done_m;
+                out_m |= done_m;
+            }
+        } while ((uint32_t)__popcll(fwd_m | rev_m) > limit);
+    }
+    if (q.dynamic) wave_retire(q);
+}
+
+// ---------------------------------------------------------------------------
 // 6-tap central differences (the reference's normal stencil): virtual point
 // 7 i + t is p_i (t = 0) or p_i +- h e_a (t = 1 + 2a, 2 + 2a), written as
 // (p_b + u_b * h, ...) with u = e_a exactly like `p + Vector3::unit_x() * delta.x`
@@ -447,6 +578,35 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
     if (rc) return rc;
     const size_t stride = (size_t)u.max_iters + 1;
     if (stride > 4096) return fail(CTH_E_INVALID, "max_iters above 4095 for the adjoint");
+    if (workspace && vjp_workspace_bytes(u.max_iters, n) > ws_bytes) return fail(CTH_E_INVALID, "workspace too small");
+    if (u.max_iters <= kFusedIters &&
+        (family == FAM_P8 || u.max_iters <= kFusedTrigIters || n <= kFusedTrigPoints)) {
+        const uint32_t lds = (u.max_iters - 1) * 64u * (uint32_t)sizeof(float4);
+        const uint32_t granules = std::max(1u, (lds + 1279u) / 1280u);  // as LDS is allocated
+        const uint32_t resident = std::min(16u, 160u * 1024u / (granules * 1280u));
+        const WaveSpread spread{std::min(8u, resident), resident};
+        LaunchShape ls = c.shape_adj;
+        ls.blocks_per_cu *= ls.block / 64;
+        ls.block = 64;
+        // `resident` need not spread evenly over a CU's four SIMDs: waves claim
+        // their chunks where there are enough to even that out (4 M points at 15
+        // iterations 558 -> 469 us, 300,000 points 65 -> 73).
+        // Not in a capture that owns no counters (replays would share the ring's).
+        ls.dynamic = n / 256u >= (uint32_t)c.num_cus * spread.fill;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (ls.dynamic && capture_pool().stream != st && hipStreamIsCapturing(st, &cs) == hipSuccess &&
+            cs != hipStreamCaptureStatusNone)
+            ls.dynamic = 0;
+        SrcPoints src{pts, powers, s.power};
+        AdjOut out{grad_d, grad_p, grad_power, normals, grad_z0, grad_c};
+        uint32_t blocks = 0;
+        WorkQueue q = make_queue(c, n, ls, spread, blocks, st);
+        if (family == FAM_P8)
+            hipLaunchKernelGGL((k_adjoint<P8Exact, false>), dim3(blocks), dim3(64), lds, st, src, u, d, out, q);
+        else
+            hipLaunchKernelGGL((k_adjoint<TrigExact, true>), dim3(blocks), dim3(64), lds, st, src, u, d, out, q);
+        return check_hip(hipGetLastError(), "adjoint launch");
+    }
     size_t per_point = stride * sizeof(float4) + sizeof(AdjRecord);
     float4* orbit = nullptr;
     AdjRecord* rec = nullptr;
@@ -461,7 +621,6 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
         // The caller's workspace holds the whole call: orbit records, then
         // (256-byte aligned) the end states.  The forward kernel writes every
         // record the reverse kernel reads, so nothing needs clearing.
-        if (vjp_workspace_bytes(u.max_iters, n) > ws_bytes) return fail(CTH_E_INVALID, "workspace too small");
         batch = n;
         orbit = static_cast<float4*>(workspace);
         rec = reinterpret_cast<AdjRecord*>(static_cast<char*>(workspace) +

@@ -349,8 +349,9 @@ int cth_render_depth_dev(cth_ctx* ctx, const cth_shape* shape, const cth_camera*
  *   grad_power[i] = grad_d[i] * dd/dpower  (nullable; CTH_SHAPE_MANDELBULB_TRIG
  *                                           only, 0 for the other kinds)
  * grad_d NULL means all ones.  The derivative ignores the measure-zero
- * switches of the loop (bailout, iteration cap).  Uses a device workspace of
- * at most ~1 GiB (stream-ordered allocation). */
+ * switches of the loop (bailout, iteration cap).  Large iteration caps (above
+ * 32, or above 20 off power 8 with many points) use a device workspace of at
+ * most ~1 GiB (stream-ordered allocation). */
 int cth_de_vjp_dev(cth_ctx* ctx, const cth_shape* shape, const float* pts, const float* powers, size_t n,
                    const float* grad_d, float* d, float* grad_p, float* grad_power, void* stream);
 

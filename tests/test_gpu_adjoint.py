@@ -88,6 +88,53 @@ def test_integer_power_normals_match_dual_oracle(ctx, torch_cuda, P):
     assert np.median(ang) < np.median(angf)
 
 
+@pytest.mark.parametrize("iters", [21, 32])
+def test_one_and_two_kernel_sweeps_agree(ctx, torch_cuda, iters):
+    """The trig map at caps of 21 to 32 runs in one kernel up to 2^18 points and
+    in two beyond: the same operations per point, so the same bits, for batch
+    sizes around a wave and around that line."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    from cantucci_amd.workloads import shell_points
+    torch = torch_cuda
+    edge = 1 << 18
+    pts, powers = shell_points(edge + 1, seed=5)
+    P, W = gpu(torch, pts), gpu(torch, powers)
+    G = torch.linspace(-1, 1, edge + 1, device="cuda")
+    shape = ca.MandelbulbTrig(iters, 2.0, 8.0, ctx=ctx)
+    whole = dev.de_vjp_split(shape, P, W, G, with_power=True)
+    for lo, n in ((0, 1), (1, 63), (64, 64), (128, 65), (193, 1000), (1, edge)):
+        s = slice(lo, lo + n)
+        for a, b in zip(whole, dev.de_vjp_split(shape, P[s], W[s], G[s], with_power=True)):
+            assert torch.equal(a[s].view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("P", [8, 5])
+@pytest.mark.parametrize("iters", [1, 2, 3, 20, 21, 32, 33])
+def test_vjp_iteration_caps(ctx, torch_cuda, P, iters):
+    """The reverse sweep at the smallest caps and on both sides of the caps where
+    the kernel changes, with points that bail at once among them: distances are
+    the forward kernel's, and gradients the FP64 dual oracle's where f32 and f64
+    iterate alike (the bars of the fixed-cap test above)."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    pts = np.random.default_rng(6).uniform(-1.6, 1.6, (20000, 3)).astype(F32)
+    shape = ca.Mandelbulb(iters, 2.0, P, ctx=ctx)
+    d, gp = dev.de_vjp(shape, gpu(torch, pts))
+    d_fwd = dev.de_points(shape, gpu(torch, pts))
+    torch.cuda.synchronize()
+    assert torch.equal(d.view(torch.int32), d_fwd.view(torch.int32))
+    _, g64, it64 = O.de_grad_f64(O.mandelbulb(iters, 2.0, P), pts)
+    _, it_o, _, _ = O.de_points(O.mandelbulb(iters, 2.0, P), pts)
+    same = it_o == it64
+    a = angle(gp.cpu().numpy()[same], g64[same, :3])
+    a = a[np.isfinite(a)]
+    assert len(a) > 0.9 * len(pts)
+    assert np.median(a) < 1e-5
+    assert np.mean(a <= 1e-3) > 0.9
+
+
 def test_vjp_is_linear_in_grad_d(ctx, torch_cuda):
     import cantucci_amd as ca
     from cantucci_amd import device as dev
