@@ -103,13 +103,6 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wsum, 
     return off + inc - v;
 }
 
-// The wave's LDS writes become visible to its other lanes.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t& total) {
     const uint32_t inc = wave_incl_scan(v);
     total = (uint32_t)__shfl((int)inc, 63, 64);

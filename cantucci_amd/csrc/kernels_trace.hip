@@ -5,9 +5,9 @@
 // stop when d < EPSILON, at most 100 steps, no escape test.  Here every lane
 // owns one ray; each ray step is one distance evaluation whose loop bodies run
 // in the same branch-free ticks as the plain distance kernel.  When a lane's
-// evaluation finishes, the lane applies the step (pos += dir * d, t += d) in
-// the same iteration and either starts the ray's next evaluation or writes
-// the ray, so lanes stay busy although both the evaluation lengths and the
+// evaluation finishes, the lane takes its step (pos += dir * d, t += d) with
+// the next batch of such lanes and either starts the ray's next evaluation or
+// writes the ray and takes another, so lanes stay busy although both the evaluation lengths and the
 // ray step counts differ wildly.  (On the camera workload an evaluation runs
 // 1.6 loop bodies on average and a third run none, so the steps are as much
 // of the work as the bodies.)  The hit test is d < eps_abs + eps_rel * t
@@ -158,27 +158,39 @@ struct TraceOut {
 };
 
 // Lanes whose evaluation has finished take their step together once this
-// many are due (or no lane is running a loop body).  On the 32 x 1080p
-// render, thresholds of 8, 16, 32, 40, 48, 56 and 64 gave 8.7, 8.2, 7.8-8.0,
-// 7.7-8.0, 7.9-8.2, 8.3-8.6 and 9.8 ms, against 9.0 ms stepping at once.
-constexpr uint32_t kStepMin = 32;
+// many are due (or no lane is running a loop body).  The 32 x 1080p render
+// takes 8.1, 7.8, 7.7, 7.65, 7.65, 8.0 ms at 16, 24, 32, 40, 48, 56 (two
+// cards 4 % apart, averaged).
+constexpr uint32_t kStepMin = 40;
+
+// Idle lanes take new rays along with a step, from this many on: the rays
+// wait in LDS (below), so taking one costs seven instructions.  2, 4 and 8 are
+// within 1 % of each other.
+constexpr uint32_t kFetchMin = 4;
 
 template <class Ev, class Rays, bool kCount = false>
 __global__ __launch_bounds__(256) void k_trace(
     Rays rays, MandelUniform u, TraceParams tp, TraceOut out, WorkQueue q) {
+    // The wave's next rays (origin, direction), built 64 at a time: building
+    // one takes some 100 instructions, and idle lanes that built their own, 8
+    // at a time, took a fifth of the render's issue time.  With the step, the
+    // new rays and the starts in one pass, 32 x 1080p takes 7.5 ms (before:
+    // 8.9), 8 x 1080p 2.97 (3.4), 1080p 1.08 (1.28), 161 x 120 0.69 (0.75).
+    // 6 KiB a block does not limit the occupancy.
+    __shared__ float ray_buf[4][6][64];
+    float(*const buf)[64] = ray_buf[threadIdx.x >> 6];
+    uint32_t b_base = 0, b_next = 0, b_end = 0;  // index of slot 0; slots not handed out
     Ev ev;
-    // Every lane that holds a ray is in one of two states, kept as
+    // Every lane that holds a ray (ray_m) is in one of two states, kept as
     // wave-uniform lane masks: running loop bodies of a distance evaluation
     // (live_m), or holding a finished evaluation whose step is due (step_m:
     // an evaluation from beyond the bailout radius runs no body, so it is
     // finished as soon as it starts).  One iteration of the loop runs one
-    // loop body on the live lanes and then, once kStepMin lanes are due or
-    // none is live, the step of every due lane: pos += dir d, t += d, the end
-    // tests, and the next evaluation's start.  An evaluation's step waits at
-    // most until half the wave's lanes are due; it never waits for the rest
-    // of the wave.  Lanes whose ray ended take new rays in batches of at
-    // least refill_min (ray generation is the costly part of a start).
-    const uint64_t wave = wave_mask(true);
+    // loop body; once kStepMin lanes are due or none is live, every due lane
+    // takes its step (pos += dir d, t += d, the end tests), lanes without a ray
+    // take one, and all of these start their next evaluation together.  An
+    // evaluation's step waits at most until half the wave's lanes are due; it
+    // never waits for the rest of the wave.
     uint64_t live_m = 0, step_m = 0, ray_m = 0;
     bool has_ray = false;
     uint32_t idx = 0, nsteps = 0;
@@ -186,16 +198,9 @@ __global__ __launch_bounds__(256) void k_trace(
     float r = idle_start(ev, u), t = 0.0f;
     float pos[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f};
     Window win;
-    bool exhausted = false;
+    const uint32_t fetch_min = q.refill_min < kFetchMin ? q.refill_min : kFetchMin;
     WorkTally<kCount> tally;
 
-    // Start the lane's next evaluation at pos; zero loop bodies when |pos|
-    // is beyond the bailout radius (its step is then due at once).
-    auto start = [&]() {
-        ev.start(pos[0], pos[1], pos[2], u.power, u);
-        t0 = tick;
-        r = ev.mag();
-    };
     // One sphere-tracing step of the lane's ray by distance d.  When the ray
     // ends (hit, escape or the step limit) its outputs are written and the
     // lane has no ray.
@@ -219,71 +224,81 @@ __global__ __launch_bounds__(256) void k_trace(
     };
 
     for (;;) {
-        // New rays for the lanes without one.
-        uint64_t need = wave & ~ray_m;
-        if (!exhausted && (uint32_t)__popcll(need) >= q.refill_min) {
-            while (need != 0) {
-                if (win.next >= win.end && !next_chunk(q, win)) {
-                    exhausted = true;
-                    break;
-                }
-                const uint32_t avail = win.end - win.next;
-                const uint32_t nneed = (uint32_t)__popcll(need);
-                const uint32_t rank = lane_rank(need);
-                const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
-                if (take) {
-                    idx = win.next + rank;
-                    rays.get(idx, pos, dir);
-                    t = 0.0f;
-                    nsteps = 0;
-                    has_ray = true;
-                    start();
-                }
-                const uint64_t took = wave_mask(take);
-                const uint64_t zero = wave_mask(r > u.bailout) & took;
-                tally.eval(took);
-                tally.bail(zero);
-                live_m |= took & ~zero;
-                step_m |= zero;
-                ray_m |= took;
-                need &= ~took;
-                win.next += (nneed < avail) ? nneed : avail;
-            }
-        }
-        // Every lane with a ray is live or has a step due; none left means
-        // the index space is exhausted (a wave without rays always fetches).
-        if (ray_m == 0) break;
-        uint64_t done_m = 0;
-        if (live_m != 0) {
-            const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;  // the max_iters-th body
-            const float rn = tick_full(ev, r, u, live_m, cap_m);
-            ++tick;
-            tally.body(live_m);
-            const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
-            tally.bail(bail_m);
-            done_m = cap_m | bail_m;
-            live_m &= ~done_m;
-        }
         // The step runs for at least kStepMin lanes at a time: due lanes wait
-        // (as step_m) while other lanes are live.  An evaluation averages
-        // under two loop bodies, so stepping every iteration would run the
-        // step's ~80 instructions for a third of the wave almost every time.
-        const uint64_t go_m = done_m | step_m;
-        if (go_m != 0 && live_m != 0 && (uint32_t)__popcll(go_m) < kStepMin) {
-            step_m = go_m;
-        } else if (go_m != 0) {
-            if (__builtin_amdgcn_inverse_ballot_w64(go_m)) {
-                step(ev.finish(r));
-                if (has_ray) start();
-            }
-            const uint64_t cont = go_m & wave_mask(has_ray);
-            const uint64_t zero = wave_mask(r > u.bailout) & cont;
-            tally.eval(cont);
-            tally.bail(zero);
-            ray_m &= ~(go_m & ~cont);
-            live_m |= cont & ~zero;
-            step_m = zero;
+        // while other lanes are live.  An evaluation averages under two loop
+        // bodies, so stepping every iteration would run the step's
+        // instructions for a third of the wave almost every time.
+        if (live_m == 0 || (uint32_t)__popcll(step_m) >= kStepMin) {
+            do {
+                if (__builtin_amdgcn_inverse_ballot_w64(step_m)) step(ev.finish(r));
+                const uint64_t cont = step_m & wave_mask(has_ray);
+                ray_m &= ~(step_m & ~cont);
+                uint64_t need = ~ray_m, took = 0;
+                if ((uint32_t)__popcll(need) < fetch_min) need = 0;
+                while (need != 0) {
+                    if (b_next >= b_end) {
+                        if (win.next >= win.end && !next_chunk(q, win)) break;
+                        const uint32_t n = win.end - win.next < 64u ? win.end - win.next : 64u;
+                        const uint32_t lane = __lane_id();
+                        wave_sync();  // the old rays have been read
+                        if (lane < n) {
+                            float o[3], d[3];
+                            rays.get(win.next + lane, o, d);
+#pragma unroll
+                            for (int a = 0; a < 3; ++a) {
+                                buf[a][lane] = o[a];
+                                buf[3 + a][lane] = d[a];
+                            }
+                        }
+                        wave_sync();
+                        b_base = win.next;
+                        b_next = 0;
+                        b_end = n;
+                        win.next += n;
+                    }
+                    const uint32_t avail = b_end - b_next;
+                    const uint32_t nneed = (uint32_t)__popcll(need);
+                    const uint32_t slot = b_next + lane_rank(need);
+                    const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && slot < b_end;
+                    if (take) {
+                        idx = b_base + slot;
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) {
+                            pos[a] = buf[a][slot];
+                            dir[a] = buf[3 + a][slot];
+                        }
+                        t = 0.0f;
+                        nsteps = 0;
+                        has_ray = true;
+                    }
+                    took |= wave_mask(take);
+                    need &= ~took;
+                    b_next += nneed < avail ? nneed : avail;
+                }
+                ray_m |= took;
+                // Start the next evaluations; zero loop bodies when |pos| is
+                // beyond the bailout radius (the step is then due at once).
+                const uint64_t start_m = cont | took;
+                if (__builtin_amdgcn_inverse_ballot_w64(start_m)) {
+                    ev.start(pos[0], pos[1], pos[2], u.power, u);
+                    t0 = tick;
+                    r = ev.mag();
+                }
+                step_m = wave_mask(r > u.bailout) & start_m;
+                live_m |= start_m & ~step_m;
+                tally.eval(start_m);
+                tally.bail(step_m);
+            } while (live_m == 0 && ray_m != 0);
+            if (ray_m == 0) break;
         }
+        const uint64_t cap_m = wave_mask(t0 == tick + 1u - u.max_iters) & live_m;  // the max_iters-th body
+        const float rn = tick_full(ev, r, u, live_m, cap_m);
+        ++tick;
+        tally.body(live_m);
+        const uint64_t bail_m = wave_mask(rn > u.bailout) & live_m & ~cap_m;
+        tally.bail(bail_m);
+        live_m &= ~(cap_m | bail_m);
+        step_m |= cap_m | bail_m;
     }
     tally.flush(q.stats);
     if (q.dynamic) wave_retire(q);

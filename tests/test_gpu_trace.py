@@ -45,6 +45,31 @@ def test_sphere_rays_bitexact(ctx, torch_cuda):
     assert np.isfinite(d_o).any() and np.isinf(d_o).any()
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 8 * 64 * 256 - 1, 8 * 64 * 256 + 1, 300001])
+def test_ray_batches_ragged(ctx, torch_cuda, n):
+    """Rays are built 64 at a time and handed to idle lanes: counts around one
+    batch, around the size up to which a launch deals fewer than 64 to a wave
+    (8 waves on each of 256 CUs), and one that leaves part batches.  Every ray
+    that misses ends in its first steps, so lanes empty whole batches at once.
+    A sphere's trace is exact arithmetic: equal to the oracle bit for bit."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(n)
+    dirs = rng.normal(size=(n, 3))
+    dirs[n // 2:, 1] = -np.abs(dirs[n // 2:, 1])  # the second half looks away
+    dirs[:n // 2, 1] = np.abs(dirs[:n // 2, 1]) * 3
+    dirs = (dirs / np.linalg.norm(dirs, axis=1, keepdims=True)).astype(F32)
+    origin = np.array([[0.1, -3.0, 0.2]], F32)
+    shape = ca.Sphere((0.0, 0.0, 0.0), 0.8, ctx=ctx)
+    d, s, p = dev.sphere_trace(shape, gpu(torch, origin), gpu(torch, dirs), 64, 0.0, 1e-4, 6.0, with_pos=True)
+    torch.cuda.synchronize()
+    d_o, s_o, p_o = O.sphere_trace(O.sphere((0, 0, 0), 0.8), origin, dirs, 64, 1e-4, 6.0, 0.0, with_pos=True)
+    assert (s.cpu().numpy().astype(np.uint32) == s_o).all()
+    assert (d.cpu().numpy().view(np.uint32) == d_o.view(np.uint32)).all()
+    assert (p.cpu().numpy().view(np.uint32) == p_o.view(np.uint32)).all()
+
+
 def test_camera_render_matches_oracle(ctx, torch_cuda):
     """Primary rays of the 32 seeded orbit poses at reduced resolution, P8
     Mandelbulb, 256 steps, hit when d < 1e-4 t, escape at t > 10."""
