@@ -225,6 +225,7 @@ struct P8Exact {
     float px, py, pz, x, y, z, dr;
     float x2, y2, w2, z2;  // squares of the last magnitude, reused by rotate
     bool pos_nan;          // the orbit's NaNs are positive (canon_nan)
+    bool in_range = false; // guard_start(): the bailout and every lane's magnitude allow the unscaled sequences
     bool fast = false;     // guard(): the next body may take the unscaled sequences
 
     __device__ __forceinline__ void start(float ax, float ay, float az, float, const MandelUniform&) {
@@ -245,9 +246,16 @@ struct P8Exact {
         return sqrt_rn_wave(w2 + z2);
     }
     // The wave test of body() (see there) on the current squares, kept for the
-    // next body_guarded().  The work loops call it after starting points.
-    __device__ __forceinline__ void guard(const MandelUniform& u) {
-        fast = u.bailout <= 16.0f && wave_mask(!(w2 >= 0x1p-15f)) == 0;
+    // next body_guarded().
+    __device__ __forceinline__ void guard() { fast = in_range && wave_mask(!(w2 >= 0x1p-15f)) == 0; }
+    // The work loops call this after starting points.  A point whose first
+    // magnitude overflows is finished at once and held, and its magnitude is
+    // recomputed with every tick (run_ticks): no unscaled square root while the
+    // wave holds one (infinite input gives NaN there; the bound is below FLT_MAX
+    // for the contracted sum's sake).
+    __device__ __forceinline__ void guard_start(const MandelUniform& u) {
+        in_range = u.bailout <= 16.0f && wave_mask(!(w2 + z2 <= 0x1p126f)) == 0;
+        guard();
     }
     // mag() after a loop body, with the wave test of the next body made here
     // and also used for this square root: m = w2 + z2 >= w2 >= 2^-15, and a
@@ -256,12 +264,12 @@ struct P8Exact {
     // z whose denominator w8 cancels against the numerator's w^8 factor), so
     // m < 2^94: the range of sqrt_rn_unscaled.  Lanes without a live point
     // may be outside it; their results are dropped.
-    __device__ __forceinline__ float mag_tick(const MandelUniform& u) {
+    __device__ __forceinline__ float mag_tick() {
         x2 = x * x;
         y2 = y * y;
         w2 = x2 + y2;
         z2 = z * z;
-        guard(u);
+        guard();
         const float m = w2 + z2;
         return fast ? sqrt_rn_unscaled(m) : sqrt_rn_wave(m);
     }
@@ -377,13 +385,13 @@ struct P8Contract : P8Exact {
         return sqrt_rn_wave(w2 + z2);
     }
     // P8Exact::mag_tick with contraction (the same ranges hold).
-    __device__ __forceinline__ float mag_tick(const MandelUniform& u) {
+    __device__ __forceinline__ float mag_tick() {
 #pragma clang fp contract(fast)
         x2 = x * x;
         y2 = y * y;
         w2 = x2 + y2;
         z2 = z * z;
-        guard(u);
+        guard();
         const float m = w2 + z2;
         return fast ? sqrt_rn_unscaled(m) : sqrt_rn_wave(m);
     }
@@ -630,7 +638,7 @@ struct SphereEv {
 
 // The tick of a work loop through an evaluator.  Evaluators with
 // kCarriedGuard make the next body's wave test in the magnitude after a body
-// (mag_tick) and in guard(), which the loops call after starting points,
+// (mag_tick) and in guard_start(), which the loops call after starting points,
 // instead of in the body (body_guarded); the others keep mag() and body().
 template <class E, class = void>
 struct CarriesGuard : std::false_type {};
@@ -639,7 +647,7 @@ struct CarriesGuard<E, std::void_t<decltype(E::kCarriedGuard)>> : std::bool_cons
 
 template <class E>
 __device__ __forceinline__ void tick_guard(E& ev, const MandelUniform& u) {
-    if constexpr (CarriesGuard<E>::value) ev.guard(u);
+    if constexpr (CarriesGuard<E>::value) ev.guard_start(u);
 }
 template <class E>
 __device__ __forceinline__ void tick_body(E& ev, float r, const MandelUniform& u, bool live) {
@@ -651,7 +659,7 @@ __device__ __forceinline__ void tick_body(E& ev, float r, const MandelUniform& u
 template <class E>
 __device__ __forceinline__ float tick_mag(E& ev, const MandelUniform& u) {
     if constexpr (CarriesGuard<E>::value)
-        return ev.mag_tick(u);
+        return ev.mag_tick();
     else
         return ev.mag();
 }

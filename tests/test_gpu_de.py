@@ -155,6 +155,27 @@ def test_points_p8_state_bitexact(ctx, torch_cuda, params):
     assert_cr_formula(d.cpu().numpy(), r_o, dr_o)
 
 
+@pytest.mark.parametrize("n", [64, 300, 5000])
+def test_overflowing_magnitude_among_ordinary_points(ctx, torch_cuda, n):
+    """A point whose |p|^2 overflows is finished before its first body and is
+    held while the other lanes of its wave run theirs (all away from the z axis,
+    so the bodies take the short square root and division): its distance stays
+    +inf, and the other points' the oracle's."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(n)
+    pts = rng.uniform(0.3, 0.6, (n, 3)).astype(F32)
+    huge = np.arange(5, n, 37)
+    pts[huge] = np.array([[1e20, 1e20, 1e20], [2e19, 0.5, 0.5], [0.5, 0.5, -3e19]], F32)[huge % 3]
+    g = dev.de_points(ca.Mandelbulb.classic(15, 2.0, ctx=ctx), gpu(torch, pts))
+    torch.cuda.synchronize()
+    g = g.cpu().numpy()
+    d = O.de_points(O.mandelbulb(15, 2.0), pts)[0]
+    assert np.isposinf(d[huge]).all()
+    assert_de_parity(g, d)
+
+
 @pytest.mark.parametrize("P", [2, 3, 5, 9])
 def test_trig_integer_power(ctx, torch_cuda, P):
     """Mandelbulb<P != 8>: the trig map with ocml transcendentals.  Iteration
