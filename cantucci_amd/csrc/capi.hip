@@ -158,6 +158,7 @@ int cth_ctx_set_launch(cth_ctx* c, int kernel, const cth_launch* l) {
     ls->chunk = l->chunk;
     ls->refill_min = l->refill_min;
     ls->dynamic = l->dynamic ? 1u : 0u;
+    ls->given = true;
     return CTH_OK;
 }
 

@@ -53,6 +53,7 @@ struct LaunchShape {
     uint32_t chunk = 256;      // indices per chunk
     uint32_t refill_min = 32;  // idle lanes that trigger a refill (1..64)
     uint32_t dynamic = 0;      // 0: static interleaved chunks, 1: atomic claims
+    bool given = false;        // set by the caller; else make_queue lets large static launches claim
 };
 
 // Device scratch slots of a context, grown on demand and kept until the

@@ -592,11 +592,8 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
         // their chunks where there are enough to even that out (4 M points at 15
         // iterations 558 -> 469 us, 300,000 points 65 -> 73).
         // Not in a capture that owns no counters (replays would share the ring's).
-        ls.dynamic = n / 256u >= (uint32_t)c.num_cus * spread.fill;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (ls.dynamic && capture_pool().stream != st && hipStreamIsCapturing(st, &cs) == hipSuccess &&
-            cs != hipStreamCaptureStatusNone)
-            ls.dynamic = 0;
+        ls.dynamic = n / 256u >= (uint32_t)c.num_cus * spread.fill && !foreign_capture(st);
+        ls.given = true;
         SrcPoints src{pts, powers, s.power};
         AdjOut out{grad_d, grad_p, grad_power, normals, grad_z0, grad_c};
         uint32_t blocks = 0;

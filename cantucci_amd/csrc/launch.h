@@ -34,6 +34,14 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
     if (iters) iters[i] = 0;
 }
 
+// Whether `st` is being captured into a graph that owns no counter entries: its
+// replays would take the ring's entries of launches in flight.
+inline bool foreign_capture(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return capture_pool().stream != st && hipStreamIsCapturing(st, &cs) == hipSuccess &&
+           cs != hipStreamCaptureStatusNone;
+}
+
 // A launch's workgroups and chunks.  Up to a chunk of `least` indices (64 or
 // fewer) for each of spread.fill waves per CU a launch is spread as thinly as possible; from four
 // chunks per wave on it grows to the launch shape's (and spread.most) waves.
@@ -46,8 +54,23 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
 // (24.6), 2 M points at power 8 34.5 (47), 700,000 at power 5 33 (49; 47 at
 // fill 32), tangent normals of 300,000 points with powers 48 (68; 69 at fill
 // 16), of 2 M points 153 (195; 175 without `most`).
-inline WorkQueue make_queue(Ctx& c, uint32_t total, const LaunchShape& ls, WaveSpread spread, uint32_t& blocks,
+//
+// A default static shape lets its waves claim once each of the waves that fit
+// on the chip (8 per SIMD, or spread.most) has 8 chunks of 64: 8 workgroups per
+// CU, chunks of up to 1024, which evens out regions that a static deal gives to
+// a few waves.  Below, the claims and their smaller share of first chunks cost
+// more than that gives.  Static / claimed, us: 256^3 grid 177 / 147, 160^3 (at
+// the line) 55.4 / 53.9, 112^3 24.4 / 26.1; 4 M points at power 5 164 / 147, of
+// tangent normals 252 / 228, 2^18 44 / 46; 4 poses of 1080p 1987 / 1536, one
+// 848 / 844; 24 mixed jobs 1796 / 1389.
+inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread spread, uint32_t& blocks,
                             hipStream_t st, uint32_t least = 64) {
+    const uint64_t resident = (uint64_t)c.num_cus * std::min(32u, spread.most);
+    if (!ls.given && !ls.dynamic && total >= 8u * 64u * resident && !foreign_capture(st)) {
+        ls.blocks_per_cu = 8 * (256 / ls.block);
+        ls.chunk = 1024;
+        ls.dynamic = 1;
+    }
     const uint64_t cus = (uint64_t)c.num_cus, waves_per_block = (uint64_t)ls.block / 64u;
     const uint64_t small = ((uint64_t)total + least - 1) / least;
     uint64_t waves = std::max(std::min(small, cus * spread.fill), std::min(small / 4u, cus * spread.most));

@@ -141,7 +141,9 @@ int cth_ctx_num_cus(const cth_ctx* ctx);
  * indices claimed per wave from the work counter (64..65536); refill_min the
  * number of idle lanes (1..64) at which a wave writes finished points and
  * takes new ones; dynamic = 1 claims chunks from an atomic counter, 0 walks
- * chunks w, w+W, w+2W, ... statically (W waves).  No counterpart in the
+ * chunks w, w+W, w+2W, ... statically (W waves).  While no shape has been set
+ * for a family whose default is static, its large launches claim chunks of up
+ * to 1024 all the same.  No counterpart in the
  * reference (its work is scheduled by a CPU thread pool,
  * src/mesh/mod.rs:60-63,141-148). */
 typedef struct cth_launch {

@@ -86,3 +86,62 @@ def test_outputs_do_not_depend_on_launch_shape(torch_cuda):
             print(f"{shape}: all {len(base)} outputs bit-identical")
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("off", [-1, 0, 1])
+@pytest.mark.parametrize("what", ["normals", "render"])
+def test_large_default_launches_claim(torch_cuda, what, off):
+    """Default static shapes claim their chunks from 8 chunks of 64 indices for
+    each resident wave on (16 waves per CU for the tangent normals, 32 for the
+    trace): below, at and beyond that size the outputs are those of a static
+    shape given by the caller; at it, also when the launch is captured into a
+    graph that has no counters of its own, over several replays with claiming
+    launches in between."""
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    from cantucci_amd import workloads as wl
+    torch = torch_cuda
+    auto, static = ca.Context(0, "parity"), ca.Context(0, "parity")
+    try:
+        for f in (_lib.CTH_KERNEL_TRACE, _lib.CTH_KERNEL_ADJOINT):
+            static.set_launch(f, 256, 16, 256, 32, dynamic=0)
+        cus = torch.cuda.get_device_properties(0).multi_processor_count
+        if what == "render":
+            W, H = 2048, 8 * 64 * 32 * cus // 2048 + off
+            cams = torch.from_numpy(wl.orbit_poses(1, 2, W, H)).cuda()
+            bufs = (torch.empty((1, H, W), device="cuda"), torch.empty((1, H, W), dtype=torch.int32, device="cuda"))
+
+            def run(c):
+                dev.render_depth(ca.Mandelbulb.classic(4, 2.0, ctx=c), cams, W, H, max_steps=12,
+                                 depth=bufs[0], steps=bufs[1])
+        else:
+            n = 8 * 64 * 16 * cus + 65 * off
+            pts = torch.rand((n, 3), device="cuda", generator=torch.Generator(device="cuda").manual_seed(7))
+            bufs = (torch.empty(n, device="cuda"), torch.empty((n, 3), device="cuda"))
+
+            def run(c):
+                dev.normals(ca.Mandelbulb.classic(6, 2.0, ctx=c), pts, out=bufs[1], d=bufs[0])
+
+        def result(f):
+            for b in bufs:
+                b.fill_(-1)
+            f()
+            torch.cuda.synchronize()
+            return [b.view(torch.int32).clone() for b in bufs]
+
+        def check(f):
+            return all(torch.equal(x, y) for x, y in zip(want, result(f)))
+
+        want = result(lambda: run(static))
+        assert check(lambda: run(auto))
+        if off == 0:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                run(auto)
+            for _ in range(3):
+                assert check(g.replay)
+                assert check(lambda: run(auto))
+    finally:
+        auto.close()
+        static.close()
