@@ -56,20 +56,24 @@ inline bool foreign_capture(hipStream_t st) {
 // 16), of 2 M points 153 (195; 175 without `most`).
 //
 // A default static shape lets its waves claim once each of the waves that fit
-// on the chip (8 per SIMD, or spread.most) has 8 chunks of 64: 8 workgroups per
+// on the chip (8 per SIMD, or spread.most) has 4 chunks of 128: 8 workgroups per
 // CU, chunks of up to 1024, which evens out regions that a static deal gives to
 // a few waves.  Below, the claims and their smaller share of first chunks cost
-// more than that gives.  Static / claimed, us: 256^3 grid 177 / 147, 160^3 (at
-// the line) 55.4 / 53.9, 112^3 24.4 / 26.1; 4 M points at power 5 164 / 147, of
-// tangent normals 252 / 228, 2^18 44 / 46; 4 poses of 1080p 1987 / 1536, one
-// 848 / 844; 24 mixed jobs 1796 / 1389.
+// more than that gives.  Static / claimed, us: 256^3 grid 177 / 147, 164^3 (just
+// over the line) 64.7 / 54.1, 112^3 24.4 / 26.1; 4 M points at power 5
+// 164 / 147, of tangent normals 252 / 228, 2^18 44 / 46; 4 poses of 1080p
+// 1987 / 1550, one 848 / 844; 24 mixed jobs 1796 / 1400.  Chunks of 64 take
+// twice the claims (200^3 grid at 6 iterations 76 us, static 73, with 128 66).
 inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread spread, uint32_t& blocks,
                             hipStream_t st, uint32_t least = 64) {
+    constexpr uint32_t kLeastClaim = 128;
     const uint64_t resident = (uint64_t)c.num_cus * std::min(32u, spread.most);
-    if (!ls.given && !ls.dynamic && total >= 8u * 64u * resident && !foreign_capture(st)) {
+    uint64_t lowest = 64;
+    if (!ls.given && !ls.dynamic && total >= 4u * kLeastClaim * resident && !foreign_capture(st)) {
         ls.blocks_per_cu = 8 * (256 / ls.block);
         ls.chunk = 1024;
         ls.dynamic = 1;
+        lowest = kLeastClaim;
     }
     const uint64_t cus = (uint64_t)c.num_cus, waves_per_block = (uint64_t)ls.block / 64u;
     const uint64_t small = ((uint64_t)total + least - 1) / least;
@@ -79,10 +83,10 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     WorkQueue q;
     q.waves = blocks * (uint32_t)waves_per_block;
     q.total = total;
-    // At least ~8 chunks per wave, so that launches still balance:
-    // chunk = clamp(total / (8 waves), 64, configured), a multiple of 64.
+    // About 8 chunks per wave, so that launches still balance:
+    // chunk = clamp(total / (8 waves), lowest, configured), a multiple of 64.
     uint64_t fair = (uint64_t)total / ((uint64_t)q.waves * 8u);
-    uint64_t ch = std::min<uint64_t>(ls.chunk, std::max<uint64_t>(64, fair));
+    uint64_t ch = std::min<uint64_t>(ls.chunk, std::max(lowest, fair));
     q.chunk = least < 64 ? least : (uint32_t)(ch & ~63ull);
     q.chunks = (uint32_t)(((uint64_t)total + q.chunk - 1) / q.chunk);
     q.refill_min = ls.refill_min < 1 ? 1 : (ls.refill_min > 64 ? 64 : ls.refill_min);
