@@ -73,6 +73,10 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
     // refill meets those of every wave in the same job on one address, and 18.4 M
     // points in 24 jobs then took 3.85 ms (2.27 so).
     uint32_t sjob = kNoJob;
+    // The job of the window's next index and the first index after that job:
+    // lanes take points of one job at a time, so that its description comes
+    // through scalar loads (per lane: a search and 13 gathered words a refill).
+    uint32_t wjob = 0, wend = 0;
     unsigned long long stamp = 0;
     float r = idle_start(ev, u);
     Window win;
@@ -106,20 +110,23 @@ __global__ __launch_bounds__(256) void k_jobs(const JobDev* __restrict__ jobs, u
             uint64_t need = wave & ~live_m;
             while (need != 0) {
                 if (win.next >= win.end && !next_chunk(q, win)) break;
-                const uint32_t avail = win.end - win.next;
+                if (win.next >= wend) {
+                    // the last offset <= the index (a wave's chunks ascend)
+                    uint32_t hi = njobs;
+                    while (hi - wjob > 1) {
+                        const uint32_t mid = (wjob + hi) >> 1;
+                        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)offs[mid]) <= win.next) wjob = mid; else hi = mid;
+                    }
+                    wend = (uint32_t)__builtin_amdgcn_readfirstlane((int)offs[wjob + 1]);
+                }
+                const JobDev& J = jobs[wjob];
+                const uint32_t avail = (win.end < wend ? win.end : wend) - win.next;
                 const uint32_t nneed = (uint32_t)__popcll(need);
                 const uint32_t rank = lane_rank(need);
                 const bool take = __builtin_amdgcn_inverse_ballot_w64(need) && rank < avail;
                 if (take) {
                     idx = win.next + rank;
-                    // job of idx: the last offset <= idx
-                    uint32_t lo = 0, hi = njobs;
-                    while (hi - lo > 1) {
-                        uint32_t mid = (lo + hi) >> 1;
-                        if (offs[mid] <= idx) lo = mid; else hi = mid;
-                    }
-                    job = lo;
-                    const JobDev& J = jobs[job];
+                    job = wjob;
                     uint32_t local = idx - J.offset;
                     uint32_t i = fdiv(local, J.n2);
                     uint32_t rem = local - i * J.n2.d;

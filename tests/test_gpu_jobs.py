@@ -90,6 +90,37 @@ def test_p8_jobs_match_oracle(ctx, torch_cuda):
     js.close()
 
 
+@pytest.mark.parametrize("njobs", [1, 7, 1024])
+def test_tiny_jobs_share_a_wave(ctx, torch_cuda, njobs):
+    """A wave takes points of one job at a time: sets whose jobs end within a
+    wave's 64 points, up to the largest set, with a cap per job.  Each job's
+    distances are those of a grid launch of its own, bit for bit, and it has a
+    stamp."""
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(njobs)
+    jobs = [dict(n=int(n), power=8.0, max_iters=int(c))
+            for n, c in zip(rng.integers(2, 6, njobs), rng.integers(1, 16, njobs))]
+    js = dev.JobSet(ctx, _lib.CTH_SHAPE_MANDELBULB, 2.0, jobs)
+    d = torch.full((js.total,), -1.0, device="cuda")
+    nrm = torch.empty((js.total, 3), device="cuda")
+    done = torch.zeros(js.njobs, dtype=torch.int64, device="cuda")
+    start = torch.zeros(1, dtype=torch.int64, device="cuda")
+    js.run(d, nrm, done, start)
+    grids = {}
+    for j in jobs:
+        key = (j["n"], j["max_iters"])
+        if key not in grids:
+            shape = ca.Mandelbulb.classic(j["max_iters"], 2.0, ctx=ctx)
+            grids[key] = dev.de_grid(shape, (-1.5,) * 3, (1.5,) * 3, j["n"], j["n"] - 1.0).flatten()
+    want = torch.cat([grids[j["n"], j["max_iters"]] for j in jobs])
+    assert torch.equal(d.view(torch.int32), want.view(torch.int32))
+    assert (done >= start).all()
+    js.close()
+
+
 def test_trig_jobs_statistics(ctx, torch_cuda):
     import cantucci_amd as ca
     from cantucci_amd import _lib
