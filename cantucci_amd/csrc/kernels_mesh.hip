@@ -84,46 +84,10 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
     return v;
 }
 
-// Exclusive scan over the workgroup (all threads must call it); `total`
-// receives the sum.  `wsum` holds one slot per wave.
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wsum, uint32_t& total) {
-    const uint32_t inc = wave_incl_scan(v);
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    if (lane == 63u) wsum[wave] = inc;
-    __syncthreads();
-    uint32_t off = 0, tot = 0;
-    const uint32_t nw = blockDim.x >> 6;
-    for (uint32_t w = 0; w < nw; ++w) {
-        uint32_t s = wsum[w];
-        off += (w < wave) ? s : 0u;
-        tot += s;
-    }
-    __syncthreads();
-    total = tot;
-    return off + inc - v;
-}
-
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t& total) {
     const uint32_t inc = wave_incl_scan(v);
     total = (uint32_t)__shfl((int)inc, 63, 64);
     return inc - v;
-}
-
-__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* wsum) {
-    uint32_t t;
-    (void)block_excl_scan(v, wsum, t);
-    return t;
-}
-
-struct MeshDims {
-    uint32_t res, lg, n1, cells;
-    float fres;
-};
-
-__device__ __forceinline__ void cell_xyz(const MeshDims& m, uint32_t c, uint32_t& x, uint32_t& y, uint32_t& z) {
-    z = c & (m.res - 1u);
-    y = (c >> m.lg) & (m.res - 1u);
-    x = c >> (2u * m.lg);
 }
 
 // ---------------------------------------------------------------------------
@@ -135,41 +99,178 @@ __device__ __forceinline__ void cell_xyz(const MeshDims& m, uint32_t c, uint32_t
 // touch) are numbered from the previous unit's offset.
 // ---------------------------------------------------------------------------
 
+// Sign fields of a corner plane: bit i of `f` is the IEEE sign bit of corner i
+// of the plane's n1 x n1 (GridTable order), one wave ballot per 64 corners, so
+// each corner is loaded once, coalesced, and a cell row is classified with a
+// few 64-bit operations (the cells' own eight corners took eight loads each:
+// 64 leaves of 64^3 cells counted in 38 us, now 19).
+template <int LG>
+struct Plane {
+    static constexpr uint32_t RES = 1u << LG, N1 = RES + 1;
+    static constexpr uint32_t CORNERS = N1 * N1;
+    static constexpr uint32_t WORDS = (CORNERS + 63) / 64;
+    static constexpr uint64_t CELLS = RES == 64 ? ~0ull : (1ull << (RES & 63u)) - 1ull;  // a row's cells
+    static constexpr uint32_t BATCH = (WORDS + kMeshBlock / 64 - 1) / (kMeshBlock / 64);  // loads in flight per wave
+    uint64_t f[WORDS + 1];
+    // Bits [o, o + 64).
+    __device__ __forceinline__ uint64_t window(uint32_t o) const {
+        const uint32_t w = o >> 6, b = o & 63u;
+        return (f[w] >> b) | ((f[w + 1] << 1) << (63u - b));
+    }
+};
+
+// The fields of N consecutive corner planes from `D` on (sgn[k]) and, if
+// `neg` is given, the `< 0.0` field of plane `neg_plane`; all threads call it.
+template <int LG>
+__device__ __forceinline__ void plane_fields(const float* __restrict__ D, uint32_t n, Plane<LG>* sgn, Plane<LG>* neg,
+                                             uint32_t neg_plane) {
+    using P = Plane<LG>;
+    const uint32_t lane = threadIdx.x & 63u, nwaves = blockDim.x >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (uint32_t p = 0; p < n; ++p) {
+        const float* C = D + (size_t)p * P::CORNERS;
+        for (uint32_t w0 = wave * P::BATCH; w0 < P::WORDS; w0 += nwaves * P::BATCH) {
+            float v[P::BATCH];
+#pragma unroll
+            for (uint32_t k = 0; k < P::BATCH; ++k) {
+                const uint32_t i = (w0 + k) * 64 + lane;
+                v[k] = i < P::CORNERS ? C[i] : 0.0f;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < P::BATCH; ++k) {
+                if (w0 + k >= P::WORDS) break;
+                const uint64_t ms = wave_mask((int)__float_as_uint(v[k]) < 0);
+                if (lane == 0) sgn[p].f[w0 + k] = ms;
+                if (neg && p == neg_plane) {
+                    const uint64_t mn = wave_mask(v[k] < 0.0f);
+                    if (lane == 0) neg->f[w0 + k] = mn;
+                }
+            }
+        }
+        if (threadIdx.x == 0) sgn[p].f[P::WORDS] = 0;
+    }
+    if (neg && threadIdx.x == 0) neg->f[P::WORDS] = 0;
+}
+
+// Cell row y between corner planes A (x) and B (x + 1): crossing bits and the
+// +x / +y / +z quad bits of its cells (src/mesh/buffer.rs:113-147, 299-350).
+template <int LG>
+struct PlaneRow {
+    uint64_t cross, fx, fy, fz;
+    __device__ __forceinline__ PlaneRow(const Plane<LG>& A, const Plane<LG>& B, uint32_t x, uint32_t y) {
+        using P = Plane<LG>;
+        const uint32_t o = y * P::N1;
+        const uint64_t a = A.window(o), a1 = A.window(o + 1), b = A.window(o + P::N1), b1 = A.window(o + P::N1 + 1);
+        const uint64_t c = B.window(o), c1 = B.window(o + 1), d = B.window(o + P::N1), d1 = B.window(o + P::N1 + 1);
+        const uint64_t all = a & a1 & b & b1 & c & c1 & d & d1, any = a | a1 | b | b1 | c | c1 | d | d1;
+        cross = any & ~all & P::CELLS;              // not all 8 signs equal
+        const uint64_t zpos = P::CELLS & ~1ull;     // z > 0
+        fx = y > 0 ? (a ^ c) & zpos : 0;            // corner 0 vs 4, needs y, z > 0
+        fy = x > 0 ? (a ^ b) & zpos : 0;            // corner 0 vs 2, needs x, z > 0
+        fz = x > 0 && y > 0 ? (a ^ a1) & P::CELLS : 0;  // corner 0 vs 1, needs x, y > 0
+    }
+    __device__ __forceinline__ uint32_t faces() const {
+        return (uint32_t)(__popcll(fx) + __popcll(fy) + __popcll(fz));
+    }
+};
+
 // Per unit: vertex count and index count (6 per quad); slot `units` of both
 // arrays is zeroed so that an exclusive scan over units + 1 entries ends
 // with the totals.  With `cross` non-null it also writes the leaf's
 // crossing words (bit c of word c / 64 = cell c crosses), the layout
-// cth_sample_spans_dev uses (res^2 is a multiple of 256, so every wave's
-// 64 cells are one word).
-__global__ __launch_bounds__(kMeshBlock) void k_mesh_count_p(const float* __restrict__ dists, MeshDims m,
-                                                             uint32_t units, uint64_t* __restrict__ vcnt,
-                                                             uint64_t* __restrict__ icnt, uint64_t* __restrict__ cross) {
-    __shared__ uint32_t wsum[kMeshBlock / 64];
-    const uint32_t u = blockIdx.x;
-    const uint32_t leaf = u >> m.lg, x = u & (m.res - 1u);
-    const float* D = dists + (size_t)leaf * m.n1 * m.n1 * m.n1;
-    const uint32_t pc = m.res * m.res;
-    const uint32_t nwords = m.cells >> 6;
+// cth_sample_spans_dev uses.
+template <int LG>
+__global__ __launch_bounds__(kMeshBlock) void k_mesh_count_p(const float* __restrict__ dists, uint32_t units,
+                                                             uint64_t* __restrict__ vcnt, uint64_t* __restrict__ icnt,
+                                                             uint64_t* __restrict__ cross) {
+    using P = Plane<LG>;
+    __shared__ P planes[2];
+    const uint32_t u = blockIdx.x, leaf = u >> LG, x = u & (P::RES - 1u), lane = threadIdx.x;
+    plane_fields<LG>(dists + ((size_t)leaf * P::N1 + x) * P::CORNERS, 2, planes, nullptr, 0);
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
     uint32_t nv = 0, nf = 0;
-    for (uint32_t j = threadIdx.x; j < pc; j += blockDim.x) {
-        const uint32_t y = j >> m.lg, z = j & (m.res - 1u);
-        float d[8];
-        const uint32_t mk = load_cell(D, m.n1, x, y, z, d);
-        const bool cr = crossing(mk);
-        nv += cr ? 1u : 0u;
-        nf += (uint32_t)__popc(face_bits(mk, x, y, z));
-        const uint64_t bits = wave_mask(cr);
-        if (cross && (threadIdx.x & 63u) == 0) cross[(size_t)leaf * nwords + ((x * pc + j) >> 6)] = bits;
+    uint64_t bits = 0;
+    if (lane < P::RES) {
+        const PlaneRow<LG> row(planes[0], planes[1], x, lane);
+        bits = row.cross;
+        nv = (uint32_t)__popcll(bits);
+        nf = row.faces();
     }
-    nv = block_sum(nv, wsum);
-    nf = block_sum(nf, wsum);
-    if (threadIdx.x == 0) {
-        vcnt[u] = nv;
-        icnt[u] = 6ull * nf;
+    if (cross) {
+        uint64_t* out = cross + (size_t)u * (P::RES * P::RES / 64);
+        if constexpr (LG == 6) {
+            out[lane] = bits;
+        } else {  // two rows to a word
+            const uint64_t odd = (uint64_t)(uint32_t)__shfl_down((int)(uint32_t)bits, 1, 64);
+            if (lane < P::RES && (lane & 1u) == 0) out[lane >> 1] = bits | odd << 32;
+        }
+    }
+    uint32_t tv, tf;
+    (void)wave_excl_scan(nv, tv);
+    (void)wave_excl_scan(nf, tf);
+    if (lane == 0) {
+        vcnt[u] = tv;
+        icnt[u] = 6ull * tf;
         if (u == 0) {
             vcnt[units] = 0;
             icnt[units] = 0;
         }
+    }
+}
+
+// Exclusive scans of up to kScanOne counts of both kinds in one workgroup:
+// entry i * 2^lg goes to voff[i] / ioff[i], and the totals also to host memory
+// (pinned).  One launch, where a library scan of each, the leaves' offsets and
+// two copies of the totals took seven, half of them longer to launch than to
+// run (one leaf of 64^3 cells: 27 us of launches a count).
+constexpr uint32_t kScanOne = 16384;
+__global__ __launch_bounds__(1024) void k_scan_counts(const uint64_t* __restrict__ vcnt,
+                                                      const uint64_t* __restrict__ icnt, uint32_t n, uint32_t lg,
+                                                      uint64_t* __restrict__ voff, uint64_t* __restrict__ ioff,
+                                                      uint64_t* totals) {
+    __shared__ uint64_t wsum[2][16];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint64_t carry[2] = {0, 0};
+    for (uint32_t base = 0; base < n; base += 4096) {
+        const uint32_t i0 = base + 4 * threadIdx.x;
+        uint64_t c[2][4], sum[2], inc[2];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool in = i0 + k < n;
+            c[0][k] = in ? vcnt[i0 + k] : 0;
+            c[1][k] = in ? icnt[i0 + k] : 0;
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            inc[a] = sum[a] = c[a][0] + c[a][1] + c[a][2] + c[a][3];
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint64_t t = __shfl_up((unsigned long long)inc[a], d, 64);
+                if (lane >= (uint32_t)d) inc[a] += t;
+            }
+            if (lane == 63u) wsum[a][wave] = inc[a];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            uint64_t at = carry[a] + inc[a] - sum[a];
+            for (uint32_t w = 0; w < 16; ++w) {
+                at += w < wave ? wsum[a][w] : 0;
+                carry[a] += wsum[a][w];
+            }
+            uint64_t* off = a ? ioff : voff;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (i0 + k < n && ((i0 + k) & ((1u << lg) - 1u)) == 0) off[(i0 + k) >> lg] = at;
+                at += c[a][k];
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < 2) {
+        (threadIdx.x ? ioff : voff)[n >> lg] = carry[threadIdx.x];
+        totals[threadIdx.x] = carry[threadIdx.x];
     }
 }
 
@@ -282,77 +383,114 @@ __device__ __forceinline__ void emit_quads(uint32_t* out, uint32_t fb, bool neg,
     }
 }
 
-// One workgroup per plane unit.  LDS: the crossing words of planes x and
-// x - 1 and their exclusive popcount prefixes (res^2 / 64 words each).  The
-// vertex records temporarily hold the leaf's 6-tap half-steps in their normal
-// slots (src/mesh/buffer.rs:257: 0.7 * (e - s) / res per axis).
+// One workgroup per plane unit.  The rows of cell planes x and x - 1 are
+// classified from the sign fields of corner planes x - 1, x, x + 1; the cells
+// with a vertex and the corners with quads are listed in LDS, so that every
+// lane places one (placing a vertex takes up to 12 divisions, which ran for the
+// few crossing cells of each 64).  A unit's place in its leaf is the sum of the
+// counts of the units before it.  The vertex records temporarily hold the
+// leaf's 6-tap half-steps in their normal slots (src/mesh/buffer.rs:257:
+// 0.7 * (e - s) / res per axis).
+template <int LG>
 __global__ __launch_bounds__(kMeshBlock) void k_mesh_emit_p(
-    const float* __restrict__ spans, const float* __restrict__ dists, MeshDims m, const uint64_t* __restrict__ uv,
-    const uint64_t* __restrict__ ui, const uint64_t* __restrict__ voff, const uint64_t* __restrict__ ioff,
+    const float* __restrict__ spans, const float* __restrict__ dists, const uint64_t* __restrict__ vcnt,
+    const uint64_t* __restrict__ icnt, const uint64_t* __restrict__ voff, const uint64_t* __restrict__ ioff,
     float* __restrict__ verts, uint32_t* __restrict__ idx) {
-    extern __shared__ uint64_t lds_words[];
-    __shared__ uint32_t wsum[kMeshBlock / 64];
-    const uint32_t u = blockIdx.x;
-    const uint32_t leaf = u >> m.lg, x = u & (m.res - 1u);
-    const uint32_t pc = m.res * m.res, pw = pc >> 6;
-    uint64_t* wc = lds_words;   // plane x
-    uint64_t* wp = wc + pw;     // plane x - 1
-    uint32_t* prc = reinterpret_cast<uint32_t*>(wp + pw);
-    uint32_t* prp = prc + pw;
-    const float* D = dists + (size_t)leaf * m.n1 * m.n1 * m.n1;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    using P = Plane<LG>;
+    constexpr uint32_t RES = P::RES;
+    __shared__ P planes[3], negs;  // corner planes x - 1, x, x + 1; `< 0` of plane x
+    __shared__ uint64_t cross[2][RES], faces[3][RES];  // cell plane x (0), x - 1 (1); +x, +y, +z quads of plane x
+    __shared__ uint32_t vpre[2][RES], fpre[RES], cpre[RES];  // vertices, quads, corners with quads before the row
+    __shared__ uint32_t totals[2], vbase[2], fbase;
+    __shared__ uint16_t vlist[RES * RES], flist[RES * RES];
+    const uint32_t u = blockIdx.x, leaf = u >> LG, x = u & (RES - 1u);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const float* D = dists + (size_t)leaf * P::N1 * P::CORNERS;
 
-    const uint32_t nplanes = (x > 0) ? 2u : 1u;
-    for (uint32_t w = wave; w < nplanes * pw; w += nwaves) {
-        const uint32_t px = (w < pw) ? x : x - 1u, ww = (w < pw) ? w : w - pw;
-        const uint32_t j = (ww << 6) | lane;
-        float d[8];
-        const bool cr = crossing(load_cell(D, m.n1, px, j >> m.lg, j & (m.res - 1u), d));
-        const uint64_t bits = wave_mask(cr);
-        if (lane == 0) ((w < pw) ? wc : wp)[ww] = bits;
-    }
+    if (x > 0)
+        plane_fields<LG>(D + (size_t)(x - 1) * P::CORNERS, 3, planes, &negs, 1);
+    else
+        plane_fields<LG>(D, 2, planes + 1, &negs, 0);
     __syncthreads();
-    if (wave < nplanes) {  // pw <= 64: one wave scans one plane's words
-        const uint64_t* words = (wave == 0) ? wc : wp;
-        uint32_t* pre = (wave == 0) ? prc : prp;
-        const uint32_t v = (lane < pw) ? (uint32_t)__popcll(words[lane]) : 0u;
-        uint32_t tot;
-        const uint32_t ex = wave_excl_scan(v, tot);
-        if (lane < pw) pre[lane] = ex;
-    }
-    __syncthreads();
-
-    const size_t u0 = (size_t)leaf * m.res;  // the leaf's first unit
-    const uint32_t vb_x = (uint32_t)(uv[u] - uv[u0]);
-    const uint32_t vb_p = (x > 0) ? (uint32_t)(uv[u - 1] - uv[u0]) : 0u;
-    auto pt = [&](uint32_t px, uint32_t py, uint32_t pz) {
-        const bool cur = (px == x);
-        const uint32_t j = (py << m.lg) | pz, w = j >> 6, b = j & 63u;
-        const uint64_t word = cur ? wc[w] : wp[w];
-        const uint64_t below = (b == 0) ? 0ull : (word & ((~0ull) >> (64u - b)));
-        return (cur ? vb_x + prc[w] : vb_p + prp[w]) + (uint32_t)__popcll(below);
-    };
-    float s1[3], step[3], delta[3];
-    leaf_frame(spans + 6 * (size_t)leaf, m.fres, s1, step, delta);
-    float* vout = verts + 7 * voff[leaf];
-    uint32_t* iout = idx + ioff[leaf] + (ui[u] - ui[u0]);
-
-    uint32_t fcarry = 0;
-    for (uint32_t base = 0; base < pc; base += blockDim.x) {
-        const uint32_t j = base + threadIdx.x;  // pc is a multiple of the block
-        const uint32_t y = j >> m.lg, z = j & (m.res - 1u);
-        float d[8];
-        const uint32_t mk = load_cell(D, m.n1, x, y, z, d);
-        const uint32_t fb = face_bits(mk, x, y, z);
-        uint32_t tile_faces;
-        const uint32_t frank = block_excl_scan((uint32_t)__popc(fb), wsum, tile_faces);
-        if (crossing(mk)) {
-            float p[3];
-            place_vertex(d, x, y, z, s1, step, p);
-            put_vertex(vout + 7 * (size_t)pt(x, y, z), p, delta);
+    if (wave == 0) {
+        const uint32_t y = lane < RES ? lane : RES - 1u;
+        PlaneRow<LG> row(planes[1], planes[2], x, y);
+        if (lane >= RES) row.cross = row.fx = row.fy = row.fz = 0;
+        uint32_t tv, tf, tc;
+        const uint32_t ve = wave_excl_scan((uint32_t)__popcll(row.cross), tv);
+        const uint32_t fe = wave_excl_scan(row.faces(), tf);
+        const uint32_t ce = wave_excl_scan((uint32_t)__popcll(row.fx | row.fy | row.fz), tc);
+        if (lane < RES) {
+            cross[0][y] = row.cross;
+            faces[0][y] = row.fx;
+            faces[1][y] = row.fy;
+            faces[2][y] = row.fz;
+            vpre[0][y] = ve;
+            fpre[y] = fe;
+            cpre[y] = ce;
         }
-        if (fb) emit_quads(iout + 6ull * (fcarry + frank), fb, d[0] < 0.0f, x, y, z, pt);
-        fcarry += tile_faces;
+        if (lane == 0) {
+            totals[0] = tv;
+            totals[1] = tc;
+        }
+    } else if (wave == 1 && x > 0) {
+        const uint32_t y = lane < RES ? lane : RES - 1u;
+        const uint64_t bits = lane < RES ? PlaneRow<LG>(planes[0], planes[1], x - 1u, y).cross : 0;
+        uint32_t tv;
+        const uint32_t ve = wave_excl_scan((uint32_t)__popcll(bits), tv);
+        if (lane < RES) {
+            cross[1][y] = bits;
+            vpre[1][y] = ve;
+        }
+    } else if (wave == 2) {
+        // counts of the leaf's units before this one
+        const uint32_t v = lane < x ? (uint32_t)vcnt[u - x + lane] : 0u;
+        const uint32_t f = lane < x ? (uint32_t)icnt[u - x + lane] : 0u;
+        uint32_t tv, tf;
+        const uint32_t ve = wave_excl_scan(v, tv);
+        (void)wave_excl_scan(f, tf);
+        if (lane == 0) {
+            vbase[0] = tv;
+            fbase = tf;
+        }
+        if (lane + 1u == x) vbase[1] = ve;
+    }
+    __syncthreads();
+    const uint32_t tv = totals[0], tc = totals[1];
+    if (tv == 0 && tc == 0) return;
+    auto below = [](uint64_t word, uint32_t z) { return (uint32_t)__popcll(word & ((1ull << z) - 1ull)); };
+    for (uint32_t j = threadIdx.x; j < RES * RES; j += kMeshBlock) {
+        const uint32_t y = j >> LG, z = j & (RES - 1u);
+        const uint64_t c = cross[0][y], fx = faces[0][y], fy = faces[1][y], fz = faces[2][y];
+        if ((c >> z) & 1u) vlist[vpre[0][y] + below(c, z)] = (uint16_t)j;
+        const uint32_t fb =
+            ((uint32_t)(fx >> z) & 1u) | ((uint32_t)(fy >> z) & 1u) << 1 | ((uint32_t)(fz >> z) & 1u) << 2;
+        if (fb) flist[cpre[y] + below(fx | fy | fz, z)] = (uint16_t)(j | fb << 12);
+    }
+    __syncthreads();
+
+    const uint32_t vb_x = vbase[0], vb_p = vbase[1];
+    float s1[3], step[3], delta[3];
+    leaf_frame(spans + 6 * (size_t)leaf, (float)RES, s1, step, delta);
+    float* vout = verts + 7 * (voff[leaf] + vb_x);
+    for (uint32_t j = threadIdx.x; j < tv; j += kMeshBlock) {
+        const uint32_t cell = vlist[j], y = cell >> LG, z = cell & (RES - 1u);
+        float d[8];
+        (void)load_cell(D, P::N1, x, y, z, d);
+        float p[3];
+        place_vertex(d, x, y, z, s1, step, p);
+        put_vertex(vout + 7 * (size_t)j, p, delta);
+    }
+    auto pt = [&](uint32_t px, uint32_t py, uint32_t pz) {
+        const uint32_t k = px == x ? 0u : 1u;
+        return (k ? vb_p : vb_x) + vpre[k][py] + below(cross[k][py], pz);
+    };
+    uint32_t* iout = idx + ioff[leaf] + fbase;
+    for (uint32_t j = threadIdx.x; j < tc; j += kMeshBlock) {
+        const uint32_t e = flist[j], cell = e & 0xFFFu, y = cell >> LG, z = cell & (RES - 1u);
+        const uint32_t q = fpre[y] + below(faces[0][y], z) + below(faces[1][y], z) + below(faces[2][y], z);
+        const bool neg = (negs.window(y * P::N1) >> z) & 1u;
+        emit_quads(iout + 6ull * q, e >> 12, neg, x, y, z, pt);
     }
 }
 
@@ -908,14 +1046,9 @@ __global__ void k_mesh_fd_combine(const float* __restrict__ taps, uint32_t n, fl
 
 inline uint32_t cdiv_u32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-int mesh_dims(uint32_t res, MeshDims& m) {
+int check_res(uint32_t res) {
     if (res == 0 || (res & (res - 1)) != 0 || res > 64)
         return fail(CTH_E_INVALID, "mesh resolution must be a power of two in [1, 64]");
-    m.res = res;
-    m.lg = (uint32_t)__builtin_ctz(res);
-    m.n1 = res + 1;
-    m.cells = res * res * res;
-    m.fres = (float)res;
     return CTH_OK;
 }
 
@@ -955,28 +1088,23 @@ static int scan_pair(Ctx& c, uint64_t* counts, size_t cnt, uint64_t* voff, uint6
     return rc;
 }
 
-// Plane-unit counts and their exclusive scans, in the context's scratch:
-// *uoff holds units + 1 vertex offsets followed by units + 1 index offsets.
-static int plane_offsets(Ctx& c, const float* dists, const MeshDims& m, uint32_t nleaves, uint64_t* cross,
-                         uint64_t** uoff, hipStream_t st) {
-    const size_t units = (size_t)nleaves * m.res;
+// Plane-unit counts in the context's scratch: *counts holds units + 1 vertex
+// counts followed by units + 1 index counts.
+static int plane_counts(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint64_t* cross, uint64_t** counts,
+                        hipStream_t st) {
+    const size_t units = (size_t)nleaves * res;
     if (units >= (size_t(1) << 31)) return fail(CTH_E_INVALID, "more than 2^31 mesh plane units");
     const size_t cnt = units + 1;
-    uint64_t* counts = nullptr;
-    if (c.scratch(WS_COUNTS, 2 * cnt * sizeof(uint64_t), (void**)&counts) ||
-        c.scratch(WS_UOFF, 2 * cnt * sizeof(uint64_t), (void**)uoff))
+    if (c.scratch(WS_COUNTS, 2 * cnt * sizeof(uint64_t), (void**)counts))
         return fail(CTH_E_NOMEM, "mesh scratch allocation failed");
-    hipLaunchKernelGGL(k_mesh_count_p, dim3((uint32_t)units), dim3(kMeshBlock), 0, st, dists, m, (uint32_t)units,
-                       counts, counts + cnt, cross);
-    int rc = check_hip(hipGetLastError(), "mesh plane count launch");
-    if (!rc) rc = scan_pair(c, counts, cnt, *uoff, *uoff + cnt, st);
-    return rc;
+    hipLaunchKernelGGL((res == 64 ? k_mesh_count_p<6> : k_mesh_count_p<5>), dim3((uint32_t)units), dim3(kMeshBlock), 0,
+                       st, dists, (uint32_t)units, *counts, *counts + cnt, cross);
+    return check_hip(hipGetLastError(), "mesh plane count launch");
 }
 
 int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint64_t* voff, uint64_t* ioff,
                uint64_t* cross, uint64_t totals[2], hipStream_t st) {
-    MeshDims m;
-    if (int rc = mesh_dims(res, m)) return rc;
+    if (int rc = check_res(res)) return rc;
     totals[0] = totals[1] = 0;
     if (nleaves == 0) {
         const uint64_t zero[2] = {0, 0};
@@ -986,10 +1114,12 @@ int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint6
         return rc;
     }
     int rc = CTH_OK;
+    const uint32_t lg = res <= 16 ? 0u : res == 32 ? 5u : 6u;  // units per leaf
+    const size_t units = (size_t)nleaves << lg;
+    uint64_t* counts = nullptr;
     if (res <= 16) {
         // wave per leaf: the counts are per leaf already
-        const size_t cnt = (size_t)nleaves + 1;
-        uint64_t* counts = nullptr;
+        const size_t cnt = units + 1;
         if (c.scratch(WS_COUNTS, 2 * cnt * sizeof(uint64_t), (void**)&counts))
             return fail(CTH_E_NOMEM, "mesh count scratch allocation failed");
         switch (res) {
@@ -1000,20 +1130,33 @@ int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint6
             default: LAUNCH_COUNT_W(16); break;
         }
         rc = check_hip(hipGetLastError(), "mesh count launch");
-        if (!rc) rc = scan_pair(c, counts, cnt, voff, ioff, st);
     } else {
-        // plane units, then the leaves' offsets from the units'
-        uint64_t* uoff = nullptr;
-        rc = plane_offsets(c, dists, m, nleaves, cross, &uoff, st);
-        if (!rc) {
-            const size_t units = (size_t)nleaves * res;
-            hipLaunchKernelGGL(k_leaf_offsets, dim3(cdiv_u32((uint64_t)nleaves + 1, 256)), dim3(256), 0, st, uoff,
-                               uoff + units + 1, nleaves, res, voff, ioff);
+        rc = plane_counts(c, dists, nleaves, res, cross, &counts, st);
+    }
+    if (!rc && units <= kScanOne) {
+        hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, counts, counts + units + 1, (uint32_t)units, lg,
+                           voff, ioff, c.pinned);
+        rc = check_hip(hipGetLastError(), "mesh scan launch");
+    } else if (!rc) {
+        uint64_t* uoff[2] = {voff, ioff};
+        if (lg) {
+            // the leaves' offsets from the units'
+            uint64_t* base = nullptr;
+            if (c.scratch(WS_UOFF, 2 * (units + 1) * sizeof(uint64_t), (void**)&base))
+                return fail(CTH_E_NOMEM, "mesh scratch allocation failed");
+            uoff[0] = base;
+            uoff[1] = base + units + 1;
+        }
+        rc = scan_pair(c, counts, units + 1, uoff[0], uoff[1], st);
+        if (!rc && lg) {
+            hipLaunchKernelGGL(k_leaf_offsets, dim3(cdiv_u32((uint64_t)nleaves + 1, 256)), dim3(256), 0, st, uoff[0],
+                               uoff[1], nleaves, res, voff, ioff);
             rc = check_hip(hipGetLastError(), "leaf offsets launch");
         }
+        if (!rc) rc = check_hip(hipMemcpyAsync(c.pinned, voff + nleaves, 8, hipMemcpyDeviceToHost, st), "D2H totals");
+        if (!rc)
+            rc = check_hip(hipMemcpyAsync(c.pinned + 1, ioff + nleaves, 8, hipMemcpyDeviceToHost, st), "D2H totals");
     }
-    if (!rc) rc = check_hip(hipMemcpyAsync(c.pinned, voff + nleaves, 8, hipMemcpyDeviceToHost, st), "D2H totals");
-    if (!rc) rc = check_hip(hipMemcpyAsync(c.pinned + 1, ioff + nleaves, 8, hipMemcpyDeviceToHost, st), "D2H totals");
     int rs = check_hip(hipStreamSynchronize(st), "mesh count sync");
     if (!rc && !rs) {
         totals[0] = c.pinned[0];
@@ -1025,8 +1168,7 @@ int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint6
 int mesh_emit(Ctx& c, const cth_shape& s, const float* spans, const float* dists, uint32_t nleaves, uint32_t res,
               int normals, const uint64_t* voff, const uint64_t* ioff, uint64_t nverts, float* verts,
               uint32_t* idx, hipStream_t st) {
-    MeshDims m;
-    if (int rc = mesh_dims(res, m)) return rc;
+    if (int rc = check_res(res)) return rc;
     if (normals != CTH_NORMALS_FD6 && normals != CTH_NORMALS_TANGENT && normals != CTH_NORMALS_DEFERRED)
         return fail(CTH_E_INVALID, "unknown normals mode");
     if (normals == CTH_NORMALS_TANGENT && s.kind == CTH_SHAPE_SPHERE)
@@ -1041,13 +1183,12 @@ int mesh_emit(Ctx& c, const cth_shape& s, const float* spans, const float* dists
             default: LAUNCH_EMIT_W(16); break;
         }
     } else {
-        // the plane units' offsets (recounted: a count call leaves only the leaves')
-        uint64_t* uoff = nullptr;
-        if (int rc = plane_offsets(c, dists, m, nleaves, nullptr, &uoff, st)) return rc;
+        // the plane units' counts (recounted: a count call leaves only the leaves' offsets)
+        uint64_t* counts = nullptr;
+        if (int rc = plane_counts(c, dists, nleaves, res, nullptr, &counts, st)) return rc;
         const size_t units = (size_t)nleaves * res;
-        const size_t lds = 2 * (size_t)(m.res * m.res / 64) * (sizeof(uint64_t) + sizeof(uint32_t));
-        hipLaunchKernelGGL(k_mesh_emit_p, dim3((uint32_t)units), dim3(kMeshBlock), lds, st, spans, dists, m, uoff,
-                           uoff + units + 1, voff, ioff, verts, idx);
+        hipLaunchKernelGGL((res == 64 ? k_mesh_emit_p<6> : k_mesh_emit_p<5>), dim3((uint32_t)units), dim3(kMeshBlock),
+                           0, st, spans, dists, counts, counts + units + 1, voff, ioff, verts, idx);
     }
     int rc = check_hip(hipGetLastError(), "mesh emit launch");
     if (rc || nverts == 0 || normals == CTH_NORMALS_DEFERRED) return rc;

@@ -133,6 +133,56 @@ def test_mesh_signed_zero_and_nan_corners(ctx, torch_cuda, res):
     assert pos_same.all()
 
 
+@pytest.mark.parametrize("res,leaves", [(32, 9), (64, 2)])
+def test_plane_units_dense_and_nan_corners(ctx, torch_cuda, res, leaves):
+    """The plane kernels on crafted corner fields in which nearly every cell
+    crosses and every corner has quads (their lists are full), with signed
+    zeros and NaNs of both signs: crossing words, counts, indices and positions
+    match the oracle's."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(res)
+    spans = octree_leaves(leaves, seed=3)
+    vals = np.array([-1.0, -0.25, -0.0, 0.0, 0.25, 1.0, np.nan, -np.nan], F32)
+    d = vals[rng.integers(0, len(vals), (leaves, (res + 1) ** 3))]
+    cb = torch.full((leaves, res ** 3 // 64), -1, dtype=torch.int64, device="cuda")
+    voff, ioff, v, ix = dev.mesh(ca.Sphere((0.0, 0.0, 0.0), 1.0, ctx=ctx), gpu(torch, spans), gpu(torch, d), res,
+                                 "deferred", cross=cb)
+    torch.cuda.synchronize()
+    assert (cb.cpu().numpy().view(np.uint64) == crossing_words(d, res)).all()
+    voff_o, ioff_o, v_o, ix_o = O.mesh_batch(O.sphere((0.0, 0.0, 0.0), 1.0), spans, res, dists=d)
+    assert_topology(voff.cpu().numpy().astype(np.uint64), ioff.cpu().numpy().astype(np.uint64),
+                    ix.cpu().numpy().view(np.uint32), voff_o, ioff_o, ix_o)
+    v = v.cpu().numpy()
+    assert (same_bits(v[:, :3], v_o[:, :3]) | (np.isnan(v[:, :3]) & np.isnan(v_o[:, :3]))).all()
+
+
+@pytest.mark.parametrize("res,leaves", [(2, 1), (2, 4095), (2, 4097), (2, 16384), (2, 16385), (32, 512), (32, 513)])
+def test_mesh_offsets_of_one_and_many_workgroups(ctx, torch_cuda, res, leaves):
+    """Offsets of up to 16,384 counts are scanned by one workgroup, 4,096 at a
+    time, of more by several: on both sides of each size they are the prefix
+    sums of the leaves' counts, which repeat a small batch's."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(leaves)
+    base = torch.from_numpy(rng.choice(np.array([-1.0, 1.0], F32), (7, (res + 1) ** 3))).cuda()
+    pick = torch.from_numpy(rng.integers(0, 7, leaves)).cuda()
+    spans = torch.tensor([[-1.0, -1.0, -1.0, 1.0, 1.0, 1.0]], device="cuda").repeat(leaves, 1)
+    shape = ca.Sphere((0.0, 0.0, 0.0), 1.0, ctx=ctx)
+    small = dev.mesh(shape, spans[:7].contiguous() if leaves >= 7 else spans[:1].repeat(7, 1), base, res, "deferred")
+    voff, ioff, v, ix = dev.mesh(shape, spans, base[pick].contiguous(), res, "deferred")
+    for off, small_off in ((voff, small[0]), (ioff, small[1])):
+        counts = (small_off[1:] - small_off[:-1])[pick]
+        assert int(off[0]) == 0
+        assert torch.equal(off[1:], torch.cumsum(counts, 0))
+    assert v.shape[0] == int(voff[-1]) and ix.shape[0] == int(ioff[-1])
+    at = int(voff[leaves - 1])
+    k = int(pick[leaves - 1])
+    assert torch.equal(v[at:], small[2][int(small[0][k]):int(small[0][k + 1])])
+
+
 def test_octree_leaf_mesh_parity(ctx, torch_cuda):
     """2,000 seeded depth-8 surface leaves of the octree workload (P8, 15 it,
     bailout 2, 8^3 cells per leaf)."""
