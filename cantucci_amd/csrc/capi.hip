@@ -112,7 +112,7 @@ int cth_ctx_create(int device, cth_ctx** out) {
     if (rc == CTH_OK) rc = check_hip(hipMalloc((void**)&c->counters, counter_words(COUNTER_RING) * sizeof(uint32_t)), "hipMalloc");
     if (rc == CTH_OK)
         rc = check_hip(hipMemset(c->counters, 0, counter_words(COUNTER_RING) * sizeof(uint32_t)), "hipMemset counters");
-    if (rc == CTH_OK) rc = check_hip(hipHostMalloc((void**)&c->pinned, 8 * sizeof(uint64_t)), "hipHostMalloc");
+    if (rc == CTH_OK) rc = check_hip(hipHostMalloc((void**)&c->pinned, kPinnedWords * sizeof(uint64_t)), "hipHostMalloc");
     if (rc == CTH_OK) rc = vjp_scratch_init(device);
     if (rc == CTH_OK) rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
     if (rc != CTH_OK) {

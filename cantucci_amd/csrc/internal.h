@@ -72,6 +72,8 @@ enum ScratchSlot {
     WS_SLOTS
 };
 
+constexpr size_t kPinnedWords = 32;
+
 struct Ctx {
     int device = 0;
     int num_cus = 0;
@@ -81,7 +83,7 @@ struct Ctx {
     uint32_t ring_pos = 0;
     void* ws[WS_SLOTS] = {};
     size_t ws_bytes[WS_SLOTS] = {};
-    uint64_t* pinned = nullptr;  // 8 host-pinned words for count read-backs
+    uint64_t* pinned = nullptr;  // kPinnedWords host-pinned words for count read-backs
     unsigned long long* stats = nullptr;  // work counters of the refill kernels (cth_ctx_count_work)
     // Slot `s` with at least `bytes` bytes (a larger buffer replaces the old
     // one after a device-wide wait, so no launch can still be using it).

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <vector>
 
 #include "internal.h"
@@ -104,9 +105,116 @@ __global__ void k_emit_leaves(const float* __restrict__ nodes, const uint32_t* _
     leaves[6 * (size_t)(incl[i] - 1u) + a] = nodes[6 * (size_t)i + a];
 }
 
+// The tree's top, all levels of at most kTopNodes nodes, in one workgroup: no
+// read-back and no launch between levels.  A level took 20-30 us whatever its
+// size (four or five launches and a wait for its split count).  Depth 2, 4, 5
+// and 7 of the octree: 82, 129, 158, 226 -> 27, 55, 98, 167 us.  Up to 512 nodes
+// gave 27, 69, 97, 166, up to 10,240 27, 55, 156, 257 (one CU is then slower
+// than a level of launches); real powers take 51 us more with 4,096.
+constexpr uint32_t kTopNodes = 2048;
+constexpr uint32_t kTopThreads = 1024;
+constexpr uint32_t kMaxDepth = 20;
+static_assert(2 + kMaxDepth + 1 <= kPinnedWords, "level counts fit");
+
+struct RefineTop {
+    float root[6];
+    float half_diag[kMaxDepth + 1];
+    uint32_t min_depth, max_depth;
+    float* nodes[2];   // level d in nodes[d & 1]
+    float* leaves;     // nullable
+    uint64_t cap;
+    uint64_t* out;     // host memory: next depth (max_depth + 1: done), its nodes (or the leaves), nodes per level
+};
+
+template <class Ev>
+__global__ __launch_bounds__(kTopThreads) void k_refine_top(RefineTop a, MandelUniform u) {
+    __shared__ uint32_t wsum[kTopThreads / 64];
+    const uint32_t wave = threadIdx.x >> 6;
+    if (threadIdx.x < 6) a.nodes[0][threadIdx.x] = a.root[threadIdx.x];
+    __syncthreads();
+    uint32_t n = 1, depth = 0;
+    for (;; ++depth) {
+        const float* cur = a.nodes[depth & 1u];
+        float* next = a.nodes[(depth & 1u) ^ 1u];
+        const bool last = depth == a.max_depth;
+        if (threadIdx.x == 0) a.out[2 + depth] = n;
+        uint32_t total = 0;
+        for (uint32_t base = 0; base < n; base += kTopThreads) {
+            const uint32_t i = base + threadIdx.x;
+            const bool valid = i < n;
+            bool split = valid;
+            if (depth >= a.min_depth) {
+                // One evaluation per lane, as in the work loops (every lane
+                // starts at once, so all reach the iteration cap together).
+                Ev ev;
+                float r = idle_start(ev, u);
+                if (valid) {
+                    float x, y, z, p;
+                    SrcCenters{cur, u.power}.get(i, x, y, z, p);
+                    ev.start(x, y, z, p, u);
+                    r = ev.mag();
+                }
+                uint64_t live_m = wave_mask(valid && !(r > u.bailout));
+                for (uint32_t k = 1; live_m != 0; ++k) {
+                    const bool cap = k == u.max_iters;
+                    const float rn = tick_full(ev, r, u, live_m, cap ? live_m : 0);
+                    live_m = cap ? 0 : live_m & ~wave_mask(rn > u.bailout);
+                }
+                const float d = ev.finish(r);
+                split = valid && ((d != d) || fabsf(d) < a.half_diag[depth]);
+            }
+            const uint64_t m = wave_mask(split);
+            if ((threadIdx.x & 63u) == 0) wsum[wave] = (uint32_t)__popcll(m);
+            __syncthreads();
+            uint32_t rank = total + lane_rank(m);
+            for (uint32_t w = 0; w < kTopThreads / 64; ++w) {
+                rank += w < wave ? wsum[w] : 0u;
+                total += wsum[w];
+            }
+            if (split && last) {
+                if (a.leaves && rank < a.cap) {
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) a.leaves[6 * (size_t)rank + k] = cur[6 * i + k];
+                }
+            } else if (split) {
+                float sp[6], ctr[3];
+#pragma unroll
+                for (int k = 0; k < 6; ++k) sp[k] = cur[6 * i + k];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) ctr[k] = sp[k] + (sp[3 + k] - sp[k]) * 0.5f;
+                float* out = next + 48 * (size_t)rank;
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c) {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const bool hi = (c >> (2 - k)) & 1u;
+                        out[6 * c + k] = hi ? ctr[k] : sp[k];
+                        out[6 * c + 3 + k] = hi ? sp[3 + k] : ctr[k];
+                    }
+                }
+            }
+            __syncthreads();  // wsum is rewritten; after the last round, the level's children are complete
+        }
+        if (last) {
+            if (threadIdx.x == 0) {
+                a.out[0] = depth + 1;
+                a.out[1] = total;
+            }
+            return;
+        }
+        n = 8 * total;
+        if (n == 0 || n > kTopNodes) break;
+    }
+    if (threadIdx.x == 0) {
+        a.out[0] = depth + 1;
+        a.out[1] = n;
+    }
+}
+
 static inline uint32_t cdiv32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-// Level-synchronous refinement.  Per level: the split flags (forced, sphere
+// Level-synchronous refinement: the top of the tree in one launch, then per
+// level the split flags (forced, sphere
 // closed form or a DE refill launch), an inclusive scan of the flags, one
 // 4-byte read-back of the split count into pinned host memory, and the
 // children.  Node, flag, offset and scan buffers are the context's scratch
@@ -121,14 +229,54 @@ int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_de
         if (rc) return rc;
     }
     const uint64_t kMaxNodes = 1ull << 28;
-    float* cur = nullptr;
-    int rc = c.scratch(WS_NODES_A, 6 * sizeof(float), (void**)&cur);
-    if (rc) return fail(rc, "refinement scratch allocation failed");
-    rc = check_hip(hipMemcpyAsync(cur, root, 6 * sizeof(float), hipMemcpyHostToDevice, st), "H2D root");
-    int slot = WS_NODES_A;
-    uint64_t n = 1;
     *nleaves = 0;
-    for (uint32_t depth = 0; depth <= max_depth && rc == CTH_OK; ++depth) {
+    uint32_t depth = 0;
+    uint64_t n = 1;
+    float* nodes[2] = {};
+    const size_t first = c.stats ? 1 : (size_t)8 * kTopNodes;
+    int rc = CTH_OK;
+    for (int k = 0; k < 2 && !rc; ++k) rc = c.scratch(WS_NODES_A + k, first * 6 * sizeof(float), (void**)&nodes[k]);
+    if (rc) return fail(rc, "refinement scratch allocation failed");
+    if (!c.stats) {
+        RefineTop top{};
+        std::copy(root, root + 6, top.root);
+        std::copy(half_diag, half_diag + max_depth + 1, top.half_diag);
+        top.min_depth = min_depth;
+        top.max_depth = max_depth;
+        top.nodes[0] = nodes[0];
+        top.nodes[1] = nodes[1];
+        top.leaves = leaves;
+        top.cap = cap;
+        top.out = c.pinned;
+        if (family == FAM_SPHERE) {
+            u.max_iters = 1;
+            u.bailout = 0.0f;
+            for (int a = 0; a < 3; ++a) u.center[a] = s.center[a];
+            u.radius = s.radius;
+            hipLaunchKernelGGL(k_refine_top<SphereEv>, dim3(1), dim3(kTopThreads), 0, st, top, u);
+        } else if (family == FAM_P8) {
+            with_p8(c.mode, [&](auto ev) {
+                hipLaunchKernelGGL(k_refine_top<decltype(ev)>, dim3(1), dim3(kTopThreads), 0, st, top, u);
+            });
+        } else {
+            hipLaunchKernelGGL(k_refine_top<TrigExact>, dim3(1), dim3(kTopThreads), 0, st, top, u);
+        }
+        rc = check_hip(hipGetLastError(), "refinement top launch");
+        int rs = check_hip(hipStreamSynchronize(st), "sync");
+        if (rc || rs) return rc ? rc : rs;
+        depth = (uint32_t)c.pinned[0];
+        n = c.pinned[1];
+        for (uint32_t d = 0; d < depth && level_counts; ++d) level_counts[d] = c.pinned[2 + d];
+        if (depth > max_depth) {
+            *nleaves = n;
+            return CTH_OK;
+        }
+    } else {  // counted work goes through the work loops
+        rc = check_hip(hipMemcpyAsync(nodes[0], root, 6 * sizeof(float), hipMemcpyHostToDevice, st), "H2D root");
+    }
+    int slot = WS_NODES_A + (int)(depth & 1u);
+    float* cur = nodes[depth & 1u];
+    for (; depth <= max_depth && rc == CTH_OK; ++depth) {
         if (level_counts) level_counts[depth] = n;
         if (n == 0) {
             for (uint32_t d2 = depth + 1; d2 <= max_depth && level_counts; ++d2) level_counts[d2] = 0;
