@@ -73,6 +73,7 @@ enum ScratchSlot {
 };
 
 constexpr size_t kPinnedWords = 32;
+constexpr size_t kHostStage = 4u << 20;  // pinned staging of a context's small host-pointer calls
 
 struct Ctx {
     int device = 0;
@@ -84,6 +85,7 @@ struct Ctx {
     void* ws[WS_SLOTS] = {};
     size_t ws_bytes[WS_SLOTS] = {};
     uint64_t* pinned = nullptr;  // kPinnedWords host-pinned words for count read-backs
+    char* host_stage = nullptr;  // kHostStage bytes, pinned
     unsigned long long* stats = nullptr;  // work counters of the refill kernels (cth_ctx_count_work)
     // Slot `s` with at least `bytes` bytes (a larger buffer replaces the old
     // one after a device-wide wait, so no launch can still be using it).

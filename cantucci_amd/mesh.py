@@ -27,6 +27,27 @@ class Timings:
     faces: int
 
 
+def _fill(leaves: int, resolution: int, run):
+    """The vertices and indices of run(verts, vert_cap, idx, idx_cap, &nverts,
+    &nidx).  The first buffers hold more than a surface through the leaves
+    usually has (their untouched pages cost nothing and are given back), so that
+    the leaves are sampled once; a mesh beyond them runs again."""
+    nv, ni = C.c_size_t(), C.c_size_t()
+    vcap = leaves * (6 * resolution * resolution + 64)
+    icap = 6 * vcap
+    while True:
+        verts = np.empty(vcap, VERTEX_DTYPE)
+        idx = np.empty(icap, np.uint32)
+        rc = run(verts.ctypes.data, vcap, idx.ctypes.data, icap, C.byref(nv), C.byref(ni))
+        if nv.value <= vcap and ni.value <= icap:
+            break
+        vcap, icap = nv.value, ni.value
+    check(rc)
+    verts.resize(nv.value, refcheck=False)
+    idx.resize(ni.value, refcheck=False)
+    return verts, idx
+
+
 @dataclass
 class MeshBuffer:
     vertices: np.ndarray  # VERTEX_DTYPE records
@@ -41,17 +62,9 @@ class MeshBuffer:
         sp.start[:] = [float(v) for v in span[0]]
         sp.end[:] = [float(v) for v in span[1]]
         mode = {"fd6": _lib.CTH_NORMALS_FD6, "tangent": _lib.CTH_NORMALS_TANGENT}[normals]
-        nv = C.c_size_t()
-        ni = C.c_size_t()
-        h = shape.ctx.handle
-        check(lib.cth_mesh_span(h, C.byref(shape.desc), C.byref(sp), resolution, mode, None, 0, None, 0,
-                                C.byref(nv), C.byref(ni)))
-        verts = np.empty(nv.value, VERTEX_DTYPE)
-        idx = np.empty(ni.value, np.uint32)
-        check(lib.cth_mesh_span(h, C.byref(shape.desc), C.byref(sp), resolution, mode,
-                                verts.ctypes.data if nv.value else None, nv.value,
-                                idx.ctypes.data if ni.value else None, ni.value, C.byref(nv), C.byref(ni)))
-        return cls(verts, idx), Timings(nv.value, ni.value // 6)
+        verts, idx = _fill(1, resolution, lambda *bufs: lib.cth_mesh_span(
+            shape.ctx.handle, C.byref(shape.desc), C.byref(sp), resolution, mode, *bufs))
+        return cls(verts, idx), Timings(len(verts), len(idx) // 6)
 
 
 def get_focii(shape: Shape, position, direction, fov: float, aspect: float, near_plane: float, far_plane: float,
@@ -157,18 +170,12 @@ class ShapeMesh:
         if not todo:
             return
         spans = np.array([[*self.leaves[i][0][0], *self.leaves[i][0][1]] for i in todo], np.float32)
-        h, n = self.shape.ctx.handle, len(todo)
-        nv, ni = C.c_size_t(), C.c_size_t()
-        check(lib.cth_mesh_spans(h, C.byref(self.shape.desc), spans.ctypes.data, n, self.RESOLUTION,
-                                 _lib.CTH_NORMALS_FD6, None, 0, None, 0, None, None, C.byref(nv), C.byref(ni)))
-        verts = np.empty(nv.value, VERTEX_DTYPE)
-        idx = np.empty(ni.value, np.uint32)
+        n = len(todo)
         voff = np.empty(n + 1, np.uint64)
         ioff = np.empty(n + 1, np.uint64)
-        check(lib.cth_mesh_spans(h, C.byref(self.shape.desc), spans.ctypes.data, n, self.RESOLUTION,
-                                 _lib.CTH_NORMALS_FD6, verts.ctypes.data if nv.value else None, nv.value,
-                                 idx.ctypes.data if ni.value else None, ni.value, voff.ctypes.data, ioff.ctypes.data,
-                                 C.byref(nv), C.byref(ni)))
+        verts, idx = _fill(n, self.RESOLUTION, lambda v, vcap, i, icap, nv, ni: lib.cth_mesh_spans(
+            self.shape.ctx.handle, C.byref(self.shape.desc), spans.ctypes.data, n, self.RESOLUTION,
+            _lib.CTH_NORMALS_FD6, v, vcap, i, icap, voff.ctypes.data, ioff.ctypes.data, nv, ni))
         for k, i in enumerate(todo):
             a, b, c, d = int(voff[k]), int(voff[k + 1]), int(ioff[k]), int(ioff[k + 1])
             self.leaves[i][1] = MeshBuffer(verts[a:b].copy(), idx[c:d].copy())

@@ -186,3 +186,29 @@ def test_create_spans_mirror_matches_oracle():
     for span in ([-1.2] * 3 + [1.2] * 3, [0.1, -0.7, 0.3, 0.35, -0.2, 0.9], [-1e-3, 2.0, -5.0, 1e-3, 2.5, 7.0]):
         got = np.array([[*a, *b] for a, b in create_spans((span[:3], span[3:]))], np.float32)
         assert (got.view(np.uint32) == O.create_spans(span).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("nv,ni", [(0, 0), (7, 12), (70, 420), (71, 12), (7, 421), (500, 3000)])
+def test_mesh_buffers_fit_or_run_again(nv, ni):
+    """The host meshing calls start from buffers of 6 res^2 + 64 vertices a leaf
+    (70 at resolution 1) and run again with the counts of a mesh beyond them;
+    other errors are raised."""
+    import cantucci_amd as ca
+    from cantucci_amd.mesh import VERTEX_DTYPE, _fill
+    calls = []
+
+    def run(v, vcap, i, icap, pnv, pni):
+        calls.append((vcap, icap))
+        pnv._obj.value, pni._obj.value = nv, ni
+        if vcap < nv or icap < ni:
+            return 1
+        C.memset(v, 1, nv * VERTEX_DTYPE.itemsize)
+        C.memset(i, 2, 4 * ni)
+        return 0
+
+    verts, idx = _fill(1, 1, run)
+    assert len(calls) == (1 if nv <= 70 and ni <= 420 else 2)
+    assert verts.shape == (nv,) and idx.shape == (ni,) and verts.dtype == VERTEX_DTYPE
+    assert (verts.view("u1") == 1).all() and (idx.view("u1") == 2).all()
+    with pytest.raises(ca.CthError):
+        _fill(1, 1, lambda *a: 1)

@@ -261,6 +261,28 @@ def test_shape_trait_host_queries(ctx):
     assert len(m.batch_min_distance_from(np.zeros((0, 3), F32))) == 0
 
 
+@pytest.mark.parametrize("n", [1, 65, 262144, 262145])
+def test_host_queries_direct_and_staged(ctx, torch_cuda, n):
+    """Host-pointer queries of up to 4 MiB of points and distances (262,144
+    points) run on pinned memory, larger ones on device staging: on both sides
+    the distances are the device entry point's, bit for bit, and a smaller call
+    after a larger one sees its own points."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    m = ca.Mandelbulb.classic(5, 2.0, ctx=ctx)
+    s = ca.Sphere((0.1, 0.2, 0.3), 0.7, ctx=ctx)
+    pts = np.random.default_rng(n).uniform(-1.2, 1.2, (n, 3)).astype(F32)
+    for part in (pts, pts[: n // 2 + 1][::-1].copy()):
+        want = dev.de_points(m, gpu(torch, part)).cpu().numpy()
+        got = m.batch_min_distance_from(part)
+        assert same_bits(got, want).all()
+        assert (m.batch_contains(part) == (want < 0)).all()
+        b = s.batch_bounded_distance_from(part)
+        ds = dev.de_points(s, gpu(torch, part)).cpu().numpy()
+        assert same_bits(b[:, 0], ds).all() and same_bits(b[:, 1], ds).all()
+
+
 def test_empty_and_invalid_device_calls(ctx, torch_cuda):
     import cantucci_amd as ca
     from cantucci_amd import device as dev
