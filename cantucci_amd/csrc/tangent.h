@@ -162,12 +162,12 @@ struct TrigTangentN : TrigExact {
         }
     }
 
-    __device__ __forceinline__ void body(float r, const MandelUniform&, bool live) {
+    __device__ __forceinline__ void body(float r, const MandelUniform& u, bool live) {
         const float zx = x, zy = y, zz = z;
         // The forward body's own terms: R = r^P, r^(P-1), theta, phi and the
         // sines/cosines of P theta, P phi.
         Terms t;
-        TrigExact::eval(r, t);
+        TrigExact::eval(r, u, t);
         float ir = 1.0f / r;
         float rho2 = zx * zx + zy * zy;
         float rho = __builtin_sqrtf(rho2);

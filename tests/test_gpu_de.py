@@ -176,6 +176,27 @@ def test_overflowing_magnitude_among_ordinary_points(ctx, torch_cuda, n):
     assert_de_parity(g, d)
 
 
+@pytest.mark.parametrize("P", [1, 2, 3, 4, 7, 16, 31, 63])
+def test_launch_power_and_point_powers_agree(ctx, torch_cuda, P):
+    """An integer power of the whole launch takes both of its powers of r from
+    one chain of squares, a per-point power its own ladders: the same distances
+    and normals, bit for bit (points around the surface, on the axes and at the
+    origin, NaN and overflowing coordinates)."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(P)
+    pts = np.concatenate([rng.uniform(-1.3, 1.3, (20001, 3)).astype(F32), edge_points(),
+                          np.array([[np.nan, 0.5, 0.5], [1e25, 1.0, 1.0], [1e-30, 0.0, 1e-30]], F32)])
+    p = gpu(torch, pts)
+    w = torch.full((len(pts),), float(P), device="cuda")
+    whole, each = ca.Mandelbulb(12, 2.0, P, ctx=ctx), ca.MandelbulbTrig(12, 2.0, float(P), ctx=ctx)
+    a, b = dev.de_points(whole, p), dev.de_points(each, p, w)
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    for x, y in zip(dev.normals(whole, p), dev.normals(each, p, w)):
+        assert (same_bits(x.cpu().numpy(), y.cpu().numpy()) | (torch.isnan(x) & torch.isnan(y)).cpu().numpy()).all()
+
+
 @pytest.mark.parametrize("P", [2, 3, 5, 9])
 def test_trig_integer_power(ctx, torch_cuda, P):
     """Mandelbulb<P != 8>: the trig map with ocml transcendentals.  Iteration
