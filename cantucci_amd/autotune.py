@@ -134,7 +134,8 @@ def _workloads(ctx):
 
     runs = {}
     m8 = Mandelbulb.classic(15, 2.0, ctx=ctx)
-    runs["grid"] = lambda: dev.de_grid(m8, (-1.5,) * 3, (1.5,) * 3, 64, 63.0)
+    # 64^3 makes no claims whatever the shape; 256^3 tells the shapes apart.
+    runs["grid"] = lambda: [dev.de_grid(m8, (-1.5,) * 3, (1.5,) * 3, n, n - 1.0) for n in (64, 256)]
     hd = wl.half_diagonals(3.0, 8)
     leaves, _ = dev.refine(m8, wl.OCTREE["root"], 2, 8, hd)
     out = torch.empty((leaves.shape[0], 729), device="cuda")
