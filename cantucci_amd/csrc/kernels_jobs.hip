@@ -3,9 +3,9 @@
 // The reference meshes each octree leaf as an independent thread-pool job
 // (src/mesh/mod.rs:129-161).  Here a batch of independent grid jobs -- each
 // with its own size n^3, power and iteration cap -- is one index space: the
-// jobs' grids are concatenated, every lane of the persistent lane-refill loop
-// finds its point's job by a binary search of the job offsets (kept in LDS),
-// and evaluates distance plus the forward-mode (tangent) gradient for the
+// jobs' grids are concatenated, every wave of the persistent lane-refill loop
+// finds its window's job by a search of the job offsets (kept in LDS), and its
+// lanes evaluate distance plus the forward-mode (tangent) gradient for the
 // unit normal.  A job's completion time is the latest wall-clock stamp of its
 // points' write-back (one atomicMax per wave and run of a job), so per-job
 // latency comes out of the same launch.  The launch (plus its small reset

@@ -908,9 +908,8 @@ __device__ __forceinline__ void put_fd_normal(float* v, const float t[7]) {
 //
 // A lane's vertex record (position, half-steps) and its tap distances are
 // only touched at the batched refill, so they live in the lane's own LDS
-// column rather than in 13 vector registers.  The kernel then fits in 72
-// VGPRs without spilling, and 7 waves share each SIMD (5 with the record in
-// registers); asking for 8 forces spills and is slower.
+// column rather than in 13 vector registers.  The kernel then fits in 54
+// VGPRs (64 for the trig map) without spilling, and 8 waves share each SIMD.
 template <class Ev, bool kCount = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_mesh_taps(float* __restrict__ verts,
                                                                                           MandelUniform u, WorkQueue q) {

@@ -2,11 +2,13 @@
 //
 // The reference refines a CPU octree one leaf at a time (ShapeMesh::update,
 // src/mesh/mod.rs:82-178, child spans from create_spans,
-// src/octree/mod.rs:315-329).  Here a whole level is one batch: the centre
-// distance of every node at depth d is evaluated by the lane-refill work loop,
-// the split flags are prefix-summed, and every split node writes its 8
-// children (create_spans order) into the next level's array.  Parents stay in
-// level order, so the level-d array equals the oracle's breadth-first order.
+// src/octree/mod.rs:315-329).  Here the top of the tree, levels of up to
+// kTopNodes nodes, is one workgroup's launch, and each level below it one
+// batch: the centre distance of every node at depth d is evaluated by the
+// lane-refill work loop, the split flags are prefix-summed, and every split
+// node writes its 8 children (create_spans order) into the next level's array.
+// Parents stay in level order, so the level-d array equals the oracle's
+// breadth-first order.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
