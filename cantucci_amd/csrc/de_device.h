@@ -220,9 +220,11 @@ struct MandelUniform {
 
 // How an evaluator's launches spread over the chip, in waves per CU
 // (make_queue): a small launch to `fill` waves, no launch beyond `most` (as
-// many as are resident, where later workgroups measured slower).
+// many as are resident, where later workgroups measured slower).  From 8/3
+// chunks for each of `fill` on, a launch grows to 3/8 wave a chunk, at most
+// `grow` waves per CU (0: not before four chunks a wave).
 struct WaveSpread {
-    uint32_t fill, most;
+    uint32_t fill, most, grow = 0;
 };
 
 // ---------------------------------------------------------------------------
@@ -480,7 +482,7 @@ struct P8Contract : P8Exact {
 // ---------------------------------------------------------------------------
 struct TrigExact {
     static constexpr int kWavesPerSimd = 1;  // no constraint (64 VGPRs would spill)
-    static constexpr WaveSpread kSpread{16, ~0u};
+    static constexpr WaveSpread kSpread{16, ~0u, 24};
     static constexpr bool kLastDr = true;
     float px, py, pz, x, y, z, dr, P;
     int Pi;       // integer power of the powi ladder (when `ladder`)

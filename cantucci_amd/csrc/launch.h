@@ -45,9 +45,13 @@ inline bool foreign_capture(hipStream_t st) {
 // A launch's workgroups and chunks.  Up to a chunk of `least` indices (64 or
 // fewer) for each of spread.fill waves per CU a launch is spread as thinly as possible; from four
 // chunks per wave on it grows to the launch shape's (and spread.most) waves.
-// In between it stays at `fill`: a lane that takes a second point while its
-// wave's slowest is still iterating costs little, more waves on a SIMD cost
-// their share of its issue slots.
+// In between it stays at `fill` up to 8/3 chunks a wave: a lane that takes a
+// second point while its wave's slowest is still iterating costs little, more
+// waves on a SIMD cost their share of its issue slots.  Then evaluators with
+// spread.grow grow to that: 500,000 / 600,000 / 800,000 tangent normals at power
+// 5 59 / 73 / 87 -> 46 / 56 / 67 us (growing from four chunks on), 0.8 / 1 / 1.2 M
+// points 34.8 / 44.0 / 51.0 -> 31.5 / 36.2 / 44.8; 20 or 24 waves per CU from the
+// start cost 300,000 points 9 %.
 //
 // Measured on the default shapes, us per launch (in parentheses with the
 // workgroup count taken from the configured 256-index chunk): 64^3 grid 10.5
@@ -77,7 +81,11 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     }
     const uint64_t cus = (uint64_t)c.num_cus, waves_per_block = (uint64_t)ls.block / 64u;
     const uint64_t small = ((uint64_t)total + least - 1) / least;
-    uint64_t waves = std::max(std::min(small, cus * spread.fill), std::min(small / 4u, cus * spread.most));
+    // Whole workgroups for each CU (16.02 waves per CU cost 700,000 points at
+    // power 5 4 %), the nearest to 3/8 wave for each chunk.
+    const uint64_t per_cu = (small * 3u / 8u + cus * waves_per_block / 2u) / (cus * waves_per_block) * waves_per_block;
+    uint64_t waves = std::max({std::min(small, cus * spread.fill), cus * std::min<uint64_t>(per_cu, spread.grow),
+                               std::min(small / 4u, cus * spread.most)});
     blocks = (uint32_t)std::max<uint64_t>(
         1, std::min(cus * (uint64_t)ls.blocks_per_cu, (waves + waves_per_block - 1) / waves_per_block));
     WorkQueue q;

@@ -31,7 +31,7 @@ __device__ __forceinline__ float grad_final(float r, float dr, float rq, float d
 // ---------------------------------------------------------------------------
 struct P8Tangent : P8Exact {
     static constexpr int kWavesPerSimd = 1;  // the tangent state does not fit 64 VGPRs
-    static constexpr WaveSpread kSpread{8, 16};
+    static constexpr WaveSpread kSpread{8, 16, 16};
     static constexpr bool kLastDr = false;   // the work loops run its last body in full
     static constexpr bool kCarriedGuard = false;  // its body() also carries the tangents
     float T[3][3];    // dz/dp
@@ -141,7 +141,7 @@ template <int NQ>
 struct TrigTangentN : TrigExact {
     static_assert(NQ == 3 || NQ == 4, "3 point columns, optionally the power");
     static constexpr int kWavesPerSimd = 1;
-    static constexpr WaveSpread kSpread{8, 16};
+    static constexpr WaveSpread kSpread{8, 16, 16};
     static constexpr bool kLastDr = false;  // the work loops run its last body in full
     float T[3][NQ];
     float tdr[NQ];

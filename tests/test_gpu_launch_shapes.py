@@ -145,3 +145,35 @@ def test_large_default_launches_claim(torch_cuda, what, off):
     finally:
         auto.close()
         static.close()
+
+
+@pytest.mark.parametrize("waves", [16, 17, 18, 20, 24, 25])
+@pytest.mark.parametrize("what", ["points", "normals"])
+def test_middle_launches_grow(torch_cuda, what, waves):
+    """Launches of the trig map and the tangents grow by whole workgroups per CU
+    from 8/3 chunks of 64 for each of their first waves on: point counts that
+    give 3/8 wave a chunk on both sides of each step, one point short of and
+    beyond a chunk, against a dense launch shape given by the caller."""
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    auto, given = ca.Context(0, "parity"), ca.Context(0, "parity")
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    w = waves if what == "points" else waves - 8
+    try:
+        for f in (_lib.CTH_KERNEL_DE, _lib.CTH_KERNEL_ADJOINT):
+            given.set_launch(f, 256, 4, 64, 64, dynamic=1)
+        for off in (-1, 1):
+            n = 64 * cus * w * 8 // 3 + off
+            gen = torch.Generator(device="cuda").manual_seed(waves)
+            pts = torch.rand((n, 3), device="cuda", generator=gen) * 2.4 - 1.2
+            outs = []
+            for c in (auto, given):
+                shape = ca.Mandelbulb(5, 2.0, 3, ctx=c)
+                outs.append(dev.normals(shape, pts) if what == "normals" else (dev.de_points(shape, pts),))
+            for a, b in zip(*outs):
+                assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    finally:
+        auto.close()
+        given.close()
