@@ -274,13 +274,23 @@ struct P8Exact {
         in_range = u.bailout <= 16.0f && wave_mask(!(w2 + z2 <= 0x1p126f)) == 0;
         guard();
     }
+    // The same after a body on the scaled sequences.  Near the z axis (w between
+    // about 2^-18.6 and 2^-16 |z|) w8 is subnormal, num / w8 overflows and the
+    // body ends at infinity, as the reference's does: that point bails and is
+    // held too.  Only wave ticks that are slow anyway make this test.
+    __device__ __forceinline__ void range_after_scaled(bool live, float ax, float ay, float az) {
+        in_range = in_range && wave_mask(live && !((ax * ax + ay * ay) + az * az <= 0x1p126f)) == 0;
+    }
     // mag() after a loop body, with the wave test of the next body made here
-    // and also used for this square root: m = w2 + z2 >= w2 >= 2^-15, and a
-    // point that was live before the body (r <= bailout <= 16) has every
-    // coordinate of its rotation below 2^46 (each is a degree-8 form in x, y,
-    // z whose denominator w8 cancels against the numerator's w^8 factor), so
-    // m < 2^94: the range of sqrt_rn_unscaled.  Lanes without a live point
-    // may be outside it; their results are dropped.
+    // and also used for this square root: m = w2 + z2 >= w2 >= 2^-15, and
+    // m <= 2^126 for a point that ran the body on the scaled sequences
+    // (range_after_scaled).  One that ran it unscaled was live (r <= bailout <=
+    // 16) with w2 >= 2^-15, so that w8 is normal and every coordinate of its
+    // rotation below 2^46 (each is a degree-8 form in x, y, z whose denominator
+    // w8 cancels against the numerator's w^8 factor), m < 2^94.  A held point
+    // has the magnitude it bailed with, which passed one of these tests or
+    // guard_start's.  So m is in the range of sqrt_rn_unscaled; lanes that never
+    // took a point start inside it.
     __device__ __forceinline__ float mag_tick() {
         x2 = x * x;
         y2 = y * y;
@@ -361,6 +371,7 @@ struct P8Exact {
                     nz = r8 * cosf(th * 8.0f);
                 }
             }
+            if constexpr (kMasked) range_after_scaled(live, nx + px, ny + py, nz + pz);
         }
         if (live) {
             if constexpr (kMasked) asm volatile("");
@@ -465,6 +476,7 @@ struct P8Contract : P8Exact {
                     nz = r8 * cosf(th * 8.0f);
                 }
             }
+            if constexpr (kMasked) range_after_scaled(live, nx + px, ny + py, nz + pz);
         }
         if (live) {
             if constexpr (kMasked) asm volatile("");

@@ -176,6 +176,87 @@ def test_overflowing_magnitude_among_ordinary_points(ctx, torch_cuda, n):
     assert_de_parity(g, d)
 
 
+def near_axis_points(n, seed):
+    """Points about 2^-17 off the z axis: the power map's num / w^8 overflows in
+    their first body, which ends at infinity (at azimuths where neither degree-8
+    form in x and y cancels to 0, which would give NaN)."""
+    rng = np.random.default_rng(seed)
+    w, phi = rng.uniform(6e-6, 1.15e-5, n), rng.uniform(0.02, 0.1, n) + rng.integers(0, 4, n) * (np.pi / 2)
+    z = rng.uniform(1.0, 1.5, n) * rng.choice([-1.0, 1.0], n)
+    return np.stack([w * np.cos(phi), w * np.sin(phi), z], 1).astype(F32)
+
+
+@pytest.mark.parametrize("mode", ["parity", "contract"])
+@pytest.mark.parametrize("n", [64, 5000])
+def test_bodies_that_overflow_near_the_axis(torch_cuda, mode, n):
+    """A point near the z axis goes to infinity in its first body, among points
+    away from the axis (their bodies take the short square root and division):
+    it bails there with distance +inf, whatever its wave's other points are."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    pts = np.random.default_rng(n).uniform(0.3, 0.6, (n, 3)).astype(F32)
+    near = np.arange(3, n, 29)
+    pts[near] = near_axis_points(len(near), n)
+    c = ca.Context(0, mode)
+    try:
+        shape = ca.Mandelbulb.classic(15, 2.0, ctx=c)
+        d, it = dev.de_points(shape, gpu(torch, pts), with_iters=True)
+        r, dr, _ = dev.de_state(shape, gpu(torch, pts))
+        torch.cuda.synchronize()
+    finally:
+        c.close()
+    d, it, r, dr = (t.cpu().numpy() for t in (d, it, r, dr))
+    d_o, it_o, r_o, dr_o = O.de_points(O.mandelbulb(15, 2.0), pts)
+    assert np.isposinf(d_o[near]).all() and (it_o[near] == 1).all()
+    assert np.isposinf(d[near]).all() and np.isposinf(r[near]).all() and (it[near] == 1).all()
+    if mode == "parity":
+        assert (it == it_o).all() and same_bits(r, r_o).all() and same_bits(dr, dr_o).all()
+        assert_de_parity(d, d_o)
+
+
+def test_spans_and_taps_near_the_axis(ctx, torch_cuda):
+    """The same in span sampling (a column of corners near the axis) and in the
+    vertex taps (vertices near the axis, and vertices whose +x tap is)."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    shape, ref = ca.Mandelbulb.classic(15, 2.0, ctx=ctx), O.mandelbulb(15, 2.0)
+    h = 0.0625
+    mid = np.array([[8e-6, 3e-6, 1.0], [-6e-6, 2e-6, -1.1], [0.4, 0.4, 0.3]])
+    spans = np.concatenate([mid - h, mid + h], 1).astype(F32)
+    d, cb = dev.sample_spans(shape, gpu(torch, spans), 8)
+    d_o, cb_o, _ = O.sample_spans(ref, spans, 8)
+    assert np.isposinf(d_o[:2]).sum() >= 10
+    d = d.cpu().numpy()
+    assert (np.isposinf(d) == np.isposinf(d_o)).all()
+    assert_de_parity(d.ravel(), d_o.ravel())
+    assert (cb.cpu().numpy().view(np.uint64) == cb_o).all()
+
+    n, delta = 3000, F32(0.015625)
+    verts = np.zeros((n, 7), F32)
+    verts[:, :3] = np.random.default_rng(7).uniform(0.3, 0.6, (n, 3))
+    verts[:, 3:6] = delta
+    near, tap = np.arange(6, n, 42), np.arange(17, n, 54)
+    verts[near, :3] = near_axis_points(len(near), 1)
+    verts[tap, :3] = near_axis_points(len(tap), 2)
+    verts[tap, 0] -= delta
+    p = verts[:, None, :3].repeat(7, 1)
+    for a in range(3):
+        p[:, 1 + 2 * a, a] += delta
+        p[:, 2 + 2 * a, a] -= delta
+    t = O.de_points(ref, p.reshape(-1, 3))[0].reshape(n, 7)
+    assert np.isposinf(t[near, 0]).all() and np.isposinf(t[tap, 1]).all()
+    with np.errstate(invalid="ignore"):
+        g = t[:, 1::2] - t[:, 2::2]
+        m = np.sqrt(g[:, 0] * g[:, 0] + g[:, 1] * g[:, 1] + g[:, 2] * g[:, 2])
+        nrm = g * (F32(1.0) / m)[:, None]
+    v = dev.mesh_vertices(shape, gpu(torch, verts)).cpu().numpy()
+    assert (np.isposinf(v[:, 6]) == np.isposinf(t[:, 0])).all()
+    assert_de_parity(v[:, 6], t[:, 0])
+    assert (np.isnan(v[:, 3:6]) == np.isnan(nrm)).all()
+
+
 @pytest.mark.parametrize("P", [1, 2, 3, 4, 7, 16, 31, 63])
 def test_launch_power_and_point_powers_agree(ctx, torch_cuda, P):
     """An integer power of the whole launch takes both of its powers of r from
