@@ -591,8 +591,7 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
         // `resident` need not spread evenly over a CU's four SIMDs: waves claim
         // their chunks where there are enough to even that out (4 M points at 15
         // iterations 558 -> 469 us, 300,000 points 65 -> 73).
-        // Not in a capture that owns no counters (replays would share the ring's).
-        ls.dynamic = n / 256u >= (uint32_t)c.num_cus * spread.fill && !foreign_capture(st);
+        ls.dynamic = n / 256u >= (uint32_t)c.num_cus * spread.fill;
         ls.given = true;
         SrcPoints src{pts, powers, s.power};
         AdjOut out{grad_d, grad_p, grad_power, normals, grad_z0, grad_c};

@@ -34,11 +34,14 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
     if (iters) iters[i] = 0;
 }
 
-// Whether `st` is being captured into a graph that owns no counter entries: its
-// replays would take the ring's entries of launches in flight.
+// Whether `st` is being captured into a graph that owns no counter entries.  Its
+// replays would claim from the entry of the context's ring that the capture took,
+// beside the launches in flight that the ring has come round to, and from freed
+// memory once the context is gone: no launch claims there, whatever its shape.
+// (The null stream cannot be captured.)
 inline bool foreign_capture(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return capture_pool().stream != st && hipStreamIsCapturing(st, &cs) == hipSuccess &&
+    return st && capture_pool().stream != st && hipStreamIsCapturing(st, &cs) == hipSuccess &&
            cs != hipStreamCaptureStatusNone;
 }
 
@@ -73,10 +76,11 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     constexpr uint32_t kLeastClaim = 128;
     const uint64_t resident = (uint64_t)c.num_cus * std::min(32u, spread.most);
     uint64_t lowest = 64;
-    if (!ls.given && !ls.dynamic && total >= 4u * kLeastClaim * resident && !foreign_capture(st)) {
+    const bool large = !ls.given && !ls.dynamic && total >= 4u * kLeastClaim * resident;
+    const bool claims = (ls.dynamic || large) && !foreign_capture(st);
+    if (large && claims) {
         ls.blocks_per_cu = 8 * (256 / ls.block);
         ls.chunk = 1024;
-        ls.dynamic = 1;
         lowest = kLeastClaim;
     }
     const uint64_t cus = (uint64_t)c.num_cus, waves_per_block = (uint64_t)ls.block / 64u;
@@ -99,7 +103,7 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     q.chunks = (uint32_t)(((uint64_t)total + q.chunk - 1) / q.chunk);
     q.refill_min = ls.refill_min < 1 ? 1 : (ls.refill_min > 64 ? 64 : ls.refill_min);
     // Only chunks beyond every wave's first are claimed.
-    q.dynamic = ls.dynamic && q.chunks > q.waves ? 1u : 0u;
+    q.dynamic = claims && q.chunks > q.waves ? 1u : 0u;
     // Static rows rotate from four rows on (128^3 grid 47 -> 42 us, 24 mixed
     // jobs 2.27 -> 1.85 ms).  With fewer, the waves of the partial last row
     // decide, and the first waves, which start first, are the best ones for it

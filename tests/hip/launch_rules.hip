@@ -1,0 +1,88 @@
+// The host rules of a launch (make_queue and the counter entries it takes),
+// checked on the CPU: no kernel is compiled or launched, and the capture state
+// of a stream is the test's own.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <vector>
+
+static bool g_capturing = false;
+static hipError_t test_stream_is_capturing(hipStream_t, hipStreamCaptureStatus* s) {
+    *s = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+#define hipStreamIsCapturing test_stream_is_capturing
+#include "launch.h"
+
+namespace cth {
+CapturePool& capture_pool() {
+    static CapturePool p;
+    return p;
+}
+}  // namespace cth
+using namespace cth;
+
+static int g_failed = 0;
+#define CHECK(x)                                                                                       \
+    do {                                                                                               \
+        if (!(x)) {                                                                                    \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);                                        \
+            ++g_failed;                                                                                \
+        }                                                                                              \
+    } while (0)
+
+static Ctx make_ctx(std::vector<uint32_t>& ring) {
+    ring.assign(counter_words(COUNTER_RING), 0);
+    Ctx c;
+    c.num_cus = 256;
+    c.counters = ring.data();
+    return c;
+}
+static const hipStream_t kStream = (hipStream_t)0x1000, kOther = (hipStream_t)0x2000;
+
+static WorkQueue queue(Ctx& c, uint32_t total, const LaunchShape& ls, hipStream_t st,
+                       WaveSpread spread = P8Exact::kSpread) {
+    uint32_t blocks = 0;
+    return make_queue(c, total, ls, spread, blocks, st);
+}
+
+// A launch into a graph that owns no counters takes no entry of the ring and
+// claims nothing: default static shapes, default claiming ones and shapes set
+// by the caller.  One recorded through the pool takes the graph's own entries.
+static void captures() {
+    std::vector<uint32_t> ring, own(counter_words(GRAPH_ENTRIES), 0);
+    Ctx c = make_ctx(ring);
+    const LaunchShape given{256, 8, 256, 32, 1, true};
+    const LaunchShape shapes[] = {c.shape_de,  c.shape_spans, c.shape_trace, c.shape_adj,
+                                  c.shape_jobs, c.shape_mesh, given};
+    for (const LaunchShape& ls : shapes) {
+        for (uint32_t total : {1u, 100000u, 20000000u}) {
+            for (hipStream_t st : {kStream, (hipStream_t) nullptr}) {
+                g_capturing = false;
+                const WorkQueue eager = queue(c, total, ls, st);
+                CHECK(eager.dynamic == (eager.ctr != nullptr));
+                if (total == 20000000u) CHECK(eager.dynamic);
+                if (total == 1u) CHECK(!eager.dynamic);
+            }
+            g_capturing = true;
+            const uint32_t pos = c.ring_pos;
+            const WorkQueue q = queue(c, total, ls, kStream);
+            CHECK(!q.dynamic && !q.ctr && c.ring_pos == pos);
+            CHECK((uint64_t)q.chunk * q.chunks >= total && (uint64_t)q.chunk * (q.chunks - 1) < total);
+            capture_pool().stream = kStream;
+            capture_pool().counters = own.data();
+            const WorkQueue g = queue(c, total, ls, kStream), f = queue(c, total, ls, kOther);
+            CHECK(!g.dynamic || (g.ctr >= own.data() && g.ctr < own.data() + own.size()));
+            if (total == 20000000u) CHECK(g.dynamic);
+            CHECK(!f.dynamic && c.ring_pos == pos);  // a stream forked off the captured one
+            capture_pool() = CapturePool{};
+            g_capturing = false;
+        }
+    }
+}
+
+int main() {
+    captures();
+    std::printf(g_failed ? "%d checks failed\n" : "launch rules ok\n", g_failed);
+    return g_failed ? 1 : 0;
+}

@@ -177,3 +177,77 @@ def test_middle_launches_grow(torch_cuda, what, waves):
     finally:
         auto.close()
         given.close()
+
+
+def test_captures_without_counters(torch_cuda):
+    """Contexts whose shapes claim (as recorded ones do), captured by torch, whose
+    graphs have no counters: replays beside claiming launches on another stream
+    give the eager outputs, and still do once the context is gone (the launches
+    hold nothing of it)."""
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    from cantucci_amd import workloads as wl
+    torch = torch_cuda
+    c, other = ca.Context(0, "parity"), ca.Context(0, "parity")
+    for f in (_lib.CTH_KERNEL_DE, _lib.CTH_KERNEL_TRACE, _lib.CTH_KERNEL_ADJOINT, _lib.CTH_KERNEL_JOBS):
+        c.set_launch(f, 256, 2, 256, 16, dynamic=1)
+    m = ca.Mandelbulb.classic(6, 2.0, ctx=c)
+    n = 1 << 20
+    pts = torch.rand((n, 3), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)) * 2.4 - 1.2
+    spans = torch.cat([pts[:2000] - 0.05, pts[:2000] + 0.05], 1).contiguous()
+    cams = torch.from_numpy(wl.orbit_poses(1, 2, 1024, 512)).cuda()
+    js = dev.JobSet(c, _lib.CTH_SHAPE_MANDELBULB, 2.0, [dict(n=40 + k, power=8.0, max_iters=5 + k) for k in range(6)])
+    nrm, d = torch.empty((n, 3), device="cuda"), torch.empty(n, device="cuda")
+    sd = torch.empty((2000, 729), device="cuda")
+    depth, steps = torch.empty((1, 512, 1024), device="cuda"), torch.empty((1, 512, 1024), dtype=torch.int32,
+                                                                           device="cuda")
+    jd, jn = torch.empty(js.total, device="cuda"), torch.empty((js.total, 3), device="cuda")
+    done = torch.zeros(js.njobs, dtype=torch.int64, device="cuda")
+    start = torch.zeros(1, dtype=torch.int64, device="cuda")
+    bufs = (nrm, d, sd, depth, steps, jd, jn)
+
+    def work(shape):
+        dev.normals(shape, pts, out=nrm, d=d)
+        dev.sample_spans(shape, spans, 8, with_cross=False, out=sd)
+        dev.render_depth(shape, cams, 1024, 512, max_steps=12, depth=depth, steps=steps)
+        js.run(jd, jn, done, start)
+        return dev.de_points(shape, pts), dev.de_grid(shape, (-1.2,) * 3, (1.2,) * 3, 96, 95.0)
+
+    def result(f, outs):
+        for b in bufs + outs:
+            b.fill_(-1)
+        f()
+        torch.cuda.synchronize()
+        return [b.view(torch.int32).clone() for b in bufs + outs]
+
+    try:
+        outs = work(m)
+        torch.cuda.synchronize()
+        want = [b.view(torch.int32).clone() for b in bufs + outs]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            gouts = work(m)
+        side = torch.cuda.Stream()
+        o2 = ca.Mandelbulb.classic(6, 2.0, ctx=c)
+        e = torch.empty_like(nrm)
+
+        def beside():
+            g.replay()
+            with torch.cuda.stream(side):
+                for _ in range(8):
+                    dev.normals(o2, pts, out=e)
+
+        for f in (g.replay, beside, beside):
+            for a, b in zip(result(f, gouts), want):
+                assert torch.equal(a, b)
+        assert torch.equal(e.view(torch.int32), want[0])
+        c.close()
+        dev.normals(ca.Mandelbulb.classic(4, 2.0, ctx=other), pts)  # claims from its own ring
+        for a, b in zip(result(g.replay, gouts), want):
+            assert torch.equal(a, b)
+    finally:
+        torch.cuda.synchronize()
+        js.close()
+        c.close()
+        other.close()
