@@ -61,6 +61,16 @@ static int check_shape(const cth_shape* s) {
     return resolve_mandel(*s, u, fam);
 }
 
+int Ctx::emit_scratch(size_t bytes, uint64_t** out, hipStream_t st) {
+    if (scratch(WS_EMIT, bytes, (void**)out)) return fail(CTH_E_NOMEM, "mesh scratch allocation failed");
+    return emit_pending ? check_hip(hipStreamWaitEvent(st, emit_event, 0), "hipStreamWaitEvent") : CTH_OK;
+}
+
+int Ctx::emit_done(hipStream_t st) {
+    emit_pending = true;
+    return check_hip(hipEventRecord(emit_event, st), "hipEventRecord");
+}
+
 // `_dev` entry points run on the caller's stream; NULL is HIP's default
 // (null) stream, as everywhere in HIP.  The context's own stream serves the
 // host-pointer entry points.
@@ -169,6 +179,8 @@ int cth_ctx_create(int device, cth_ctx** out) {
         rc = check_hip(hipMemset(c->counters, 0, counter_words(COUNTER_RING) * sizeof(uint32_t)), "hipMemset counters");
     if (rc == CTH_OK) rc = check_hip(hipHostMalloc((void**)&c->pinned, kPinnedWords * sizeof(uint64_t)), "hipHostMalloc");
     if (rc == CTH_OK) rc = check_hip(hipHostMalloc((void**)&c->host_stage, kHostStage), "hipHostMalloc");
+    if (rc == CTH_OK)
+        rc = check_hip(hipEventCreateWithFlags(&c->emit_event, hipEventDisableTiming), "hipEventCreate");
     if (rc == CTH_OK) rc = vjp_scratch_init(device);
     if (rc == CTH_OK) rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
     if (rc != CTH_OK) {
@@ -188,6 +200,7 @@ void cth_ctx_destroy(cth_ctx* c) {
         if (p) (void)hipFree(p);
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->host_stage) (void)hipHostFree(c->host_stage);
+    if (c->emit_event) (void)hipEventDestroy(c->emit_event);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }

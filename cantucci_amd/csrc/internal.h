@@ -58,7 +58,8 @@ struct LaunchShape {
 
 // Device scratch slots of a context, grown on demand and kept until the
 // context is destroyed (calls on one context never overlap, and the users
-// below finish with a stream synchronisation).
+// below finish with a stream synchronisation; WS_EMIT goes through
+// emit_scratch).
 enum ScratchSlot {
     WS_NODES_A = 0,
     WS_NODES_B,
@@ -66,6 +67,7 @@ enum ScratchSlot {
     WS_OFFS,
     WS_SCAN,
     WS_COUNTS,
+    WS_EMIT,
     WS_UOFF,
     WS_HOST_IN,   // staging of the host-buffer entry points
     WS_HOST_OUT,
@@ -107,6 +109,13 @@ struct Ctx {
         *out = ws[s];
         return CTH_OK;
     }
+    // WS_EMIT for an emission on `st`.  Emissions return while they still read
+    // their counts, so each ends with emit_done(), and the next, which may be on
+    // another stream, waits for that.
+    int emit_scratch(size_t bytes, uint64_t** out, hipStream_t st);
+    int emit_done(hipStream_t st);
+    hipEvent_t emit_event = nullptr;
+    bool emit_pending = false;  // emit_event was recorded
     LaunchShape shape_de;
     LaunchShape shape_spans{256, 8, 1024, 32, 1};
     // The counter entry of a launch on stream `st`: from the capturing graph's
@@ -138,6 +147,11 @@ struct Ctx {
 // Status helpers (capi.hip)
 int fail(int code, const std::string& msg);
 int check_hip(hipError_t e, const char* what);
+
+inline bool is_capturing(hipStream_t st) {  // the null stream cannot be captured
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
 
 // Resolve a shape descriptor into kernel uniforms.  Returns CTH_OK or an error.
 int resolve_mandel(const cth_shape& s, MandelUniform& u, int& family);

@@ -1087,18 +1087,18 @@ static int scan_pair(Ctx& c, uint64_t* counts, size_t cnt, uint64_t* voff, uint6
     return rc;
 }
 
-// Plane-unit counts in the context's scratch: *counts holds units + 1 vertex
-// counts followed by units + 1 index counts.
-static int plane_counts(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint64_t* cross, uint64_t** counts,
+// Plane-unit counts: units + 1 vertex counts followed by units + 1 index counts.
+static int plane_counts(const float* dists, uint32_t nleaves, uint32_t res, uint64_t* cross, uint64_t* counts,
                         hipStream_t st) {
     const size_t units = (size_t)nleaves * res;
-    if (units >= (size_t(1) << 31)) return fail(CTH_E_INVALID, "more than 2^31 mesh plane units");
-    const size_t cnt = units + 1;
-    if (c.scratch(WS_COUNTS, 2 * cnt * sizeof(uint64_t), (void**)counts))
-        return fail(CTH_E_NOMEM, "mesh scratch allocation failed");
     hipLaunchKernelGGL((res == 64 ? k_mesh_count_p<6> : k_mesh_count_p<5>), dim3((uint32_t)units), dim3(kMeshBlock), 0,
-                       st, dists, (uint32_t)units, *counts, *counts + cnt, cross);
+                       st, dists, (uint32_t)units, counts, counts + units + 1, cross);
     return check_hip(hipGetLastError(), "mesh plane count launch");
+}
+
+static int check_units(uint32_t nleaves, uint32_t res) {
+    if ((uint64_t)nleaves * res >= (1ull << 31)) return fail(CTH_E_INVALID, "more than 2^31 mesh plane units");
+    return CTH_OK;
 }
 
 int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint64_t* voff, uint64_t* ioff,
@@ -1112,15 +1112,17 @@ int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint6
         if (!rc) rc = check_hip(hipStreamSynchronize(st), "mesh count sync");
         return rc;
     }
+    if (res > 16) {
+        if (int rc = check_units(nleaves, res)) return rc;
+    }
     int rc = CTH_OK;
     const uint32_t lg = res <= 16 ? 0u : res == 32 ? 5u : 6u;  // units per leaf
-    const size_t units = (size_t)nleaves << lg;
+    const size_t units = (size_t)nleaves << lg, cnt = units + 1;
     uint64_t* counts = nullptr;
+    if (c.scratch(WS_COUNTS, 2 * cnt * sizeof(uint64_t), (void**)&counts))
+        return fail(CTH_E_NOMEM, "mesh count scratch allocation failed");
     if (res <= 16) {
         // wave per leaf: the counts are per leaf already
-        const size_t cnt = units + 1;
-        if (c.scratch(WS_COUNTS, 2 * cnt * sizeof(uint64_t), (void**)&counts))
-            return fail(CTH_E_NOMEM, "mesh count scratch allocation failed");
         switch (res) {
             case 1: LAUNCH_COUNT_W(1); break;
             case 2: LAUNCH_COUNT_W(2); break;
@@ -1130,7 +1132,7 @@ int mesh_count(Ctx& c, const float* dists, uint32_t nleaves, uint32_t res, uint6
         }
         rc = check_hip(hipGetLastError(), "mesh count launch");
     } else {
-        rc = plane_counts(c, dists, nleaves, res, cross, &counts, st);
+        rc = plane_counts(dists, nleaves, res, cross, counts, st);
     }
     if (!rc && units <= kScanOne) {
         hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, counts, counts + units + 1, (uint32_t)units, lg,
@@ -1173,6 +1175,8 @@ int mesh_emit(Ctx& c, const cth_shape& s, const float* spans, const float* dists
     if (normals == CTH_NORMALS_TANGENT && s.kind == CTH_SHAPE_SPHERE)
         return fail(CTH_E_UNSUPPORTED, "tangent normals need a Mandelbulb kind");
     if (nleaves == 0) return CTH_OK;
+    int rc = CTH_OK;
+    bool captured = false;
     if (res <= 16) {
         switch (res) {
             case 1: LAUNCH_EMIT_W(1); break;
@@ -1181,17 +1185,31 @@ int mesh_emit(Ctx& c, const cth_shape& s, const float* spans, const float* dists
             case 8: LAUNCH_EMIT_W(8); break;
             default: LAUNCH_EMIT_W(16); break;
         }
+        rc = check_hip(hipGetLastError(), "mesh emit launch");
     } else {
-        // the plane units' counts (recounted: a count call leaves only the leaves' offsets)
+        // The plane units' counts (recounted: a count call leaves only the leaves'
+        // offsets).  A graph's emission keeps them in memory of the graph.
+        rc = check_units(nleaves, res);
+        const size_t units = (size_t)nleaves * res, bytes = 2 * (units + 1) * sizeof(uint64_t);
         uint64_t* counts = nullptr;
-        if (int rc = plane_counts(c, dists, nleaves, res, nullptr, &counts, st)) return rc;
-        const size_t units = (size_t)nleaves * res;
-        hipLaunchKernelGGL((res == 64 ? k_mesh_emit_p<6> : k_mesh_emit_p<5>), dim3((uint32_t)units), dim3(kMeshBlock),
-                           0, st, spans, dists, counts, counts + units + 1, voff, ioff, verts, idx);
+        captured = is_capturing(st);
+        if (!rc && captured) rc = check_hip(hipMallocAsync((void**)&counts, bytes, st), "hipMallocAsync counts");
+        if (!rc && !captured) rc = c.emit_scratch(bytes, &counts, st);
+        if (!rc) rc = plane_counts(dists, nleaves, res, nullptr, counts, st);
+        if (!rc) {
+            hipLaunchKernelGGL((res == 64 ? k_mesh_emit_p<6> : k_mesh_emit_p<5>), dim3((uint32_t)units),
+                               dim3(kMeshBlock), 0, st, spans, dists, counts, counts + units + 1, voff, ioff, verts,
+                               idx);
+            rc = check_hip(hipGetLastError(), "mesh emit launch");
+        }
+        if (counts && captured) (void)hipFreeAsync(counts, st);
     }
-    int rc = check_hip(hipGetLastError(), "mesh emit launch");
-    if (rc || nverts == 0 || normals == CTH_NORMALS_DEFERRED) return rc;
-    return mesh_vertices(c, s, normals, nverts, verts, st);
+    if (!rc && nverts != 0 && normals != CTH_NORMALS_DEFERRED) rc = mesh_vertices(c, s, normals, nverts, verts, st);
+    if (res > 16 && !captured) {
+        const int re = c.emit_done(st);
+        if (!rc) rc = re;
+    }
+    return rc;
 }
 
 // The vertex pass: distance and normal of records that hold their position

@@ -38,12 +38,7 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
 // replays would claim from the entry of the context's ring that the capture took,
 // beside the launches in flight that the ring has come round to, and from freed
 // memory once the context is gone: no launch claims there, whatever its shape.
-// (The null stream cannot be captured.)
-inline bool foreign_capture(hipStream_t st) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return st && capture_pool().stream != st && hipStreamIsCapturing(st, &cs) == hipSuccess &&
-           cs != hipStreamCaptureStatusNone;
-}
+inline bool foreign_capture(hipStream_t st) { return capture_pool().stream != st && is_capturing(st); }
 
 // A launch's workgroups and chunks.  Up to a chunk of `least` indices (64 or
 // fewer) for each of spread.fill waves per CU a launch is spread as thinly as possible; from four

@@ -502,7 +502,8 @@ int cth_mesh_count_dev(cth_ctx* ctx, const float* dists, size_t nspans, uint32_t
  * EDGES order with the reference's distance weights (:149-250).  `nverts` is
  * the total from pass 1.  spans: 6 floats per leaf (the unadjusted span, as
  * given to cth_sample_spans_dev).  Uses a stream-ordered workspace of 28 bytes
- * per vertex for CTH_NORMALS_FD6. */
+ * per vertex for CTH_NORMALS_FD6 of a sphere.  Returns while it runs: the
+ * context's next call may be on another stream. */
 int cth_mesh_emit_dev(cth_ctx* ctx, const cth_shape* shape, const float* spans, const float* dists, size_t nspans,
                       uint32_t res, int normals, const uint64_t* vert_offsets, const uint64_t* idx_offsets,
                       uint64_t nverts, cth_vertex* vertices, uint32_t* indices, void* stream);

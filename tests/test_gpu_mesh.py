@@ -183,6 +183,53 @@ def test_mesh_offsets_of_one_and_many_workgroups(ctx, torch_cuda, res, leaves):
     assert torch.equal(v[at:], small[2][int(small[0][k]):int(small[0][k + 1])])
 
 
+@pytest.mark.parametrize("res", [32, 64])
+def test_emission_beside_calls_on_another_stream(ctx, torch_cuda, res):
+    """An emission returns while it still runs: the context's next calls, counts
+    and emissions of other leaves on another stream, leave its outputs alone.
+    Captured, it replays beside such calls too."""
+    import ctypes as C
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    rng = np.random.default_rng(res)
+    big, small = 40, 3000
+    shape = ca.Sphere((0.0, 0.0, 0.0), 1.0, ctx=ctx)
+    fields, spans, want = {}, {}, {}
+    for r, leaves in ((res, big), (8, small), (64 if res == 32 else 32, 7)):
+        base = torch.from_numpy(rng.choice(np.array([-1.0, 1.0], F32), (5, (r + 1) ** 3))).cuda()
+        fields[r] = base[torch.from_numpy(rng.integers(0, 5, leaves)).cuda()].contiguous()
+        spans[r] = torch.tensor([[-1.0, -1.0, -1.0, 1.0, 1.0, 1.0]], device="cuda").repeat(leaves, 1)
+        want[r] = dev.mesh(shape, spans[r], fields[r], r, "deferred")
+    voff, ioff, v_ref, i_ref = want[res]
+    v, ix = torch.empty_like(v_ref), torch.empty_like(i_ref)
+
+    def emit():
+        _lib.check(_lib.lib.cth_mesh_emit_dev(
+            ctx.handle, C.byref(shape.desc), spans[res].data_ptr(), fields[res].data_ptr(), big, res,
+            _lib.CTH_NORMALS_DEFERRED, voff.data_ptr(), ioff.data_ptr(), v.shape[0], v.data_ptr(), ix.data_ptr(),
+            torch.cuda.current_stream().cuda_stream))
+
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s1):
+        emit()
+    for rep, run in enumerate([emit, emit, g.replay, g.replay, g.replay]):
+        v.fill_(-1.0)
+        ix.fill_(-1)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s1):
+            run()
+        with torch.cuda.stream(s2):
+            others = {r: dev.mesh(shape, spans[r], fields[r], r, "deferred") for r in want if r != res}
+        torch.cuda.synchronize()
+        assert torch.equal(v, v_ref) and torch.equal(ix, i_ref), rep
+        for r, out in others.items():
+            for a, b in zip(out, want[r]):
+                assert torch.equal(a, b), (rep, r)
+
+
 def test_octree_leaf_mesh_parity(ctx, torch_cuda):
     """2,000 seeded depth-8 surface leaves of the octree workload (P8, 15 it,
     bailout 2, 8^3 cells per leaf)."""
