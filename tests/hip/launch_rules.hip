@@ -81,8 +81,26 @@ static void captures() {
     }
 }
 
+// A launch takes an entry of the ring only if it has more chunks than waves: of
+// 8^3-cell spans on one wave per CU, 30 take one, one takes none.  The ring comes
+// round after COUNTER_RING entries.
+static void ring_advances() {
+    std::vector<uint32_t> ring;
+    Ctx c = make_ctx(ring);
+    const LaunchShape thin{64, 1, 64, 32, 1, true}, full{256, 8, 256, 32, 1, true};
+    const WorkQueue first = queue(c, 3000 * 729, full, kStream);
+    CHECK(first.dynamic && c.ring_pos == 1);
+    for (uint32_t i = 1; i < COUNTER_RING; ++i) {
+        CHECK(!queue(c, 729, thin, kStream).ctr);
+        const WorkQueue q = queue(c, 30 * 729, thin, kStream);
+        CHECK(q.dynamic && q.ctr != first.ctr && c.ring_pos == i + 1);
+    }
+    CHECK(queue(c, 3000 * 729, full, kOther).ctr == first.ctr);
+}
+
 int main() {
     captures();
+    ring_advances();
     std::printf(g_failed ? "%d checks failed\n" : "launch rules ok\n", g_failed);
     return g_failed ? 1 : 0;
 }

@@ -260,3 +260,45 @@ def test_graph_counters_not_shared_with_eager_launches(torch_cuda):
         assert torch.equal(out_e.nan_to_num(7.0), ref.nan_to_num(7.0)), rep
     g.close()
     c.close()
+
+
+def test_graph_counters_not_shared_with_claiming_launches(ctx, torch_cuda):
+    """The same with launches in between that take an entry of the ring each (the
+    tiny ones above have no more chunks than waves, so they take none): 30 spans
+    of 8^3 cells on one wave per CU (tests/hip/launch_rules.hip counts their
+    entries)."""
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    from cantucci_amd.workloads import half_diagonals
+    torch = torch_cuda
+    assert torch.cuda.get_device_properties(0).multi_processor_count < 30 * 729 // 64
+    c = ca.Context(0, "parity")
+    big = lambda: c.set_launch(_lib.CTH_KERNEL_SPANS, 256, 8, 256, 32, dynamic=1)
+    big()
+    shape = ca.Mandelbulb.classic(15, 2.0, ctx=c)
+    leaves, _ = O.refine(O.mandelbulb(15, 2.0), [-1.5, -1.5, -1.5, 1.5, 1.5, 1.5], 2, 6, half_diagonals(3.0, 6))
+    spans = torch.from_numpy(leaves[:3000].copy()).cuda()
+    few = spans[:30].clone()
+    ref, _ = dev.sample_spans(shape, spans, 8, with_cross=False)
+    few_out = torch.empty((30, 729), device="cuda")
+    out_g, out_e = torch.empty_like(ref), torch.empty_like(ref)
+    s, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    g = dev.Graph(lambda: dev.sample_spans(shape, spans, 8, with_cross=False, out=out_g), s)
+    for rep in range(3):
+        for o in (out_g, out_e, few_out):
+            o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        c.set_launch(_lib.CTH_KERNEL_SPANS, 64, 1, 64, 32, dynamic=1)
+        for _ in range(4095):
+            dev.sample_spans(shape, few, 8, with_cross=False, out=few_out)
+        torch.cuda.synchronize()
+        big()
+        g.launch()
+        with torch.cuda.stream(s2):
+            dev.sample_spans(shape, spans, 8, with_cross=False, out=out_e)
+        torch.cuda.synchronize()
+        for got, want in ((out_g, ref), (out_e, ref), (few_out, ref[:30])):
+            assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), rep
+    g.close()
+    c.close()
