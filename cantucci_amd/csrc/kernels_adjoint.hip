@@ -368,11 +368,18 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
 // Workgroups are single waves: a wave needs (max_iters - 1) KiB of LDS, which
 // bounds the waves per CU (10 at 15 iterations, 5 at 30), and a SIMD needs
 // about three waves to issue at full rate.  So large caps stay with the two
-// kernels above: us for power 8 and for per-point powers, two kernels -> one,
-//   15 iterations: 300,000 points 62 -> 38, 94 -> 65; 1 M 135 -> 96, 158 -> 167;
-//                  4 M 545 -> 272, 615 -> 469;
-//   30 iterations: 300,000 points 107 -> 73, 162 -> 137; 1 M 196 -> 170,
-//                  232 -> 314; 4 M 674 -> 500, 883 -> 962.
+// kernels above.  A call, the workspace's allocation included, us for power 5
+// and for per-point powers, two kernels -> one:
+//   15 iterations: 2^18 points 149 -> 55, 149 -> 67; 2^20 227 -> 140, 187 -> 177;
+//                  2^22 598 -> 374, 658 -> 492;
+//   20 iterations: 2^18 139 -> 64, 153 -> 79; 2^20 252 -> 159, 282 -> 204;
+//                  2^22 713 -> 474, 702 -> 611;
+//   24 iterations: 2^18 182 -> 76, 192 -> 96; 2^20 237 -> 207, 302 -> 267;
+//                  2^22 683 -> 629, 726 -> 806;
+//   32 iterations: 2^18 167 -> 103, 213 -> 153; 2^20 305 -> 264, 276 -> 345;
+//                  2^22 851 -> 816, 941 -> 1057.
+// The kernels alone at 2^20 points and 15 iterations: 97 and 103 at power 8, 145
+// and 183 with per-point powers; the allocation of 268 MB takes the difference.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kFusedIters = 32;            // any point count at power 8
 constexpr uint32_t kFusedTrigIters = 20;        // trig map, any point count
@@ -579,15 +586,13 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
     const size_t stride = (size_t)u.max_iters + 1;
     if (stride > 4096) return fail(CTH_E_INVALID, "max_iters above 4095 for the adjoint");
     if (workspace && vjp_workspace_bytes(u.max_iters, n) > ws_bytes) return fail(CTH_E_INVALID, "workspace too small");
+    LaunchShape ls = single_waves(c.shape_adj);
     if (u.max_iters <= kFusedIters &&
         (family == FAM_P8 || u.max_iters <= kFusedTrigIters || n <= kFusedTrigPoints)) {
         const uint32_t lds = (u.max_iters - 1) * 64u * (uint32_t)sizeof(float4);
         const uint32_t granules = std::max(1u, (lds + 1279u) / 1280u);  // as LDS is allocated
         const uint32_t resident = std::min(16u, 160u * 1024u / (granules * 1280u));
         const WaveSpread spread{std::min(8u, resident), resident};
-        LaunchShape ls = c.shape_adj;
-        ls.blocks_per_cu *= ls.block / 64;
-        ls.block = 64;
         // `resident` need not spread evenly over a CU's four SIMDs: waves claim
         // their chunks where there are enough to even that out (4 M points at 15
         // iterations 558 -> 469 us, 300,000 points 65 -> 73).
@@ -627,27 +632,26 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
         SrcPoints src{pts + 3 * off, powers ? powers + off : nullptr, s.power};
         // kernel 1: parity forward with orbit recording
         uint32_t blocks = 0;
-        const WaveSpread spread = family == FAM_P8 ? P8Exact::kSpread : TrigExact::kSpread;
-        WorkQueue q = make_queue(c, m, c.shape_adj, spread, blocks, st);
+        WorkQueue q = make_queue(c, m, ls, kOrbitSpread, blocks, st);
         if (family == FAM_P8)
-            hipLaunchKernelGGL((k_adj_forward<P8Exact>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src, u, orbit, rec,
+            hipLaunchKernelGGL((k_adj_forward<P8Exact>), dim3(blocks), dim3(ls.block), 0, st, src, u, orbit, rec,
                                d ? d + off : nullptr, q);
         else
-            hipLaunchKernelGGL((k_adj_forward<TrigExact>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src, u, orbit,
-                               rec, d ? d + off : nullptr, q);
+            hipLaunchKernelGGL((k_adj_forward<TrigExact>), dim3(blocks), dim3(ls.block), 0, st, src, u, orbit, rec,
+                               d ? d + off : nullptr, q);
         rc = check_hip(hipGetLastError(), "adjoint forward launch");
         if (rc) break;
         // kernel 2: reverse sweep
         AdjOut out{grad_d ? grad_d + off : nullptr,         grad_p ? grad_p + 3 * off : nullptr,
                    grad_power ? grad_power + off : nullptr, normals ? normals + 3 * off : nullptr,
                    grad_z0 ? grad_z0 + 3 * off : nullptr,   grad_c ? grad_c + 3 * off : nullptr};
-        WorkQueue q2 = make_queue(c, m, c.shape_adj, spread, blocks, st);
+        WorkQueue q2 = make_queue(c, m, ls, kOrbitSpread, blocks, st);
         if (family == FAM_P8)
-            hipLaunchKernelGGL((k_adj_reverse<false>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src, u, orbit, rec,
-                               out, q2);
+            hipLaunchKernelGGL((k_adj_reverse<false>), dim3(blocks), dim3(ls.block), 0, st, src, u, orbit, rec, out,
+                               q2);
         else
-            hipLaunchKernelGGL((k_adj_reverse<true>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src, u, orbit, rec,
-                               out, q2);
+            hipLaunchKernelGGL((k_adj_reverse<true>), dim3(blocks), dim3(ls.block), 0, st, src, u, orbit, rec, out,
+                               q2);
         rc = check_hip(hipGetLastError(), "adjoint reverse launch");
     }
     if (own && orbit) (void)hipFreeAsync(orbit, st);

@@ -111,6 +111,23 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     return q;
 }
 
+// The reverse sweep's workgroups are single waves: the family's shape with as
+// many waves per CU.
+inline LaunchShape single_waves(LaunchShape ls) {
+    ls.blocks_per_cu *= ls.block / 64;
+    ls.block = 64;
+    return ls;
+}
+
+// Its two kernels (orbits in memory): a lane writes and reads its own orbit, 64
+// rows to a wave, and the waves of a CU share its vector cache, so few waves are
+// best and they start on CUs of their own.  Both kernels at 120 iterations, us,
+// on four-wave workgroups with the forward kernels' spread -> so: power 8
+// 5,000 points 233 -> 134, 2^18 298 -> 187, 2^20 1059 -> 431, 2^22 4077 -> 1770;
+// per-point powers 396 -> 282, 597 -> 371, 1228 -> 803, 4737 -> 3212.  (The
+// workspace's place in memory moves single figures by up to a quarter.)
+constexpr WaveSpread kOrbitSpread{8, 8};
+
 template <class Src, class Sink>
 inline int run_refill(Ctx& c, int family, const MandelUniform& u, const Src& src, const Sink& sink,
                       uint32_t total, hipStream_t st, const LaunchShape& ls) {

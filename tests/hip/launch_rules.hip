@@ -98,8 +98,25 @@ static void ring_advances() {
     CHECK(queue(c, 3000 * 729, full, kOther).ctr == first.ctr);
 }
 
+// The reverse sweep's two kernels run on single-wave workgroups, at most eight to
+// a CU and no more than the shape allows, whatever the size.
+static void orbit_sweep() {
+    std::vector<uint32_t> ring;
+    Ctx c = make_ctx(ring);
+    for (uint32_t n : {1u, 64u, 65u, 5000u, 262144u, 1048576u, 4194304u, 100000000u}) {
+        uint32_t blocks = 0;
+        const LaunchShape ls = single_waves(c.shape_adj);
+        WorkQueue q = make_queue(c, n, ls, kOrbitSpread, blocks, kStream);
+        CHECK(ls.block == 64 && blocks == q.waves && q.waves <= 8u * 256u);
+        CHECK(q.waves == std::min((n + 63u) / 64u, 8u * 256u));
+        q = make_queue(c, n, single_waves(LaunchShape{256, 1, 256, 32, 0, true}), kOrbitSpread, blocks, kStream);
+        CHECK(blocks == q.waves && q.waves <= 4u * 256u);
+    }
+}
+
 int main() {
     captures();
+    orbit_sweep();
     ring_advances();
     std::printf(g_failed ? "%d checks failed\n" : "launch rules ok\n", g_failed);
     return g_failed ? 1 : 0;
