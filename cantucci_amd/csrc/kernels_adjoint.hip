@@ -586,18 +586,13 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
     const size_t stride = (size_t)u.max_iters + 1;
     if (stride > 4096) return fail(CTH_E_INVALID, "max_iters above 4095 for the adjoint");
     if (workspace && vjp_workspace_bytes(u.max_iters, n) > ws_bytes) return fail(CTH_E_INVALID, "workspace too small");
-    LaunchShape ls = single_waves(c.shape_adj);
     if (u.max_iters <= kFusedIters &&
         (family == FAM_P8 || u.max_iters <= kFusedTrigIters || n <= kFusedTrigPoints)) {
         const uint32_t lds = (u.max_iters - 1) * 64u * (uint32_t)sizeof(float4);
         const uint32_t granules = std::max(1u, (lds + 1279u) / 1280u);  // as LDS is allocated
         const uint32_t resident = std::min(16u, 160u * 1024u / (granules * 1280u));
         const WaveSpread spread{std::min(8u, resident), resident};
-        // `resident` need not spread evenly over a CU's four SIMDs: waves claim
-        // their chunks where there are enough to even that out (4 M points at 15
-        // iterations 558 -> 469 us, 300,000 points 65 -> 73).
-        ls.dynamic = n / 256u >= (uint32_t)c.num_cus * spread.fill;
-        ls.given = true;
+        const LaunchShape ls = sweep_shape(c.shape_adj, n, c.num_cus, spread.fill);
         SrcPoints src{pts, powers, s.power};
         AdjOut out{grad_d, grad_p, grad_power, normals, grad_z0, grad_c};
         uint32_t blocks = 0;
@@ -608,6 +603,7 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
             hipLaunchKernelGGL((k_adjoint<TrigExact, true>), dim3(blocks), dim3(64), lds, st, src, u, d, out, q);
         return check_hip(hipGetLastError(), "adjoint launch");
     }
+    const LaunchShape ls = single_waves(c.shape_adj);
     size_t per_point = stride * sizeof(float4) + sizeof(AdjRecord);
     float4* orbit = nullptr;
     AdjRecord* rec = nullptr;

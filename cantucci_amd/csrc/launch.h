@@ -119,6 +119,18 @@ inline LaunchShape single_waves(LaunchShape ls) {
     return ls;
 }
 
+// Its one kernel (orbits in LDS), for n points on at least `fill` waves per CU:
+// what fits beside the orbits need not spread evenly over a CU's four SIMDs, so
+// waves claim their chunks where there are enough to even that out (4 M points
+// at 15 iterations 558 -> 469 us, 300,000 points 65 -> 73), unless the caller's
+// shape is static.
+inline LaunchShape sweep_shape(const LaunchShape& family, uint32_t n, int num_cus, uint32_t fill) {
+    LaunchShape ls = single_waves(family);
+    ls.dynamic = (!family.given || family.dynamic) && n / 256u >= (uint32_t)num_cus * fill;
+    ls.given = true;
+    return ls;
+}
+
 // Its two kernels (orbits in memory): a lane writes and reads its own orbit, 64
 // rows to a wave, and the waves of a CU share its vector cache, so few waves are
 // best and they start on CUs of their own.  Both kernels at 120 iterations, us,

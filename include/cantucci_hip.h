@@ -143,7 +143,9 @@ int cth_ctx_num_cus(const cth_ctx* ctx);
  * takes new ones; dynamic = 1 claims chunks from an atomic counter, 0 walks
  * chunks w, w+W, w+2W, ... statically (W waves).  While no shape has been set
  * for a family whose default is static, its large launches claim chunks of up
- * to 1024 all the same.  Launches recorded by a stream capture that
+ * to 1024 all the same.  The reverse sweep takes the ADJOINT shape in workgroups
+ * of one wave, and its launches of few chunks are static with 1 too.  Launches
+ * recorded by a stream capture that
  * cth_graph_begin did not begin are static whatever the shape: such a graph
  * owns no counters.  No counterpart in the
  * reference (its work is scheduled by a CPU thread pool,

@@ -114,8 +114,22 @@ static void orbit_sweep() {
     }
 }
 
+// The reverse sweep's one kernel claims from four chunks of 64 a wave on, and not
+// at all where the caller's shape is static.
+static void sweep_shapes() {
+    for (uint32_t n : {1u, 300000u, 524287u, 524288u, 30000000u}) {
+        CHECK(sweep_shape(LaunchShape{}, n, 256, 8).dynamic == (n >= 524288u));
+        for (uint32_t dyn : {0u, 1u}) {
+            const LaunchShape w = sweep_shape(LaunchShape{128, 16, 128, 32, dyn, true}, n, 256, 8);
+            CHECK(w.given && w.dynamic == (dyn && n >= 524288u));
+            CHECK(w.block == 64 && w.blocks_per_cu == 32 && w.chunk == 128);
+        }
+    }
+}
+
 int main() {
     captures();
+    sweep_shapes();
     orbit_sweep();
     ring_advances();
     std::printf(g_failed ? "%d checks failed\n" : "launch rules ok\n", g_failed);
