@@ -54,6 +54,18 @@ struct LaunchShape {
     uint32_t refill_min = 32;  // idle lanes that trigger a refill (1..64)
     uint32_t dynamic = 0;      // 0: static interleaved chunks, 1: atomic claims
     bool given = false;        // set by the caller; else make_queue lets large static launches claim
+    // As cth_launch; its dynamic is 2 for a static shape whose large launches claim.
+    cth_launch get() const {
+        return {block, blocks_per_cu, chunk, refill_min, dynamic ? 1u : (given ? 0u : 2u)};
+    }
+    void set(const cth_launch& l) {
+        block = l.block;
+        blocks_per_cu = l.blocks_per_cu;
+        chunk = l.chunk;
+        refill_min = l.refill_min;
+        dynamic = l.dynamic == 0 || l.dynamic == 2 ? 0u : 1u;
+        given = l.dynamic != 2;
+    }
 };
 
 // Device scratch slots of a context, grown on demand and kept until the

@@ -140,15 +140,14 @@ int cth_ctx_num_cus(const cth_ctx* ctx);
  * or 256 threads; blocks_per_cu persistent workgroups per CU (1..32); chunk
  * indices claimed per wave from the work counter (64..65536); refill_min the
  * number of idle lanes (1..64) at which a wave writes finished points and
- * takes new ones; dynamic = 1 claims chunks from an atomic counter, 0 walks
- * chunks w, w+W, w+2W, ... statically (W waves).  While no shape has been set
- * for a family whose default is static, its large launches claim chunks of up
- * to 1024 all the same.  The reverse sweep takes the ADJOINT shape in workgroups
- * of one wave, and its launches of few chunks are static with 1 too.  Launches
- * recorded by a stream capture that
- * cth_graph_begin did not begin are static whatever the shape: such a graph
- * owns no counters.  No counterpart in the
- * reference (its work is scheduled by a CPU thread pool,
+ * takes new ones; dynamic = 1 claims chunks from atomic counters, 0 deals them
+ * statically (a wave walks one chunk of each row of W, for W waves), 2 (the
+ * default of most families) deals small launches statically and lets large ones
+ * claim chunks of up to 1024 whatever the other numbers.  The reverse sweep takes
+ * the ADJOINT shape in workgroups of one wave, and its launches of few chunks are
+ * static with 1 too.  Launches recorded by a stream capture that cth_graph_begin
+ * did not begin are static whatever the shape: such a graph owns no counters.  No
+ * counterpart in the reference (its work is scheduled by a CPU thread pool,
  * src/mesh/mod.rs:60-63,141-148). */
 typedef struct cth_launch {
     int32_t block;

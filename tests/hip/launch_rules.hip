@@ -127,8 +127,40 @@ static void sweep_shapes() {
     }
 }
 
+static bool same(const WorkQueue& a, const WorkQueue& b) {
+    return a.waves == b.waves && a.chunk == b.chunk && a.chunks == b.chunks && a.rotate == b.rotate &&
+           a.dynamic == b.dynamic && a.refill_min == b.refill_min;
+}
+
+// A shape that was read and is set back, also after another, leaves every launch
+// as it was; the caller's static and claiming shapes are kept in all sizes.
+static void shapes_kept() {
+    std::vector<uint32_t> r0, r1;
+    Ctx c = make_ctx(r0), d = make_ctx(r1);
+    for (int k : {CTH_KERNEL_DE, CTH_KERNEL_TRACE, CTH_KERNEL_ADJOINT, CTH_KERNEL_SPANS, CTH_KERNEL_JOBS,
+                  CTH_KERNEL_MESH}) {
+        LaunchShape *a = c.launch_shape(k), *b = d.launch_shape(k);
+        const cth_launch was = b->get();
+        b->set({128, 3, 128, 7, 1});
+        b->set(was);
+        for (uint32_t n : {1u, 300000u, 4000000u, 30000000u}) {
+            CHECK(same(queue(c, n, *a, kStream), queue(d, n, *b, kStream)));
+            for (int dyn : {0, 1}) {
+                LaunchShape s;
+                s.set({256, 16, 256, 32, (uint32_t)dyn});
+                CHECK(s.get().dynamic == (uint32_t)dyn);
+                const WorkQueue q = queue(c, n, s, kStream);
+                CHECK(!q.dynamic || dyn);
+                CHECK(q.chunk <= 256u);
+                CHECK(n != 30000000u || q.dynamic == (uint32_t)dyn);
+            }
+        }
+    }
+}
+
 int main() {
     captures();
+    shapes_kept();
     sweep_shapes();
     orbit_sweep();
     ring_advances();

@@ -251,3 +251,23 @@ def test_captures_without_counters(torch_cuda):
         js.close()
         c.close()
         other.close()
+
+
+def test_shape_read_and_set_back(torch_cuda):
+    """A family's shape can be read, replaced and set back: what it reports tells
+    the default, whose large launches claim, from the same numbers set static."""
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    c = ca.Context(0, "parity")
+    try:
+        for f in (_lib.CTH_KERNEL_DE, _lib.CTH_KERNEL_TRACE, _lib.CTH_KERNEL_ADJOINT, _lib.CTH_KERNEL_SPANS,
+                  _lib.CTH_KERNEL_JOBS, _lib.CTH_KERNEL_MESH):
+            was = c.get_launch(f)
+            assert was["dynamic"] == (1 if f in (_lib.CTH_KERNEL_SPANS, _lib.CTH_KERNEL_MESH) else 2)
+            for dyn in (0, 1):
+                c.set_launch(f, **{**was, "dynamic": dyn})
+                assert c.get_launch(f) == {**was, "dynamic": dyn}
+            c.set_launch(f, **was)
+            assert c.get_launch(f) == was
+    finally:
+        c.close()
