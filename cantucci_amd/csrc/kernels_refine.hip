@@ -113,7 +113,15 @@ __global__ void k_emit_leaves(const float* __restrict__ nodes, const uint32_t* _
 // and 7 of the octree: 82, 129, 158, 226 -> 27, 55, 98, 167 us.  Up to 512 nodes
 // gave 27, 69, 97, 166, up to 10,240 27, 55, 156, 257 (one CU is then slower
 // than a level of launches); real powers take 51 us more with 4,096.
+//
+// One CU's waves share its issue slots, a level's own launch spreads over the
+// chip: with caps above kTopIters the top's points take longer than the launches
+// it saves, except under the trig map's integer powers.  One launch / level by
+// level, us, depths 2 to 4: power 8 at 100 / 150 / 400 / 1000 iterations 194 / 218,
+// 273 / 262, 671 / 472, 1624 / 981; power 5 201 / 271, 270 / 336, 615 / 661,
+// 1441 / 1451; a real power 454 / 493, 652 / 673, 1634 / 1566, 3977 / 3708.
 constexpr uint32_t kTopNodes = 2048;
+constexpr uint32_t kTopIters = 128;
 constexpr uint32_t kTopThreads = 1024;
 constexpr uint32_t kMaxDepth = 20;
 static_assert(2 + kMaxDepth + 1 <= kPinnedWords, "level counts fit");
@@ -216,10 +224,9 @@ __global__ __launch_bounds__(kTopThreads) void k_refine_top(RefineTop a, MandelU
 static inline uint32_t cdiv32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 // Level-synchronous refinement: the top of the tree in one launch, then per
-// level the split flags (forced, sphere
-// closed form or a DE refill launch), an inclusive scan of the flags, one
-// 4-byte read-back of the split count into pinned host memory, and the
-// children.  Node, flag, offset and scan buffers are the context's scratch
+// level the split flags (forced, sphere closed form or a DE refill launch), an
+// inclusive scan of the flags, one 4-byte read-back of the split count into
+// pinned host memory, and the children.  Node, flag, offset and scan buffers are the context's scratch
 // slots (ping-pong for the nodes), so a level allocates nothing.
 int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_depth, uint32_t max_depth,
                   const float* half_diag, float* leaves, size_t cap, size_t* nleaves, uint64_t* level_counts,
@@ -235,11 +242,14 @@ int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_de
     uint32_t depth = 0;
     uint64_t n = 1;
     float* nodes[2] = {};
-    const size_t first = c.stats ? 1 : (size_t)8 * kTopNodes;
+    // counted work goes through the work loops
+    const bool top_launch = !c.stats && (family == FAM_SPHERE || u.max_iters <= kTopIters ||
+                                         (family == FAM_TRIG && u.integral));
+    const size_t first = top_launch ? (size_t)8 * kTopNodes : 1;
     int rc = CTH_OK;
     for (int k = 0; k < 2 && !rc; ++k) rc = c.scratch(WS_NODES_A + k, first * 6 * sizeof(float), (void**)&nodes[k]);
     if (rc) return fail(rc, "refinement scratch allocation failed");
-    if (!c.stats) {
+    if (top_launch) {
         RefineTop top{};
         std::copy(root, root + 6, top.root);
         std::copy(half_diag, half_diag + max_depth + 1, top.half_diag);
@@ -273,7 +283,7 @@ int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_de
             *nleaves = n;
             return CTH_OK;
         }
-    } else {  // counted work goes through the work loops
+    } else {
         rc = check_hip(hipMemcpyAsync(nodes[0], root, 6 * sizeof(float), hipMemcpyHostToDevice, st), "H2D root");
     }
     int slot = WS_NODES_A + (int)(depth & 1u);

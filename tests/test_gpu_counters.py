@@ -109,3 +109,28 @@ def test_refinement_top_matches_levels(ctx, torch_cuda, kind, min_depth, max_dep
         m = min(keep.shape[0], want.shape[0])
         assert torch.equal(keep[:m], want[:m])
         assert (few[-1] == 7.0).all()
+
+
+@pytest.mark.parametrize("iters", [128, 129, 300])
+@pytest.mark.parametrize("kind", ["p8", "p5", "real"])
+def test_refinement_at_large_caps(ctx, torch_cuda, kind, iters):
+    """Iteration caps on both sides of the one up to which the tree's top is one
+    launch for every map: the counted refinement's leaves and level counts."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    from cantucci_amd.workloads import half_diagonals
+    torch = torch_cuda
+    shape = {"p8": lambda: ca.Mandelbulb.classic(iters, 2.0, ctx=ctx),
+             "p5": lambda: ca.Mandelbulb(iters, 2.0, 5, ctx=ctx),
+             "real": lambda: ca.MandelbulbTrig(iters, 2.0, 6.5, ctx=ctx)}[kind]()
+    root, hd = (-1.5,) * 3 + (1.5,) * 3, half_diagonals(3.0, 5)
+    cnt = torch.zeros(4, dtype=torch.int64, device="cuda")
+    ctx.count_work(cnt)
+    try:
+        want, want_lc = dev.refine(shape, root, 1, 5, hd)
+        torch.cuda.synchronize()
+    finally:
+        ctx.count_work(None)
+    got, lc = dev.refine(shape, root, 1, 5, hd)
+    assert (lc == want_lc).all()
+    assert torch.equal(got, want)
