@@ -111,6 +111,17 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     return q;
 }
 
+// A refinement level's launch: the span family's shape with 64-point chunks dealt
+// statically, which spreads a level over the whole chip; levels of millions of
+// nodes claim as every default shape does, whether the span shape is the caller's
+// or not (depth 10 of the octree, 16 M nodes: static 2.78 ms, so 2.50).
+inline LaunchShape level_shape(LaunchShape spans) {
+    spans.chunk = 64;
+    spans.dynamic = 0;
+    spans.given = false;
+    return spans;
+}
+
 // The reverse sweep's workgroups are single waves: the family's shape with as
 // many waves per CU.
 inline LaunchShape single_waves(LaunchShape ls) {

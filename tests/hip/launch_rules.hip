@@ -158,7 +158,23 @@ static void shapes_kept() {
     }
 }
 
+// A refinement level is launched the same on a default span shape and on one
+// set by the caller: static, and claiming from 4 chunks of 128 a wave on.
+static void refinement_levels() {
+    std::vector<uint32_t> ring;
+    Ctx c = make_ctx(ring);
+    LaunchShape set = c.shape_spans;
+    set.given = true;
+    for (uint32_t n : {1u, 100000u, 4194303u, 4194304u, 200000000u}) {
+        const WorkQueue q = queue(c, n, level_shape(c.shape_spans), kStream);
+        CHECK(same(q, queue(c, n, level_shape(set), kStream)));
+        CHECK(q.dynamic == (n >= 4194304u));
+        CHECK(q.dynamic || q.chunk == 64u);
+    }
+}
+
 int main() {
+    refinement_levels();
     captures();
     shapes_kept();
     sweep_shapes();
