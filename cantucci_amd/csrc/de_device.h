@@ -210,13 +210,17 @@ __device__ __forceinline__ void powi_pair(float x, uint32_t n, float& lo, float&
 struct MandelUniform {
     uint32_t max_iters;
     float bailout;
-    float power;    // used when no per-point power is given
+    float power;    // used when no per-point power is given (else kPointPower)
     int ipower;     // integer power when `integral`
     int integral;   // 1: every point uses ipower (reference Mandelbulb<P>);
                     // 0: real power per point (powf unless integral and < 64)
     float center[3];  // sphere evaluator only
     float radius;
 };
+
+// `power` of a launch with a power per point, for its lanes without a point
+// (idle_start): such powers are seldom integers.
+constexpr float kPointPower = 8.5f;
 
 // How an evaluator's launches spread over the chip, in waves per CU
 // (make_queue): a small launch to `fill` waves, no launch beyond `most` (as
@@ -739,13 +743,15 @@ __device__ __forceinline__ float tick_full(E& ev, float& r, const MandelUniform&
 
 // A lane that has not taken a point yet: the work loops run bodies on all
 // lanes of a wave, and what such a lane computes is dropped, but it must not
-// send the wave through a rare path.  (Left uninitialised, the 16 spare lanes
-// of a last wave of 48 points ran the power ladder and the large-argument sine
-// on leftover registers: 62 us against 17 us for 30,000 points at power 5.)
-// Returns its magnitude.
+// send the wave through a path that its other lanes do not take: it has the
+// launch's power.  (Left uninitialised, the 16 spare lanes of a last wave of 48
+// points ran the power ladder and the large-argument sine on leftover registers:
+// 62 us against 17 us for 30,000 points at power 5.  At power 8, whose ladder
+// the waves of a real power then ran beside powf, 25 rays at power 6.5 took 317 us
+// and a 320 x 200 image 2.28 ms; so 232 us and 1.75 ms.)  Returns its magnitude.
 template <class E>
 __device__ __forceinline__ float idle_start(E& ev, const MandelUniform& u) {
-    ev.start(0.5f, 0.5f, 0.5f, 8.0f, u);
+    ev.start(0.5f, 0.5f, 0.5f, u.power, u);
     return ev.mag();
 }
 

@@ -583,6 +583,7 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
     int family = 0;
     int rc = resolve_mandel(s, u, family);
     if (rc) return rc;
+    if (powers) u.power = kPointPower;
     const size_t stride = (size_t)u.max_iters + 1;
     if (stride > 4096) return fail(CTH_E_INVALID, "max_iters above 4095 for the adjoint");
     if (workspace && vjp_workspace_bytes(u.max_iters, n) > ws_bytes) return fail(CTH_E_INVALID, "workspace too small");
@@ -665,6 +666,7 @@ int launch_tangent(Ctx& c, const cth_shape& s, const float* pts, const float* po
     int family = 0;
     int rc = resolve_mandel(s, u, family);
     if (rc) return rc;
+    if (powers) u.power = kPointPower;
     SrcPoints src{pts, powers, s.power};
     SinkGrad sink{d, normals, grad_p, grad_power, grad_d, u.max_iters};
     uint32_t blocks = 0;
@@ -698,6 +700,7 @@ int launch_fd_normals(Ctx& c, const cth_shape& s, const float* pts, const float*
         MandelUniform u;
         int family = 0;
         rc = resolve_mandel(s, u, family);
+        if (powers) u.power = kPointPower;
         if (!rc) rc = run_refill(c, family, u, src, SinkDist{taps}, n * 7, st, c.shape_de);
     }
     if (!rc) {

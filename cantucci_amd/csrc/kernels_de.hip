@@ -88,6 +88,7 @@ int launch_de_points(Ctx& c, const cth_shape& s, const float* pts, const float* 
     int family = 0;
     int rc = resolve_mandel(s, u, family);
     if (rc != CTH_OK) return rc;
+    if (powers) u.power = kPointPower;
     if (r_out) {
         SinkState sink{r_out, dr_out, iters};
         return run_refill(c, family, u, src, sink, n, st, c.shape_de);

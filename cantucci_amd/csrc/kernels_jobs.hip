@@ -249,7 +249,7 @@ int jobs_run(Ctx& c, const JobSet& js, float* dists, float* normals, unsigned lo
     MandelUniform u{};
     u.max_iters = 0;  // per job
     u.bailout = js.bailout;
-    u.power = 8.0f;
+    u.power = kPointPower;
     u.integral = (js.kind == CTH_SHAPE_MANDELBULB) ? 1 : 0;
     u.ipower = 8;
     hipLaunchKernelGGL(k_jobs_reset, dim3((js.njobs + 255) / 256), dim3(256), 0, st, done, js.njobs, start);
