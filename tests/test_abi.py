@@ -212,3 +212,17 @@ def test_mesh_buffers_fit_or_run_again(nv, ni):
     assert (verts.view("u1") == 1).all() and (idx.view("u1") == 2).all()
     with pytest.raises(ca.CthError):
         _fill(1, 1, lambda *a: 1)
+
+
+def test_tuner_job_sets_are_layouts_of_their_own():
+    """The tuner's job sets differ from each other and from the full-size mixed
+    jobs, job for job (a set is not the first jobs of another)."""
+    from cantucci_amd import autotune
+    from cantucci_amd import workloads as wl
+    import numpy as np
+    full = wl.mixed_jobs(**{k: v for k, v in wl.MIXED_JOBS.items() if k != "bailout"})
+    sets = [full] + [wl.mixed_jobs(n, seed=s) for n, s in autotune.JOB_SETS]
+    assert len({n for n, _ in autotune.JOB_SETS}) >= 4
+    for i, a in enumerate(sets):
+        for b in sets[:i]:
+            assert not np.isin(a[1], b[1]).any()
