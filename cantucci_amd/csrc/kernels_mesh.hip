@@ -990,7 +990,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 #pragma unroll
                     for (int b = 0; b < 3; ++b) c[b] = c[b] + ((a == b) ? 1.0f : 0.0f) * h;
                 }
-                ev.start(c[0], c[1], c[2], 0.0f, u);
+                ev.start(c[0], c[1], c[2], u.power, u);
                 t0 = tick;
                 r = ev.mag();
             }

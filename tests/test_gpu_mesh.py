@@ -183,6 +183,38 @@ def test_mesh_offsets_of_one_and_many_workgroups(ctx, torch_cuda, res, leaves):
     assert torch.equal(v[at:], small[2][int(small[0][k]):int(small[0][k + 1])])
 
 
+@pytest.mark.parametrize("kind", ["p8", "p5", "p2", "real", "sphere"])
+@pytest.mark.parametrize("res", [8, 32])
+def test_tap_normals_are_those_of_the_distances(ctx, torch_cuda, kind, res):
+    """distance_from_surface and the 6-tap normal of every kind of shape are formed
+    from the distances of point batches at the vertex and its taps
+    (src/mesh/buffer.rs:254-272), bit for bit."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    shape = {"p8": lambda: ca.Mandelbulb.classic(6, 2.0, ctx=ctx), "p5": lambda: ca.Mandelbulb(6, 2.0, 5, ctx=ctx),
+             "p2": lambda: ca.Mandelbulb(4, 2.0, 2, ctx=ctx), "real": lambda: ca.MandelbulbTrig(6, 2.0, 6.5, ctx=ctx),
+             "sphere": lambda: ca.Sphere((0.0, 0.1, 0.2), 0.9, ctx=ctx)}[kind]()
+    spans = gpu(torch, np.array([[-0.6, -0.6, 0.2, 0.6, 0.6, 1.2], [-1.1, -0.3, -0.5, -0.1, 0.5, 0.4]], F32))
+    d, _ = dev.sample_spans(shape, spans, res)
+    _, _, raw, _ = dev.mesh(shape, spans, d, res, "deferred")
+    _, _, v, _ = dev.mesh(shape, spans, d, res, "fd6")
+    assert len(v) > 100
+    raw, v = raw.cpu().numpy(), v.cpu().numpy()
+    p = raw[:, None, :3].repeat(7, 1)
+    for a in range(3):
+        p[:, 1 + 2 * a, a] = raw[:, a] + raw[:, 3 + a]
+        p[:, 2 + 2 * a, a] = raw[:, a] - raw[:, 3 + a]
+    t = dev.de_points(shape, gpu(torch, p.reshape(-1, 3))).cpu().numpy().reshape(-1, 7)
+    g = t[:, 1::2] - t[:, 2::2]
+    m = np.sqrt((g[:, 0] * g[:, 0] + g[:, 1] * g[:, 1]) + g[:, 2] * g[:, 2])
+    with np.errstate(all="ignore"):
+        n = g * (F32(1.0) / m)[:, None]
+    assert same_bits(v[:, :3], raw[:, :3]).all()
+    assert same_bits(v[:, 6], t[:, 0]).all()
+    assert (same_bits(v[:, 3:6], n) | (np.isnan(v[:, 3:6]) & np.isnan(n))).all()
+
+
 @pytest.mark.parametrize("res", [32, 64])
 def test_emission_beside_calls_on_another_stream(ctx, torch_cuda, res):
     """An emission returns while it still runs: the context's next calls, counts
