@@ -27,18 +27,26 @@ class Timings:
     faces: int
 
 
+_FIRST_BYTES = 1 << 28  # what the first buffers of _fill may take (some 200 leaves of 64^3 cells)
+
+
 def _fill(leaves: int, resolution: int, run):
     """The vertices and indices of run(verts, vert_cap, idx, idx_cap, &nverts,
     &nidx).  The first buffers hold more than a surface through the leaves
     usually has (their untouched pages cost nothing and are given back), so that
-    the leaves are sampled once; a mesh beyond them runs again."""
+    the leaves are sampled once; a mesh beyond them runs again.  Where they would
+    be large, the first run only counts (null buffers)."""
     nv, ni = C.c_size_t(), C.c_size_t()
-    vcap = leaves * (6 * resolution * resolution + 64)
+    r = int(resolution) if 0 < resolution <= 64 else 0  # others are refused
+    vcap = leaves * (6 * r * r + 64)
     icap = 6 * vcap
+    if vcap * VERTEX_DTYPE.itemsize + icap * 4 > _FIRST_BYTES:
+        vcap = icap = 0
     while True:
         verts = np.empty(vcap, VERTEX_DTYPE)
         idx = np.empty(icap, np.uint32)
-        rc = run(verts.ctypes.data, vcap, idx.ctypes.data, icap, C.byref(nv), C.byref(ni))
+        rc = run(verts.ctypes.data if vcap else None, vcap, idx.ctypes.data if icap else None, icap, C.byref(nv),
+                 C.byref(ni))
         if nv.value <= vcap and ni.value <= icap:
             break
         vcap, icap = nv.value, ni.value

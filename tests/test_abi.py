@@ -226,3 +226,30 @@ def test_tuner_job_sets_are_layouts_of_their_own():
     for i, a in enumerate(sets):
         for b in sets[:i]:
             assert not np.isin(a[1], b[1]).any()
+
+
+@pytest.mark.parametrize("leaves", [150, 300, 100000])
+def test_mesh_buffers_of_many_leaves(leaves):
+    """The first buffers stay within a fixed size whatever the leaves: beyond it the
+    first run gets none and only counts.  A resolution the library refuses asks
+    for no large buffer first."""
+    import cantucci_amd as ca
+    from cantucci_amd import mesh as M
+    calls, nv, ni = [], 1000, 6000
+
+    def run(v, vcap, i, icap, pnv, pni):
+        assert vcap * M.VERTEX_DTYPE.itemsize + icap * 4 <= M._FIRST_BYTES
+        assert (v is None) == (vcap == 0) and (i is None) == (icap == 0)
+        calls.append(vcap)
+        pnv._obj.value, pni._obj.value = nv, ni
+        if v:
+            C.memset(v, 1, nv * M.VERTEX_DTYPE.itemsize)
+            C.memset(i, 2, 4 * ni)
+        return 0
+
+    verts, idx = M._fill(leaves, 64, run)
+    assert len(verts) == nv and len(idx) == ni and (idx.view("u1") == 2).all()
+    assert calls == ([0, nv] if leaves > 200 else [leaves * (6 * 64 * 64 + 64)])
+    for res in (0, -4, 128, 10 ** 9):
+        with pytest.raises(ca.CthError):
+            M._fill(1, res, lambda v, vcap, *a: 1 if vcap <= 64 else 0)

@@ -563,3 +563,25 @@ def test_shape_mesh_new_and_update(ctx, torch_cuda):
     assert flags.sum() > 0 and same_bits(spans_of(), np.array(want2, F32)).all()
     assert all(buf is not None for _, buf in sm.leaves)
     check_meshes(children)
+
+
+@pytest.mark.parametrize("res", [8, 64])
+def test_counted_first(ctx, torch_cuda, monkeypatch, res):
+    """Host meshes whose first run only counts, as those of many leaves do, are the
+    ones that are filled at once."""
+    import cantucci_amd as ca
+    from cantucci_amd import mesh as M
+    shape = ca.Mandelbulb.classic(6, 2.0, ctx=ctx)
+    for box in (((-0.6, -0.6, 0.2), (0.6, 0.6, 1.2)), ((3.0, 3.0, 3.0), (4.0, 4.0, 4.0))):
+        a, _ = M.MeshBuffer.generate_for_box(box, shape, res)
+        with monkeypatch.context() as m:
+            m.setattr(M, "_FIRST_BYTES", 0)
+            b, _ = M.MeshBuffer.generate_for_box(box, shape, res)
+        assert np.array_equal(a.vertices, b.vertices) and np.array_equal(a.indices, b.indices)
+    if res == M.ShapeMesh.RESOLUTION:
+        meshes = [M.ShapeMesh(shape), M.ShapeMesh(shape)]
+        meshes[0]._mesh_empty_leaves()
+        monkeypatch.setattr(M, "_FIRST_BYTES", 0)
+        meshes[1]._mesh_empty_leaves()
+        for (_, x), (_, y) in zip(meshes[0].leaves, meshes[1].leaves):
+            assert np.array_equal(x.vertices, y.vertices) and np.array_equal(x.indices, y.indices)
