@@ -219,8 +219,11 @@ struct MandelUniform {
 };
 
 // `power` of a launch with a power per point, for its lanes without a point
-// (idle_start): such powers are seldom integers.
-constexpr float kPointPower = 8.5f;
+// (idle_start): an integer, whose ladder is one squaring, so that they cost
+// little beside real powers' powf and beside other ladders.  100 points at
+// integer / real powers with 8.5 here 27.0 / 20.7 us, so 16.8 / 22.1; 100,000
+// 28.4 / 27.1 and 18.5 / 27.2.
+constexpr float kPointPower = 1.0f;
 
 // How an evaluator's launches spread over the chip, in waves per CU
 // (make_queue): a small launch to `fill` waves, no launch beyond `most` (as

@@ -173,7 +173,16 @@ static void refinement_levels() {
     }
 }
 
+// Lanes without a point in a launch with a power per point run the shortest
+// power ladder (powi_ladder halves its exponent once per turn), not powf.
+static void idle_power() {
+    const int n = (int)kPointPower;
+    CHECK((float)n == kPointPower && n >= 1 && n < 64);
+    CHECK(n / 2 == 0);
+}
+
 int main() {
+    idle_power();
     refinement_levels();
     captures();
     shapes_kept();
