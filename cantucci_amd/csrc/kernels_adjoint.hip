@@ -367,24 +367,9 @@ __global__ __launch_bounds__(256) void k_adj_reverse(SrcPoints src, MandelUnifor
 //
 // Workgroups are single waves: a wave needs (max_iters - 1) KiB of LDS, which
 // bounds the waves per CU (10 at 15 iterations, 5 at 30), and a SIMD needs
-// about three waves to issue at full rate.  So large caps stay with the two
-// kernels above.  A call, the workspace's allocation included, us for power 5
-// and for per-point powers, two kernels -> one:
-//   15 iterations: 2^18 points 149 -> 55, 149 -> 67; 2^20 227 -> 140, 187 -> 177;
-//                  2^22 598 -> 374, 658 -> 492;
-//   20 iterations: 2^18 139 -> 64, 153 -> 79; 2^20 252 -> 159, 282 -> 204;
-//                  2^22 713 -> 474, 702 -> 611;
-//   24 iterations: 2^18 182 -> 76, 192 -> 96; 2^20 237 -> 207, 302 -> 267;
-//                  2^22 683 -> 629, 726 -> 806;
-//   32 iterations: 2^18 167 -> 103, 213 -> 153; 2^20 305 -> 264, 276 -> 345;
-//                  2^22 851 -> 816, 941 -> 1057.
-// The kernels alone at 2^20 points and 15 iterations: 97 and 103 at power 8, 145
-// and 183 with per-point powers; the allocation of 268 MB takes the difference.
+// about three waves to issue at full rate: one_sweep_kernel (launch.h) leaves
+// large caps with many points to the two kernels above.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kFusedIters = 32;            // any point count at power 8
-constexpr uint32_t kFusedTrigIters = 20;        // trig map, any point count
-constexpr uint32_t kFusedTrigPoints = 1u << 18;  // trig map, up to kFusedIters
-
 template <class Ev, bool TRIG>
 __global__ __launch_bounds__(64) void k_adjoint(SrcPoints src, MandelUniform u, float* __restrict__ dout, AdjOut out,
                                                 WorkQueue q) {
@@ -587,8 +572,7 @@ int launch_adjoint(Ctx& c, const cth_shape& s, const float* pts, const float* po
     const size_t stride = (size_t)u.max_iters + 1;
     if (stride > 4096) return fail(CTH_E_INVALID, "max_iters above 4095 for the adjoint");
     if (workspace && vjp_workspace_bytes(u.max_iters, n) > ws_bytes) return fail(CTH_E_INVALID, "workspace too small");
-    if (u.max_iters <= kFusedIters &&
-        (family == FAM_P8 || u.max_iters <= kFusedTrigIters || n <= kFusedTrigPoints)) {
+    if (one_sweep_kernel(u.max_iters, n, family == FAM_P8 ? 22u : u.integral ? 20u : 16u)) {
         const uint32_t lds = (u.max_iters - 1) * 64u * (uint32_t)sizeof(float4);
         const uint32_t granules = std::max(1u, (lds + 1279u) / 1280u);  // as LDS is allocated
         const uint32_t resident = std::min(16u, 160u * 1024u / (granules * 1280u));

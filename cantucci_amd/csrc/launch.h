@@ -122,6 +122,31 @@ inline LaunchShape level_shape(LaunchShape spans) {
     return spans;
 }
 
+// Whether the reverse sweep of n points runs in one kernel (orbits in LDS) or in
+// two (orbits in memory).  The LDS leaves fewer waves per CU with every
+// iteration, which costs nothing while there are few points for each CU; `any`
+// is the cap up to which one kernel is the better one at every size: 22 at
+// power 8, 20 at another integer power of the launch, 16 with real powers, whose
+// steps are the longest and want the most waves.  A call on points spread evenly
+// over the cube, us, two kernels (the workspace's allocation included) / one:
+//   iterations    18         20         22         24         28         32
+//   P8   2^17     57 / 30    54 / 32    58 / 38    60 / 41    59 / 47    85 / 53
+//        2^18     72 / 37    75 / 40    77 / 63    80 / 66    86 / 100   91 / 112
+//        2^20    152 / 136  162 / 140  166 / 165  172 / 193  192 / 236  201 / 257
+//        2^22    641 / 425  632 / 476  657 / 555  679 / 660  729 / 828  791 / 898
+//   p5   2^18     82 / 49    86 / 52    89 / 85    94 / 94   101 / 124  108 / 139
+//        2^20    174 / 184  187 / 188  194 / 219  200 / 260  227 / 319  232 / 349
+//        2^22    657 / 594  665 / 657  703 / 768  714 / 909  811 / 1142 860 / 1238
+//   real 2^17     72 / 51    76 / 57    87 / 66    89 / 72    98 / 82   127 / 93
+//        2^18     99 / 64   104 / 69   109 / 115  115 / 123  125 / 165  136 / 185
+//        2^20    209 / 237  223 / 249  235 / 288  245 / 343  275 / 427  300 / 474
+//        2^22    740 / 781  773 / 868  820 / 1025 880 / 1218 955 / 1540 1056 / 1694
+// (15 iterations, 2^20: 136 / 118, 155 / 154, 185 / 196; 2^22: 584 / 364,
+// 590 / 494, 658 / 644.)
+inline bool one_sweep_kernel(uint32_t max_iters, uint32_t n, uint32_t any) {
+    return max_iters <= (n <= 1u << 17 ? 32u : n <= 1u << 18 ? std::max(any, 21u) : any);
+}
+
 // The reverse sweep's workgroups are single waves: the family's shape with as
 // many waves per CU.
 inline LaunchShape single_waves(LaunchShape ls) {

@@ -355,8 +355,8 @@ int cth_render_depth_dev(cth_ctx* ctx, const cth_shape* shape, const cth_camera*
  *                                           only, 0 for the other kinds)
  * grad_d NULL means all ones.  The derivative ignores the measure-zero
  * switches of the loop (bailout, iteration cap).  Large iteration caps (above
- * 32, or above 20 off power 8 with many points) use a device workspace of at
- * most ~1 GiB (stream-ordered allocation). */
+ * 32, or with more than 2^17 points above 16 to 22) use a device workspace of
+ * at most ~1 GiB (stream-ordered allocation). */
 int cth_de_vjp_dev(cth_ctx* ctx, const cth_shape* shape, const float* pts, const float* powers, size_t n,
                    const float* grad_d, float* d, float* grad_p, float* grad_power, void* stream);
 

@@ -127,6 +127,22 @@ static void sweep_shapes() {
     }
 }
 
+// One kernel while it is the faster one: at every size up to `any` iterations,
+// with fewer points beyond.
+static void sweep_kernels() {
+    for (uint32_t any : {16u, 20u, 22u}) {
+        for (uint32_t n : {1u, 1u << 17, 1u << 18, 1u << 20, 1u << 22}) {
+            for (uint32_t it = 1; it <= any; ++it) CHECK(one_sweep_kernel(it, n, any));
+            for (uint32_t it = any + 1; it <= 40; ++it) {
+                const bool one = one_sweep_kernel(it, n, any);
+                CHECK(one == (n <= 1u << 17 ? it <= 32 : n <= 1u << 18 && it <= 21));
+            }
+        }
+        CHECK(!one_sweep_kernel(32, (1u << 17) + 1, any) && !one_sweep_kernel(24, 1000000, any));
+        CHECK(!one_sweep_kernel(4095, 1, any));
+    }
+}
+
 static bool same(const WorkQueue& a, const WorkQueue& b) {
     return a.waves == b.waves && a.chunk == b.chunk && a.chunks == b.chunks && a.rotate == b.rotate &&
            a.dynamic == b.dynamic && a.refill_min == b.refill_min;
@@ -186,6 +202,7 @@ int main() {
     refinement_levels();
     captures();
     shapes_kept();
+    sweep_kernels();
     sweep_shapes();
     orbit_sweep();
     ring_advances();

@@ -135,6 +135,29 @@ def test_vjp_iteration_caps(ctx, torch_cuda, P, iters):
     assert np.mean(a <= 1e-3) > 0.9
 
 
+@pytest.mark.parametrize("kind", ["p8", "p5", "real", "powers"])
+@pytest.mark.parametrize("iters", [16, 17, 20, 22, 23])
+def test_sweep_kernels_agree_at_their_lines(ctx, torch_cuda, kind, iters):
+    """Caps on both sides of those up to which one kernel serves every size: a
+    batch of over 2^18 points and its parts, which one kernel serves, give the
+    same bits."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    from cantucci_amd.workloads import shell_points
+    torch = torch_cuda
+    n = (1 << 18) + 65
+    pts, powers = shell_points(n, seed=iters)
+    P, W = gpu(torch, pts), gpu(torch, powers) if kind == "powers" else None
+    shape = {"p8": lambda: ca.Mandelbulb(iters, 2.0, 8, ctx=ctx), "p5": lambda: ca.Mandelbulb(iters, 2.0, 5, ctx=ctx),
+             "real": lambda: ca.MandelbulbTrig(iters, 2.0, 6.5, ctx=ctx),
+             "powers": lambda: ca.MandelbulbTrig(iters, 2.0, 8.0, ctx=ctx)}[kind]()
+    whole = dev.de_vjp(shape, P, W)
+    for lo in range(0, n, 1 << 17):
+        part = dev.de_vjp(shape, P[lo:lo + (1 << 17)], None if W is None else W[lo:lo + (1 << 17)])
+        for a, b in zip(whole, part):
+            assert torch.equal(a[lo:lo + (1 << 17)].view(torch.int32), b.view(torch.int32))
+
+
 def test_vjp_is_linear_in_grad_d(ctx, torch_cuda):
     import cantucci_amd as ca
     from cantucci_amd import device as dev
