@@ -7,8 +7,8 @@
 // in the same branch-free ticks as the plain distance kernel.  When a lane's
 // evaluation finishes, the lane takes its step (pos += dir * d, t += d) with
 // the next batch of such lanes and either starts the ray's next evaluation or
-// writes the ray and takes another, so lanes stay busy although both the evaluation lengths and the
-// ray step counts differ wildly.  (On the camera workload an evaluation runs
+// writes the ray and takes another, so lanes stay busy although both the
+// evaluation lengths and the ray step counts differ wildly.  (On the camera workload an evaluation runs
 // 1.6 loop bodies on average and a third run none, so the steps are as much
 // of the work as the bodies.)  The hit test is d < eps_abs + eps_rel * t
 // (eps_rel = 0 gives the reference's absolute test; eps_abs = 0 the relative
@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "internal.h"
 #include "launch.h"
@@ -157,11 +158,20 @@ struct TraceOut {
     float* hit_pos;  // nullable: position after the last step
 };
 
-// Lanes whose evaluation has finished take their step together once this
-// many are due (or no lane is running a loop body).  The 32 x 1080p render
-// takes 8.1, 7.8, 7.7, 7.65, 7.65, 8.0 ms at 16, 24, 32, 40, 48, 56 (two
-// cards 4 % apart, averaged).
-constexpr uint32_t kStepMin = 40;
+// Lanes whose evaluation has finished take their step together once step_min
+// are due (or no lane is running a loop body).  The 32 x 1080p render at power 8
+// takes 8.1, 7.8, 7.7, 7.65, 7.65, 8.0 ms at 16, 24, 32, 40, 48, 56 (two cards
+// 4 % apart, averaged).  A body of the trig map costs more beside a step, and with
+// real powers so much that waiting lanes do not pay: power 5, 1080p and
+// 4 x 960 x 540, 2.37 / 3.25, 2.16 / 2.59, 2.10 / 2.55, 2.13 / 2.50, 2.16 / 2.86
+// ms at 1, 16, 24, 32, 40; power 6.5, 161 x 120, 960 x 540 and 1080p, 2.06 / 3.18 /
+// 4.66, 1.94 / 3.16 / 4.59, 2.30 / 3.33 / 4.75, 2.30 / 3.60 / 4.79, 2.30 / 3.63 /
+// 4.96, 2.30 / 3.59 / 4.98 at 1, 2, 4, 16, 32, 40.
+template <class Ev>
+__device__ __forceinline__ uint32_t step_min(const MandelUniform& u) {
+    if constexpr (std::is_same<Ev, TrigExact>::value) return u.integral ? 32u : 2u;
+    return 40u;
+}
 
 // Idle lanes take new rays along with a step, from this many on: the rays
 // wait in LDS (below), so taking one costs seven instructions.  2, 4 and 8 are
@@ -186,11 +196,11 @@ __global__ __launch_bounds__(256) void k_trace(
     // (live_m), or holding a finished evaluation whose step is due (step_m:
     // an evaluation from beyond the bailout radius runs no body, so it is
     // finished as soon as it starts).  One iteration of the loop runs one
-    // loop body; once kStepMin lanes are due or none is live, every due lane
+    // loop body; once step_min lanes are due or none is live, every due lane
     // takes its step (pos += dir d, t += d, the end tests), lanes without a ray
     // take one, and all of these start their next evaluation together.  An
-    // evaluation's step waits at most until half the wave's lanes are due; it
-    // never waits for the rest of the wave.
+    // evaluation's step waits at most until step_min lanes are due; it never
+    // waits for the rest of the wave.
     uint64_t live_m = 0, step_m = 0, ray_m = 0;
     bool has_ray = false;
     uint32_t idx = 0, nsteps = 0;
@@ -198,6 +208,7 @@ __global__ __launch_bounds__(256) void k_trace(
     float r = idle_start(ev, u), t = 0.0f;
     float pos[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f};
     Window win;
+    const uint32_t step_at = step_min<Ev>(u);
     const uint32_t fetch_min = q.refill_min < kFetchMin ? q.refill_min : kFetchMin;
     WorkTally<kCount> tally;
 
@@ -224,11 +235,11 @@ __global__ __launch_bounds__(256) void k_trace(
     };
 
     for (;;) {
-        // The step runs for at least kStepMin lanes at a time: due lanes wait
+        // The step runs for at least step_min lanes at a time: due lanes wait
         // while other lanes are live.  An evaluation averages under two loop
         // bodies, so stepping every iteration would run the step's
         // instructions for a third of the wave almost every time.
-        if (live_m == 0 || (uint32_t)__popcll(step_m) >= kStepMin) {
+        if (live_m == 0 || (uint32_t)__popcll(step_m) >= step_at) {
             do {
                 if (__builtin_amdgcn_inverse_ballot_w64(step_m)) step(ev.finish(r));
                 const uint64_t cont = step_m & wave_mask(has_ray);

@@ -250,3 +250,42 @@ def test_trace_rejects_bad_arguments(ctx, torch_cuda):
     assert get_focii(shape, (-3, 0, 0), (1, 0, 0), 1.0, 16 / 9, 0.00004, 10.0, focus_points=0).shape == (0, 3)
     with pytest.raises(ValueError):
         dev.get_focii(shape, torch.zeros((1, 9), device="cuda"))
+
+
+@pytest.mark.parametrize("kind", ["p8", "p5", "real", "sphere"])
+def test_trace_is_the_march_of_the_distances(ctx, torch_cuda, kind):
+    """Every evaluator batches its steps and its new rays by thresholds of its own:
+    depth, steps and end position are those of a march over point batches
+    (src/mesh/mod.rs:205-243), bit for bit, for rays that hit, escape and run to
+    the step limit, at counts around a wave and beyond."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    shape = {"p8": lambda: ca.Mandelbulb.classic(6, 2.5, ctx=ctx), "p5": lambda: ca.Mandelbulb(6, 2.5, 5, ctx=ctx),
+             "real": lambda: ca.MandelbulbTrig(6, 2.5, 6.5, ctx=ctx),
+             "sphere": lambda: ca.Sphere((0.0, 0.1, 0.2), 0.9, ctx=ctx)}[kind]()
+    eps_abs, eps_rel, t_max, limit = 1e-4, 1e-3, 6.0, 40
+    for n in (1, 63, 65, 5000):
+        rng = np.random.default_rng(n)
+        o = rng.uniform(-1.0, 1.0, (n, 3)) + np.array([0.0, 0.0, 3.0])
+        d = rng.uniform(-1.2, 1.2, (n, 3)) - o
+        org, dirs = gpu(torch, o.astype(F32)), gpu(torch, (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(F32))
+        depth, steps, end = dev.sphere_trace(shape, org, dirs, limit, eps_abs, eps_rel, t_max, with_pos=True)
+        pos, t = org.clone(), torch.zeros(n, device="cuda")
+        want_d = torch.full((n,), float("inf"), device="cuda")
+        want_s = torch.zeros(n, dtype=torch.int32, device="cuda")
+        live = torch.ones(n, dtype=torch.bool, device="cuda")
+        rel, absolute = torch.tensor(eps_rel, device="cuda"), torch.tensor(eps_abs, device="cuda")
+        for k in range(1, limit + 1):
+            dist = dev.de_points(shape, pos)
+            moved, tn = pos + dirs * dist[:, None], t + dist
+            pos, t = torch.where(live[:, None], moved, pos), torch.where(live, tn, t)
+            hit = live & (dist < absolute + rel * t)
+            want_d = torch.where(hit, t, want_d)
+            want_s = torch.where(live, torch.full_like(want_s, k), want_s)
+            live = live & ~hit & ~(t > t_max)
+        assert torch.equal(steps.view(torch.int32), want_s)
+        assert torch.equal(depth.view(torch.int32), want_d.view(torch.int32))
+        assert torch.equal(end.view(torch.int32), pos.view(torch.int32))
+        if n == 5000:
+            assert 0 < torch.isinf(want_d).sum() < n
