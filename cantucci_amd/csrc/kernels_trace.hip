@@ -175,8 +175,11 @@ __device__ __forceinline__ uint32_t step_min(const MandelUniform& u) {
 
 // Idle lanes take new rays along with a step, from this many on: the rays
 // wait in LDS (below), so taking one costs seven instructions.  2, 4 and 8 are
-// within 1 % of each other.
-constexpr uint32_t kFetchMin = 4;
+// within 1 % of each other.  A sphere's evaluation is one short body, after which
+// every lane steps, so that there the taking is a large part: 1080p, 4 x 960 x 540
+// and 640 x 360 170, 151, 108 us at 4, 162, 155, 104 at 16, 150, 158, 104 at 32.
+template <class Ev>
+constexpr uint32_t kFetchMin = std::is_same<Ev, SphereEv>::value ? 32 : 4;
 
 template <class Ev, class Rays, bool kCount = false>
 __global__ __launch_bounds__(256) void k_trace(
@@ -209,7 +212,7 @@ __global__ __launch_bounds__(256) void k_trace(
     float pos[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f};
     Window win;
     const uint32_t step_at = step_min<Ev>(u);
-    const uint32_t fetch_min = q.refill_min < kFetchMin ? q.refill_min : kFetchMin;
+    const uint32_t fetch_min = q.refill_min < kFetchMin<Ev> ? q.refill_min : kFetchMin<Ev>;
     WorkTally<kCount> tally;
 
     // One sphere-tracing step of the lane's ray by distance d.  When the ray
