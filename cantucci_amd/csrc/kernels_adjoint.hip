@@ -653,17 +653,18 @@ int launch_tangent(Ctx& c, const cth_shape& s, const float* pts, const float* po
     if (powers) u.power = kPointPower;
     SrcPoints src{pts, powers, s.power};
     SinkGrad sink{d, normals, grad_p, grad_power, grad_d, u.max_iters};
+    const LaunchShape ls = tangent_shape(c.shape_adj, n, c.num_cus);
     uint32_t blocks = 0;
-    WorkQueue q = make_queue(c, n, c.shape_adj, family == FAM_P8 ? P8Tangent::kSpread : TrigNormal::kSpread,
+    WorkQueue q = make_queue(c, n, ls, family == FAM_P8 ? P8Tangent::kSpread : TrigNormal::kSpread,
                              blocks, st);
     if (family == FAM_P8)
-        hipLaunchKernelGGL((k_refill<P8Tangent, SrcPoints, SinkGrad>), dim3(blocks), dim3(c.shape_adj.block), 0, st, src,
+        hipLaunchKernelGGL((k_refill<P8Tangent, SrcPoints, SinkGrad>), dim3(blocks), dim3(ls.block), 0, st, src,
                            u, sink, q);
     else if (grad_power)  // the power column only when its gradient is asked for
-        hipLaunchKernelGGL((k_refill<TrigTangent, SrcPoints, SinkGrad>), dim3(blocks), dim3(c.shape_adj.block), 0, st,
+        hipLaunchKernelGGL((k_refill<TrigTangent, SrcPoints, SinkGrad>), dim3(blocks), dim3(ls.block), 0, st,
                            src, u, sink, q);
     else
-        hipLaunchKernelGGL((k_refill<TrigNormal, SrcPoints, SinkGrad>), dim3(blocks), dim3(c.shape_adj.block), 0, st,
+        hipLaunchKernelGGL((k_refill<TrigNormal, SrcPoints, SinkGrad>), dim3(blocks), dim3(ls.block), 0, st,
                            src, u, sink, q);
     return check_hip(hipGetLastError(), "tangent launch");
 }

@@ -147,8 +147,8 @@ inline bool one_sweep_kernel(uint32_t max_iters, uint32_t n, uint32_t any) {
     return max_iters <= (n <= 1u << 17 ? 32u : n <= 1u << 18 ? std::max(any, 21u) : any);
 }
 
-// The reverse sweep's workgroups are single waves: the family's shape with as
-// many waves per CU.
+// The family's shape in workgroups of a single wave, with as many waves per CU
+// (the reverse sweep's, and small tangent launches').
 inline LaunchShape single_waves(LaunchShape ls) {
     ls.blocks_per_cu *= ls.block / 64;
     ls.block = 64;
@@ -175,6 +175,17 @@ inline LaunchShape sweep_shape(const LaunchShape& family, uint32_t n, int num_cu
 // per-point powers 396 -> 282, 597 -> 371, 1228 -> 803, 4737 -> 3212.  (The
 // workspace's place in memory moves single figures by up to a quarter.)
 constexpr WaveSpread kOrbitSpread{8, 8};
+
+// A tangent evaluator's launch: on the default shape in single-wave workgroups
+// while there is at most one wave for each CU, since the four waves of a
+// workgroup slow each other down on one CU (a body is 8 KB of code).  256 / 5,000 /
+// 16,384 points, normals at power 5 and gradients with a power per point, 15
+// iterations 21 / 30 / 22 and 29 / 40 / 31 -> 19 / 19 / 18 and 28 / 27 / 27 us, 60
+// iterations 83 / 109 / 72 and 117 / 144 / 109 -> 68 / 62 / 62 and 102 / 96 / 96;
+// power 8 within 1 us.
+inline LaunchShape tangent_shape(const LaunchShape& family, uint64_t n, int num_cus) {
+    return !family.given && n <= 64u * (uint64_t)num_cus ? single_waves(family) : family;
+}
 
 template <class Src, class Sink>
 inline int run_refill(Ctx& c, int family, const MandelUniform& u, const Src& src, const Sink& sink,

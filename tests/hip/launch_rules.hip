@@ -13,6 +13,7 @@ static hipError_t test_stream_is_capturing(hipStream_t, hipStreamCaptureStatus* 
 }
 #define hipStreamIsCapturing test_stream_is_capturing
 #include "launch.h"
+#include "tangent.h"
 
 namespace cth {
 CapturePool& capture_pool() {
@@ -127,6 +128,22 @@ static void sweep_shapes() {
     }
 }
 
+// A tangent launch of at most a wave per CU gives every wave a workgroup of its
+// own, unless the caller has set the shape.
+static void tangent_shapes() {
+    std::vector<uint32_t> ring;
+    Ctx c = make_ctx(ring);
+    for (uint32_t n : {1u, 64u, 65u, 5000u, 16384u, 16385u, 4000000u}) {
+        uint32_t blocks = 0;
+        const LaunchShape ls = tangent_shape(c.shape_adj, n, 256);
+        const WorkQueue q = make_queue(c, n, ls, P8Tangent::kSpread, blocks, kStream);
+        CHECK(ls.block == (n <= 16384u ? 64 : c.shape_adj.block));
+        CHECK(q.waves == blocks * (ls.block / 64u) && (n > 16384u || blocks == (n + 63u) / 64u));
+        const LaunchShape set{256, 4, 128, 16, 0, true};
+        CHECK(tangent_shape(set, n, 256).block == 256);
+    }
+}
+
 // One kernel while it is the faster one: at every size up to `any` iterations,
 // with fewer points beyond.
 static void sweep_kernels() {
@@ -202,6 +219,7 @@ int main() {
     refinement_levels();
     captures();
     shapes_kept();
+    tangent_shapes();
     sweep_kernels();
     sweep_shapes();
     orbit_sweep();
