@@ -3,7 +3,7 @@
 // The reference refines a CPU octree one leaf at a time (ShapeMesh::update,
 // src/mesh/mod.rs:82-178, child spans from create_spans,
 // src/octree/mod.rs:315-329).  Here the top of the tree, levels of up to
-// kTopNodes nodes, is one workgroup's launch, and each level below it one
+// top_nodes() nodes, is one workgroup's launch, and each level below it one
 // batch: the centre distance of every node at depth d is evaluated by the
 // lane-refill work loop, the split flags are prefix-summed, and every split
 // node writes its 8 children (create_spans order) into the next level's array.
@@ -107,21 +107,10 @@ __global__ void k_emit_leaves(const float* __restrict__ nodes, const uint32_t* _
     leaves[6 * (size_t)(incl[i] - 1u) + a] = nodes[6 * (size_t)i + a];
 }
 
-// The tree's top, all levels of at most kTopNodes nodes, in one workgroup: no
-// read-back and no launch between levels.  A level took 20-30 us whatever its
-// size (four or five launches and a wait for its split count).  Depth 2, 4, 5
-// and 7 of the octree: 82, 129, 158, 226 -> 27, 55, 98, 167 us.  Up to 512 nodes
-// gave 27, 69, 97, 166, up to 10,240 27, 55, 156, 257 (one CU is then slower
-// than a level of launches); real powers take 51 us more with 4,096.
-//
-// One CU's waves share its issue slots, a level's own launch spreads over the
-// chip: with caps above kTopIters the top's points take longer than the launches
-// it saves, except under the trig map's integer powers.  One launch / level by
-// level, us, depths 2 to 4: power 8 at 100 / 150 / 400 / 1000 iterations 194 / 218,
-// 273 / 262, 671 / 472, 1624 / 981; power 5 201 / 271, 270 / 336, 615 / 661,
-// 1441 / 1451; a real power 454 / 493, 652 / 673, 1634 / 1566, 3977 / 3708.
-constexpr uint32_t kTopNodes = 2048;
-constexpr uint32_t kTopIters = 128;
+// The tree's top, all levels of at most top_nodes() (launch.h) nodes, in one
+// workgroup: no read-back and no launch between levels.  A level took 20-30 us
+// whatever its size (four or five launches and a wait for its split count).
+// Depth 2, 4, 5 and 7 of the octree: 82, 129, 158, 226 -> 27, 55, 98, 167 us.
 constexpr uint32_t kTopThreads = 1024;
 constexpr uint32_t kMaxDepth = 20;
 static_assert(2 + kMaxDepth + 1 <= kPinnedWords, "level counts fit");
@@ -130,6 +119,7 @@ struct RefineTop {
     float root[6];
     float half_diag[kMaxDepth + 1];
     uint32_t min_depth, max_depth;
+    uint32_t top_nodes;
     float* nodes[2];   // level d in nodes[d & 1]
     float* leaves;     // nullable
     uint64_t cap;
@@ -213,7 +203,7 @@ __global__ __launch_bounds__(kTopThreads) void k_refine_top(RefineTop a, MandelU
             return;
         }
         n = 8 * total;
-        if (n == 0 || n > kTopNodes) break;
+        if (n == 0 || n > a.top_nodes) break;
     }
     if (threadIdx.x == 0) {
         a.out[0] = depth + 1;
@@ -226,8 +216,9 @@ static inline uint32_t cdiv32(uint64_t a, uint64_t b) { return (uint32_t)((a + b
 // Level-synchronous refinement: the top of the tree in one launch, then per
 // level the split flags (forced, sphere closed form or a DE refill launch), an
 // inclusive scan of the flags, one 4-byte read-back of the split count into
-// pinned host memory, and the children.  Node, flag, offset and scan buffers are the context's scratch
-// slots (ping-pong for the nodes), so a level allocates nothing.
+// pinned host memory, and the children.  Node, flag, offset and scan buffers are
+// the context's scratch slots (ping-pong for the nodes), so a level allocates
+// nothing.
 int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_depth, uint32_t max_depth,
                   const float* half_diag, float* leaves, size_t cap, size_t* nleaves, uint64_t* level_counts,
                   hipStream_t st) {
@@ -242,9 +233,7 @@ int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_de
     uint32_t depth = 0;
     uint64_t n = 1;
     float* nodes[2] = {};
-    // counted work goes through the work loops
-    const bool top_launch = !c.stats && (family == FAM_SPHERE || u.max_iters <= kTopIters ||
-                                         (family == FAM_TRIG && u.integral));
+    const bool top_launch = !c.stats;  // counted work goes through the work loops
     const size_t first = top_launch ? (size_t)8 * kTopNodes : 1;
     int rc = CTH_OK;
     for (int k = 0; k < 2 && !rc; ++k) rc = c.scratch(WS_NODES_A + k, first * 6 * sizeof(float), (void**)&nodes[k]);
@@ -255,6 +244,7 @@ int refine_levels(Ctx& c, const cth_shape& s, const float* root, uint32_t min_de
         std::copy(half_diag, half_diag + max_depth + 1, top.half_diag);
         top.min_depth = min_depth;
         top.max_depth = max_depth;
+        top.top_nodes = top_nodes(family == FAM_SPHERE ? 1u : u.max_iters, family == FAM_TRIG && !u.integral);
         top.nodes[0] = nodes[0];
         top.nodes[1] = nodes[1];
         top.leaves = leaves;

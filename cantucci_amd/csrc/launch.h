@@ -111,6 +111,21 @@ inline WorkQueue make_queue(Ctx& c, uint32_t total, LaunchShape ls, WaveSpread s
     return q;
 }
 
+// The largest level that the refinement's one workgroup takes (k_refine_top).
+// Beyond, a level's own launches are faster: one CU's waves share its issue
+// slots, and long evaluations take longer there than the launches cost (64 nodes
+// are a single wave, which takes as long anywhere).  Depths 2 to 4 of the octree
+// at 64 / 512 / 2,048 nodes, us: power 8 at 15, 60, 129, 300, 1000
+// iterations 162 / 127 / 109, 240 / 207 / 250, 355 / 330 / 469, 648 / 635 / 1009,
+// 1838 / 1883 / 3220; power 5 183 / 150 / 151, 306 / 279 / 278, 490 / 476 / 476,
+// 946 / 963 / 962, 2813 / 2952 / 2951; a real power 245 / 220 / 220, 567 / 570 /
+// 570, 1061 / 1106 / 1106, 2280 / 2433 / 2432, 7292 / 7866 / 7870.
+constexpr uint32_t kTopNodes = 2048;
+inline uint32_t top_nodes(uint32_t max_iters, bool real_power) {
+    if (max_iters <= 28) return kTopNodes;
+    return max_iters <= (real_power ? 64u : 512u) ? 512u : 64u;
+}
+
 // A refinement level's launch: the span family's shape with 64-point chunks dealt
 // statically, which spreads a level over the whole chip; levels of millions of
 // nodes claim as every default shape does, whether the span shape is the caller's

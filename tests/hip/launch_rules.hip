@@ -144,6 +144,20 @@ static void tangent_shapes() {
     }
 }
 
+// The refinement's one workgroup takes the whole levels it has room for, fewer
+// nodes the longer their evaluations are.
+static void refinement_tops() {
+    for (bool real : {false, true}) {
+        uint32_t was = kTopNodes;
+        for (uint32_t it : {1u, 15u, 28u, 29u, 64u, 65u, 512u, 513u, 4000u}) {
+            const uint32_t n = top_nodes(it, real);
+            CHECK(n <= was && n >= 64 && n <= kTopNodes);
+            was = n;
+        }
+    }
+    CHECK(top_nodes(15, true) == 2048 && top_nodes(129, false) == 512 && top_nodes(129, true) == 64);
+}
+
 // One kernel while it is the faster one: at every size up to `any` iterations,
 // with fewer points beyond.
 static void sweep_kernels() {
@@ -220,6 +234,7 @@ int main() {
     captures();
     shapes_kept();
     tangent_shapes();
+    refinement_tops();
     sweep_kernels();
     sweep_shapes();
     orbit_sweep();

@@ -134,3 +134,31 @@ def test_refinement_at_large_caps(ctx, torch_cuda, kind, iters):
     got, lc = dev.refine(shape, root, 1, 5, hd)
     assert (lc == want_lc).all()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("iters", [1, 28, 29, 64, 65, 512, 513])
+@pytest.mark.parametrize("kind", ["p8", "real", "sphere"])
+def test_refinement_hands_over_at_any_level(ctx, torch_cuda, kind, iters):
+    """The one workgroup hands over to the levels' own launches earlier the longer
+    the evaluations are: leaves and level counts are the counted refinement's on
+    both sides of each cap, from single levels to trees beyond its largest."""
+    import cantucci_amd as ca
+    from cantucci_amd import device as dev
+    from cantucci_amd.workloads import half_diagonals
+    torch = torch_cuda
+    shape = {"p8": lambda: ca.Mandelbulb.classic(iters, 2.0, ctx=ctx),
+             "real": lambda: ca.MandelbulbTrig(iters, 2.0, 6.5, ctx=ctx),
+             "sphere": lambda: ca.Sphere((0.0, 0.1, 0.2), 0.9, ctx=ctx)}[kind]()
+    root = (-1.5,) * 3 + (1.5,) * 3
+    for mind, d in ((0, 0), (0, 3), (2, 2), (2, 3), (3, 5), (4, 4)):
+        hd = half_diagonals(3.0, d)
+        cnt = torch.zeros(4, dtype=torch.int64, device="cuda")
+        ctx.count_work(cnt)
+        try:
+            want, want_lc = dev.refine(shape, root, mind, d, hd)
+            torch.cuda.synchronize()
+        finally:
+            ctx.count_work(None)
+        got, lc = dev.refine(shape, root, mind, d, hd)
+        assert (lc == want_lc).all()
+        assert torch.equal(got, want)
