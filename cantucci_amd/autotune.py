@@ -32,8 +32,9 @@ SPACE = {
 
 # The job sets the jobs shape is tuned on, (jobs, seed of their layout): small,
 # middle and large ones and several of each size, since a shape that suits one
-# layout of 24 jobs costs another 10 %.  They are not those of the bench and the
-# tests.
+# layout of 24 jobs costs another 10 %.  Each is timed at power 8 and under the
+# trig map, whose large sets want other chunks.  They are not those of the bench
+# and the tests.
 JOB_SETS = tuple((n, 70001 + i) for i, n in enumerate((6, 6, 12, 12, 24, 24, 24, 24, 48, 48, 64, 64)))
 
 # The trace kernel batches finished evaluations' steps by a fixed threshold
@@ -161,10 +162,11 @@ def _workloads(ctx):
     runs["tangent"] = lambda: dev.normals(tr, P, W, out=nrm, d=dd)
     runs["fd"] = lambda: dev.normals_fd(tr, P, 1e-3, W, out=nrm, d=dd)
     sets = []
-    for njobs, seed in JOB_SETS:
+    for kind, (njobs, seed) in itertools.product((_lib.CTH_SHAPE_MANDELBULB, _lib.CTH_SHAPE_MANDELBULB_TRIG), JOB_SETS):
         N, Pw, cap = wl.mixed_jobs(njobs, seed=seed)
-        js = dev.JobSet(ctx, _lib.CTH_SHAPE_MANDELBULB_TRIG, 2.0,
-                        [dict(n=int(n), power=float(p), max_iters=int(c)) for n, p, c in zip(N, Pw, cap)])
+        power = (lambda p: 8.0) if kind == _lib.CTH_SHAPE_MANDELBULB else float
+        js = dev.JobSet(ctx, kind, 2.0,
+                        [dict(n=int(n), power=power(p), max_iters=int(c)) for n, p, c in zip(N, Pw, cap)])
         sets.append((js, torch.empty(js.total, device="cuda"), torch.empty((js.total, 3), device="cuda"),
                      torch.zeros(js.njobs, dtype=torch.int64, device="cuda"),
                      torch.zeros(1, dtype=torch.int64, device="cuda")))
