@@ -92,13 +92,15 @@ int staging(Ctx& c, int slot, const size_t (&bytes)[N], void* (&out)[N]) {
     return CTH_OK;
 }
 
-// The buffers of a host-pointer call whose kernels read each input and write
-// each output once.  Calls of up to kHostStage bytes keep them in the context's
-// pinned memory, which the kernels reach directly: memcpys on the host take the
-// place of a copy launch for each buffer.  Distances of 1 / 4,096 / 32,768 /
-// 100,000 points 32 / 38 / 52 / 106 -> 20 / 21 / 35 / 80 us, of 300,000 (beyond)
-// 214 against 192; 25 focus rays 266 -> 239.  Larger ones go through device
-// staging.
+// The buffers of a host-pointer call.  Calls of up to kHostStage bytes keep them
+// in the context's pinned memory, which the kernels reach directly: memcpys on the
+// host take the place of a copy launch for each buffer.  Distances of 1 / 4,096 /
+// 32,768 / 100,000 points 32 / 38 / 52 / 106 -> 20 / 21 / 35 / 80 us, of 300,000
+// (beyond) 214 against 192; 25 focus rays 266 -> 239.  Most are read or written
+// once; those read again are no slower either (an origin shared by 25 / 70,000
+// rays 277 / 995 -> 204 / 639 us, the points of the two-kernel reverse sweep,
+// 40,000 at 40 iterations, 224 -> 145, a sphere's distances of bounded queries,
+// 100,003, 110 -> 100).  Larger calls go through device staging.
 class HostCall {
 public:
     explicit HostCall(Ctx& ctx) : c(ctx) {}

@@ -41,9 +41,9 @@ __global__ __launch_bounds__(256) void k_sphere(Src src, uint32_t n, float cx, f
 inline bool foreign_capture(hipStream_t st) { return capture_pool().stream != st && is_capturing(st); }
 
 // A launch's workgroups and chunks.  Up to a chunk of `least` indices (64 or
-// fewer) for each of spread.fill waves per CU a launch is spread as thinly as possible; from four
-// chunks per wave on it grows to the launch shape's (and spread.most) waves.
-// In between it stays at `fill` up to 8/3 chunks a wave: a lane that takes a
+// fewer) for each of spread.fill waves per CU a launch is spread as thinly as
+// possible; from four chunks per wave on it grows to the launch shape's (and
+// spread.most) waves.  In between it stays at `fill` up to 8/3 chunks a wave: a lane that takes a
 // second point while its wave's slowest is still iterating costs little, more
 // waves on a SIMD cost their share of its issue slots.  Then evaluators with
 // spread.grow grow to that: 500,000 / 600,000 / 800,000 tangent normals at power

@@ -117,11 +117,12 @@ struct Window {
 // whole domain, so that slow and fast regions average out; its place moves by
 // `rotate` from row to row, so that a row length that fits the domain, 4096
 // waves of 256 indices in 128^3 grids, does not give a wave the same region
-// every time); dynamic, the next unclaimed chunk of the workgroup's shard.  Claims on one counter serialise at about 14 ns
-// each, whatever the number of waves (17.6 M corners in 68,600 chunks of 256
-// took 971 us, and 137 us with 32 shards), hence the shards: row j of the
-// remaining chunks holds one for each shard, rotated from row to row so that
-// no shard gets the same region of a regular index space every time.
+// every time); dynamic, the next unclaimed chunk of the workgroup's shard.
+// Claims on one counter serialise at about 14 ns each, whatever the number of
+// waves (17.6 M corners in 68,600 chunks of 256 took 971 us, and 137 us with 32
+// shards), hence the shards: row j of the remaining chunks holds one for each
+// shard, rotated from row to row so that no shard gets the same region of a
+// regular index space every time.
 __device__ __forceinline__ bool next_chunk(const WorkQueue& q, Window& w) {
     if (w.last) return false;
     uint32_t c;

@@ -14,7 +14,7 @@ import sys
 
 def main() -> None:
     ap = argparse.ArgumentParser()
-    ap.add_argument("--legs", default="spans,mesh,trace,tangent,fd,jobs,copy")
+    ap.add_argument("--legs", default="spans,mesh,trace,points,tangent,fd,adjoint,jobs,planes,copy")
     ap.add_argument("--reps", type=int, default=5)
     args = ap.parse_args()
     legs = set(args.legs.split(","))
@@ -25,6 +25,7 @@ def main() -> None:
     from cantucci_amd import _lib, autotune
     from cantucci_amd import device as dev
     from cantucci_amd import workloads as wl
+    from cantucci_amd.mesh import create_spans
 
     ctx = ca.Context(0, "parity")
     m8 = ca.Mandelbulb.classic(15, 2.0, ctx=ctx)
@@ -68,6 +69,30 @@ def main() -> None:
             dev.normals_fd(tr, P, 1e-3, W)
         torch.cuda.synchronize()
         print("fd done", flush=True)
+    if "points" in legs:
+        m5 = ca.Mandelbulb(15, 2.0, 5)
+        U = torch.from_numpy(wl.uniform(2, 3 << 20, -1.5, 1.5).astype("float32").reshape(-1, 3)).cuda()
+        for _ in range(args.reps):
+            dev.de_points(m5, U)
+        torch.cuda.synchronize()
+        print("points done", flush=True)
+    if "adjoint" in legs:
+        tr0 = ca.MandelbulbTrig(15, 2.0, 8.0)
+        for _ in range(args.reps):
+            dev.de_vjp(tr0, P[:300001], W[:300001], with_power=True)
+        torch.cuda.synchronize()
+        print("adjoint done", flush=True)
+    if "planes" in legs:
+        app = ca.Mandelbulb.classic(6, 2.5)
+        spans = [app.bounding_box()]
+        for _ in range(2):
+            spans = [c for a in spans for c in create_spans(a)]
+        S = torch.tensor([[*a, *b] for a, b in spans], dtype=torch.float32, device="cuda")
+        D, _ = dev.sample_spans(app, S, 64, with_cross=False)
+        for _ in range(args.reps):
+            dev.mesh(app, S, D, 64, "fd6")
+        torch.cuda.synchronize()
+        print("planes done", flush=True)
     if "jobs" in legs:
         autotune.apply(ctx, "jobs")
         N, Pw, cap = wl.mixed_jobs(64, seed=5)
