@@ -62,11 +62,14 @@ static int check_shape(const cth_shape* s) {
 }
 
 int Ctx::emit_scratch(size_t bytes, uint64_t** out, hipStream_t st) {
-    if (scratch(WS_EMIT, bytes, (void**)out)) return fail(CTH_E_NOMEM, "mesh scratch allocation failed");
-    return emit_pending ? check_hip(hipStreamWaitEvent(st, emit_event, 0), "hipStreamWaitEvent") : CTH_OK;
+    const int slot = st == nullptr ? WS_EMIT_NULL : st == stream ? WS_EMIT_OWN : WS_EMIT;
+    if (scratch(slot, bytes, (void**)out)) return fail(CTH_E_NOMEM, "mesh scratch allocation failed");
+    if (slot != WS_EMIT || !emit_pending) return CTH_OK;
+    return check_hip(hipStreamWaitEvent(st, emit_event, 0), "hipStreamWaitEvent");
 }
 
 int Ctx::emit_done(hipStream_t st) {
+    if (st == nullptr || st == stream) return CTH_OK;
     emit_pending = true;
     return check_hip(hipEventRecord(emit_event, st), "hipEventRecord");
 }

@@ -262,6 +262,53 @@ def test_emission_beside_calls_on_another_stream(ctx, torch_cuda, res):
                 assert torch.equal(a, b), (rep, r)
 
 
+@pytest.mark.parametrize("first,second", [("null", "side"), ("side", "null"), ("own", "null"), ("null", "own"),
+                                          ("own", "side"), ("side", "other"), ("null", "null")])
+def test_emissions_of_every_stream(torch_cuda, first, second):
+    """Two emissions in a row on the null stream, the context's own and others, in
+    every pairing, each with the memory or the order that its stream needs: both
+    meshes are those emitted alone, after growth of the memory too."""
+    import ctypes as C
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    c = ca.Context(0, "parity")
+    shape = ca.Sphere((0.0, 0.0, 0.0), 1.0, ctx=c)
+    rng = np.random.default_rng(9)
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    handles = {"null": 0, "own": c.stream, "side": side.cuda_stream, "other": other.cuda_stream}
+    jobs = []
+    for res, leaves in ((64, 20), (64, 33), (32, 150), (64, 5)):
+        base = torch.from_numpy(rng.choice(np.array([-1.0, 1.0], F32), (3, (res + 1) ** 3))).cuda()
+        field = base[torch.from_numpy(rng.integers(0, 3, leaves)).cuda()].contiguous()
+        spans = torch.tensor([[-1.0, -1.0, -1.0, 1.0, 1.0, 1.0]], device="cuda").repeat(leaves, 1)
+        jobs.append((res, leaves, spans, field, *dev.mesh(shape, spans, field, res, "deferred")))
+    outs = [(torch.empty_like(j[6]), torch.empty_like(j[7])) for j in jobs]
+
+    def emit(k, stream):
+        res, leaves, spans, field, voff, ioff, v, _ = jobs[k]
+        _lib.check(_lib.lib.cth_mesh_emit_dev(
+            c.handle, C.byref(shape.desc), spans.data_ptr(), field.data_ptr(), leaves, res,
+            _lib.CTH_NORMALS_DEFERRED, voff.data_ptr(), ioff.data_ptr(), v.shape[0], outs[k][0].data_ptr(),
+            outs[k][1].data_ptr(), handles[stream]))
+
+    try:
+        for a, b in ((0, 1), (2, 3), (1, 0), (3, 2)):
+            for o in outs:
+                o[0].fill_(-1.0)
+                o[1].fill_(-1)
+            torch.cuda.synchronize()
+            emit(a, first)
+            emit(b, second)
+            torch.cuda.synchronize()
+            for k in (a, b):
+                assert torch.equal(outs[k][0], jobs[k][6]) and torch.equal(outs[k][1], jobs[k][7]), (a, b, k)
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def test_octree_leaf_mesh_parity(ctx, torch_cuda):
     """2,000 seeded depth-8 surface leaves of the octree workload (P8, 15 it,
     bailout 2, 8^3 cells per leaf)."""
