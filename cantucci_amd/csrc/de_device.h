@@ -282,9 +282,11 @@ struct P8Exact {
         guard();
     }
     // The same after a body on the scaled sequences.  Near the z axis (w between
-    // about 2^-18.6 and 2^-16 |z|) w8 is subnormal, num / w8 overflows and the
-    // body ends at infinity, as the reference's does: that point bails and is
-    // held too.  Only wave ticks that are slow anyway make this test.
+    // about 2^-18.6 and 2^-16 |z|) num / w8 overflows and the body ends at
+    // infinity, as the reference's does: that point bails and is held too.  Only
+    // wave ticks that are slow anyway make this test.  (Made only where some lane
+    // has w2 < 2^-23, 1 M points at 100 iterations gain 3 % and meshes of 64^3
+    // cells lose 0.7: left.)
     __device__ __forceinline__ void range_after_scaled(bool live, float ax, float ay, float az) {
         in_range = in_range && wave_mask(live && !((ax * ax + ay * ay) + az * az <= 0x1p126f)) == 0;
     }

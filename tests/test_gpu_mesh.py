@@ -309,6 +309,39 @@ def test_emissions_of_every_stream(torch_cuda, first, second):
         c.close()
 
 
+@pytest.mark.parametrize("res", [16, 64])
+def test_captured_emission_replays(ctx, torch_cuda, res):
+    """An emission recorded by cth_graph_begin keeps its counts in memory of the
+    graph: replays, with emissions and counts of the context in between, give the
+    eager mesh."""
+    import ctypes as C
+    import cantucci_amd as ca
+    from cantucci_amd import _lib
+    from cantucci_amd import device as dev
+    torch = torch_cuda
+    shape = ca.Mandelbulb.classic(6, 2.5, ctx=ctx)
+    spans = gpu(torch, np.array([[-0.6, -0.6, 0.2, 0.6, 0.6, 1.2], [-1.1, -0.3, -0.5, -0.1, 0.5, 0.4]], F32))
+    d, _ = dev.sample_spans(shape, spans, res, with_cross=False)
+    voff, ioff, v_ref, i_ref = dev.mesh(shape, spans, d, res, "fd6")
+    v, ix = torch.empty_like(v_ref), torch.empty_like(i_ref)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = dev.Graph(lambda: _lib.check(_lib.lib.cth_mesh_emit_dev(
+        ctx.handle, C.byref(shape.desc), spans.data_ptr(), d.data_ptr(), 2, res, _lib.CTH_NORMALS_FD6,
+        voff.data_ptr(), ioff.data_ptr(), v.shape[0], v.data_ptr(), ix.data_ptr(),
+        torch.cuda.current_stream().cuda_stream)), s)
+    for rep in range(4):
+        v.fill_(-1.0)
+        ix.fill_(-1)
+        torch.cuda.synchronize()
+        g.launch()
+        again = dev.mesh(shape, spans, d, res, "fd6")
+        torch.cuda.synchronize()
+        assert torch.equal(v.view(torch.int32), v_ref.view(torch.int32)) and torch.equal(ix, i_ref), rep
+        assert torch.equal(again[2].view(torch.int32), v_ref.view(torch.int32)) and torch.equal(again[3], i_ref)
+    g.close()
+
+
 def test_octree_leaf_mesh_parity(ctx, torch_cuda):
     """2,000 seeded depth-8 surface leaves of the octree workload (P8, 15 it,
     bailout 2, 8^3 cells per leaf)."""
